@@ -1028,8 +1028,11 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
                         const uint32_t kmin = zs_total_key(-INFINITY);
                         thr_o = a0 > kmin ? (long long)a0 - 1 : -1;
                         thr_s = a1 > kmin ? (long long)a1 - 1 : (long long)kmin;
-                        sh.fthr[0] = a0 > kmin ? zs_key_to_float(a0 - 1u) : -INFINITY;
-                        sh.fthr[1] = a1 > kmin ? zs_key_to_float(a1 - 1u) : -INFINITY;
+                        // (as a value, the key below that of +0 is -0, which no
+                        // zero exceeds: the value below both zeros then)
+                        const uint32_t kneg0 = zs_total_key(-0.0f);
+                        sh.fthr[0] = a0 > kmin ? zs_key_to_float(a0 - 1u == kneg0 ? kneg0 - 1u : a0 - 1u) : -INFINITY;
+                        sh.fthr[1] = a1 > kmin ? zs_key_to_float(a1 - 1u == kneg0 ? kneg0 - 1u : a1 - 1u) : -INFINITY;
                     }
                     rw_bar();
                     load_thr();
