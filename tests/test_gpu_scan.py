@@ -1,11 +1,98 @@
-"""The row kernel's candidate lists at thresholds and sizes where they can go
-wrong, compared with the oracle (tokens and top ids bit for bit)."""
+"""The row kernel's lists from group maxima (zs_k_scan): rows where the groups
+of 16, 32 or 64 ids, their thresholds or the listed groups can go wrong, at
+the widths where the group size changes, compared with the oracle (tokens and
+top ids bit for bit, floats within gpu_util.compare's 1e-5)."""
 import numpy as np
 import pytest
 
-from tests.gpu_util import compare, run_gpu
+from tests.gpu_util import compare, oracle_row, run_gpu
 
 pytestmark = pytest.mark.gpu
+
+
+def _case(V):
+    rng = np.random.default_rng(V)
+    B = 20
+    x = rng.normal(0, 2, (B, V)).astype(np.float32)
+    P = [dict(temperature=0.9, top_k=40, top_p=0.95, top_logprobs=20, seed=i) for i in range(B)]
+    x[0].sort()                                    # the top entries adjacent: whole groups pass the threshold
+    x[1] = 1.5                                     # every group at the threshold
+    x[2, -3:] = [9.0, 11.0, 10.0]                  # the last, partial group
+    x[3, V // 2:V // 2 + 200] = 20.0               # more equal entries than k, adjacent
+    x[4] = -np.inf                                 # fewer ids above -inf than candidates
+    x[4, [0, 70, V - 1]] = [1.0, 2.0, 0.5]
+    x[5] = -np.inf                                 # 600 survivors, most in a few groups
+    x[5, 100:700] = rng.normal(0, 1, 600)
+    P[5].update(top_k=0)
+    x[6] = -np.inf                                 # 500 survivors spread over the row
+    x[6, rng.choice(V, 500, replace=False)] = rng.normal(0, 3, 500).astype(np.float32)
+    P[6].update(top_k=0, min_p=0.01)
+    for i, k in ((7, 129), (8, 300), (9, 511), (10, 512), (11, 1500), (12, V - 5)):
+        P[i].update(top_k=k, top_p=0.97)           # larger k: by sorted list, by keys alone, by the big-row engine
+    top = np.argsort(-x[13])[:64]                  # bans and biases in the top groups
+    P[13].update(ban=[int(t) for t in top[:30]], bias=[(int(top[40]), 9.0), (int(top[41]), -9.0), (7, 30.0), (7, -4.0)])
+    P[14].update(counts=[(int(t), int(c)) for t, c in zip(rng.choice(V, 1500, replace=False), rng.integers(1, 4, 1500))],
+                 presence=0.4, frequency=0.3, repeat=1.2)   # lists longer than the registers hold
+    x[15, [5, V // 3, V - 2]] = 30.0               # greedy: the last of the equal maxima
+    P[15].update(temperature=0.0)
+    x[16] = np.where(rng.random(V) < 0.5, np.float32(0.0), np.float32(-0.0))   # zeros of both signs at the threshold
+    x[17, 11] = np.nan                             # streamed: NaN
+    x[18, V // 2] = np.inf
+    P[19].update(temperature=0.0, counts=[(int(np.argmax(x[19])), 1)], presence=50.0)   # greedy, the maximum penalised
+    return x, P
+
+
+@pytest.mark.parametrize("V", [4095, 4096, 4099, 50257, 81920, 81921, 151936, 163844])
+def test_lists_from_group_maxima(V):
+    x, params = _case(V)
+    print(f"[case] group maxima V={V}", flush=True)
+    errs = compare(x, params, _run_padded(x, params))
+    assert not errs, "\n".join(errs[:20])
+
+
+def _run_padded(x, params, allow=None):
+    """run_gpu for widths that are no multiple of 4 (rows padded in memory)."""
+    import torch
+
+    from tests.gpu_util import ctx, make_rows
+    from zllm_amd.engine import BatchSampler
+    B, V = x.shape
+    c = ctx(max(64, B), max(151936, V))
+    xs = torch.zeros((B, (V + 3) // 4 * 4), device="cuda")
+    xs[:, :V] = torch.from_numpy(x)
+    bs = BatchSampler(c)
+    ab = torch.from_numpy(allow).cuda() if allow is not None else None
+    out = bs.run(xs[:, :V], bs.pack(xs[:, :V], make_rows(params)), ab)
+    torch.cuda.synchronize()
+    return {k: v.cpu().numpy() for k, v in out.items()}
+
+
+@pytest.mark.parametrize("V", [4096, 50257, 151936])
+def test_lists_under_masks(V):
+    """Allowed sets of 0 to most of the row, adjacent (all in the groups of a
+    few waves) and spread, gathered and not, with bans and penalties inside."""
+    rng = np.random.default_rng(V + 1)
+    sizes = [1, 20, 27, 28, 300, 512, 513, 1000, 1024, 2048, 2049, min(V // 2, 30000)]
+    B = 2 * len(sizes)
+    x = rng.normal(0, 2, (B, V)).astype(np.float32)
+    allow = np.zeros((B, V), bool)
+    P = []
+    for i in range(B):
+        n = sizes[i // 2]
+        ids = rng.choice(V, n, replace=False) if i % 2 else (np.arange(n) + V // 3) % V
+        allow[i, ids] = True
+        P.append(dict(temperature=[0.8, 1.0, 0.0][i % 3], top_k=[0, 30, 400][i // 3 % 3], top_p=0.9, top_logprobs=20,
+                      seed=i, masked=True, ban=[int(t) for t in ids[:n // 10]],
+                      counts=[(int(t), 1) for t in ids[n // 2:n // 2 + 40]], presence=0.5))
+    bits = np.zeros((B, (V + 31) // 32), np.uint32)
+    for i in range(B):
+        b = np.packbits(np.pad(allow[i], (0, -V % 32)), bitorder="little")
+        bits[i] = b.view(np.uint32)
+    print(f"[case] group maxima under masks V={V}", flush=True)
+    out = _run_padded(x, P, bits.view(np.int32))
+    refs = [oracle_row(x[i], P[i], allow[i]) for i in range(B)]
+    errs = compare(x, P, out, allow=allow, refs=refs)
+    assert not errs, "\n".join(errs[:20])
 
 
 @pytest.mark.parametrize("V", [4092, 151936])

@@ -16,13 +16,16 @@
 //       first ZS_PATCH_LDS entries in LDS, the rest in row scratch), ranked by
 //       a bitmap of the patched ids with per-word prefix counts, and stored
 //       for the later kernels;
-//   P1  one read of the logits: observer maximum / NaN / +inf, sampler maximum,
-//       finite count and flags, greedy argmax (last maximal element, a NaN
-//       restarts the fold: sampler.rs:35-43), and candidate lists kept in LDS
-//       behind a rising threshold: the observers' top entries by (x~ desc, id
-//       asc) for top_logprobs / margin, the sampler's top-k by (z desc, id asc)
-//       (sampler.rs:53-64: its k-th key is the threshold), or every finite z
-//       when no top-k applies and at most ZS_SMALL_CAP are finite;
+//   P1  the row's maxima and candidate lists (the observers' top entries by
+//       (x~ desc, id asc) for top_logprobs / margin; the sampler's top-k by
+//       (z desc, id asc), sampler.rs:53-64: its k-th key is the threshold; or
+//       every finite z when no top-k applies and at most ZS_SMALL_CAP are
+//       finite) from the group maxima that zs_k_scan took over the whole GPU
+//       (rw_groups), or from a masked row's gathered ids. Rows these cannot
+//       serve (narrow rows, T = inf, NaN, lists that would overflow) read
+//       their logits here, keeping the lists in LDS behind a rising
+//       threshold (greedy argmax: the last maximal element, a NaN restarts
+//       the fold, sampler.rs:35-43);
 //   decisions: greedy / non-finite rows get their token; rows whose survivors
 //       fit ZS_SMALL_CAP are sampled exactly by one wave (small_path_wave);
 //       other rows are "big" and continue in zs_sample.hip;
@@ -50,11 +53,6 @@ __device__ unsigned long long rw_dbg[16];
 #define RW_G 2048          // ids per tile: one float4 per thread
 #define RW_BUF 2048        // candidate buffer entries (per list)
 #define RW_KEEP 1024       // a list above this is compacted to its top K
-// per (row, half) slot of a split row: statistics, then the observers' and
-// the sampler's list entries
-#define RW_PART_O 16
-#define RW_PART_S (RW_PART_O + 32)
-#define RW_PART (RW_PART_S + ZS_SMALL_CAP)
 
 struct rw_shared {
     uint32_t pid[4096];             // the patch list's head (ZS_PATCH_LDS): ids (sorted) | flags << 30
@@ -75,7 +73,7 @@ struct rw_shared {
     float fcut[2];                  // largest values cut from the lists
     unsigned long long rl[RW_NW];
     uint32_t n_surv, tok;
-    uint32_t merge;                 // split rows: the halves that finished before this one
+    uint32_t n_gl;                  // groups listed by rw_groups
     uint32_t ovf[3];                // first tile that lost a list entry, per group slot
     uint32_t thr_o, thr_s;          // candidate admission thresholds (keys)
     float fsh;
@@ -125,6 +123,18 @@ __device__ __forceinline__ uint32_t rw_wave_sum(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// Inclusive scan of a u32 over the wave (no overflow check): shifts inside
+// each row of 16 lanes, then the rows by broadcasts.
+__device__ __forceinline__ uint32_t rw_wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);    // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);    // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);    // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);    // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
 // Workgroup barrier that orders LDS accesses only. __syncthreads() also waits
 // for every outstanding global load of the calling wave, which would drain the
 // loads the tile loops keep in flight ahead of the tile being processed.
@@ -169,8 +179,8 @@ __device__ __forceinline__ uint32_t rw_rank(uint32_t id, uint32_t words) {
     return rw_pbits[words + (id >> 5)] + __popc(wd & ((1u << (id & 31)) - 1u));
 }
 
-__device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const zs_row_params& P, uint32_t& has_y, rw_shared& sh,
-                                          bool wr = true) {
+#define RW_PE 2   // list entries a thread keeps in registers
+__device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const zs_row_params& P, rw_shared& sh) {
     const zs_batch& b = a.b;
     const uint32_t t = threadIdx.x, V = b.V;
     const uint32_t words = (V + 31) / 32;
@@ -178,18 +188,66 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
     uint32_t* dup = rw_pbits + 3 * words;
     const uint32_t ban0 = b.d_ban_off ? b.d_ban_off[r] : 0, ban1 = b.d_ban_off ? b.d_ban_off[r + 1] : 0;
     const uint32_t bi0 = b.d_bias_off ? b.d_bias_off[r] : 0, bi1 = b.d_bias_off ? b.d_bias_off[r + 1] : 0;
-    for (uint32_t i = t; i < words; i += RW_NT) {
-        rw_pbits[i] = 0u;
-        if (bi1 != bi0) { seen[i] = 0u; dup[i] = 0u; }
-    }
     uint32_t c0 = b.d_cnt_off ? b.d_cnt_off[r] : 0, c1 = b.d_cnt_off ? b.d_cnt_off[r + 1] : 0;
     if (!zs_penalty_active(P)) c1 = c0;  // counts only matter when penalties are active
-    const uint32_t nb = ban1 - ban0, nbi = bi1 - bi0, nc = c1 - c0;
+    const uint32_t nb = ban1 - ban0, nbi = bi1 - bi0, nc = c1 - c0, ne = nb + nbi + nc;
     const uint32_t nsub = (V + ZS_SUB - 1) / ZS_SUB;
     uint32_t* psub = a.p_sub + (size_t)r * (a.max_subs + 1);
     uint32_t* out_id = a.p_id + (size_t)r * a.pstride;
     uint32_t* out_fl = a.p_flags + (size_t)r * a.pstride;
     float* out_y = a.p_y + (size_t)r * a.pstride;
+    if (ne == 0) {
+        // (the bitmap is read only for rows with patches)
+        if (t == 0) a.p_cnt[r] = 0;
+        for (uint32_t j = t; j <= nsub; j += RW_NT) psub[j] = 0;
+        __syncthreads();
+        return 0;
+    }
+    // Entry i of the row's three lists (bans, biases, counts in this order):
+    // its id and its value (bias or count, as bits). The first RW_PE entries
+    // of a thread stay in registers with their logit, so that every list
+    // element of a row of up to 1024 is loaded once, all loads at once: the
+    // lists re-read per step and the logits gathered word by word took 13 us
+    // on 256 counts, 6 us now.
+    const bool masked = (P.flags & ZS_ROW_MASKED) && b.d_allow_bits;
+    auto id_of = [&](uint32_t i) -> uint32_t {
+        return i < nb ? b.d_ban_ids[ban0 + i] : i < nb + nbi ? b.d_bias_ids[bi0 + i - nb] : b.d_cnt_ids[c0 + i - nb - nbi];
+    };
+    auto val_of = [&](uint32_t i) -> uint32_t {
+        return i < nb ? 0u : i < nb + nbi ? zs_f2u(b.d_bias_vals[bi0 + i - nb]) : b.d_cnt_vals[c0 + i - nb - nbi];
+    };
+    auto x_of = [&](uint32_t id) -> float {
+        const float x = b.d_logits[(size_t)r * b.ld + id];
+        return masked && !zs_allowed_bit(b, r, id) ? -INFINITY : x;
+    };
+    uint32_t eid[RW_PE], ev[RW_PE];
+    float ex[RW_PE];
+#pragma unroll
+    for (int u = 0; u < RW_PE; u++) {
+        const uint32_t i = t + (uint32_t)u * RW_NT;
+        eid[u] = i < ne ? id_of(i) : 0xffffffffu;
+        ev[u] = i < ne ? val_of(i) : 0u;
+    }
+    for (uint32_t i = t; i < words; i += RW_NT) {
+        rw_pbits[i] = 0u;
+        if (nbi) { seen[i] = 0u; dup[i] = 0u; }
+    }
+#pragma unroll
+    for (int u = 0; u < RW_PE; u++) ex[u] = eid[u] < V ? x_of(eid[u]) : 0.0f;
+    // calls f(i, id, value, x) for this thread's entries of [i0, i1) with an id
+    // in the row
+    auto each = [&](uint32_t i0, uint32_t i1, auto&& f) {
+#pragma unroll
+        for (int u = 0; u < RW_PE; u++) {
+            const uint32_t i = t + (uint32_t)u * RW_NT;
+            if (i >= i0 && i < i1 && eid[u] < V) f(i, eid[u], ev[u], [&] { return ex[u]; });
+        }
+        for (uint32_t i = t + RW_PE * RW_NT; i < i1; i += RW_NT) {
+            if (i < i0) continue;
+            const uint32_t id = id_of(i);
+            if (id < V) f(i, id, val_of(i), [&] { return x_of(id); });
+        }
+    };
     // entry k: in LDS (ids and flags in sh.pid, y in sh.py) for the list's
     // head, in row scratch past it; the head is copied out at the end
     auto FL = [&](uint32_t k) -> uint32_t { return k < ZS_PATCH_LDS ? sh.pid[k] >> RW_PF_SHIFT : out_fl[k]; };
@@ -202,86 +260,90 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
         if (k < ZS_PATCH_LDS) sh.py[k] = y;
         else out_y[k] = y;
     };
-    __syncthreads();
+    rw_bar();
     // the patched ids, and the bias ids that occur more than once
-    for (uint32_t i = t; i < nb + nbi + nc; i += RW_NT) {
-        uint32_t id;
-        if (i < nb) id = b.d_ban_ids[ban0 + i];
-        else if (i < nb + nbi) id = b.d_bias_ids[bi0 + i - nb];
-        else id = b.d_cnt_ids[c0 + i - nb - nbi];
-        if (id >= V) continue;
+    each(0, ne, [&](uint32_t i, uint32_t id, uint32_t, auto&&) {
         const uint32_t bit = 1u << (id & 31);
         atomicOr(&rw_pbits[id >> 5], bit);
         if (i >= nb && i < nb + nbi && (atomicOr(&seen[id >> 5], bit) & bit)) atomicOr(&dup[id >> 5], bit);
-    }
-    __syncthreads();
-    // per-word prefix counts of the bitmap (words / RW_NT words per thread at most 8)
+    });
+    rw_bar();
+    // per-word prefix counts of the bitmap: each wave its own stretch of
+    // words, 64 at a time
     uint32_t np;
     {
-        const uint32_t per = (words + RW_NT - 1) / RW_NT;
-        const uint32_t w0 = t * per;
+        const uint32_t lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+        const uint32_t per = ((words + RW_NT - 1) / RW_NT) * 64u, w0 = wid * per, w1 = min(w0 + per, words);
         uint32_t c = 0;
-        for (uint32_t w = w0; w < min(w0 + per, words); w++) c += __popc(rw_pbits[w]);
-        uint32_t run = block_excl_scan_u<RW_NT>(c, sh.ru[2], &np);
-        for (uint32_t w = w0; w < min(w0 + per, words); w++) {
-            rw_pbits[words + w] = run;
-            // the list in id order: every patched id with its masked logit
-            uint32_t m = rw_pbits[w];
-            while (m) {
-                const uint32_t id = w * 32 + (uint32_t)__builtin_ctz(m);
-                m &= m - 1u;
-                float x = b.d_logits[(size_t)r * b.ld + id];
-                if ((P.flags & ZS_ROW_MASKED) && b.d_allow_bits && !zs_allowed_bit(b, r, id)) x = -INFINITY;
-                if (run < ZS_PATCH_LDS) {
-                    sh.pid[run] = id;
-                    sh.py[run] = x;
-                } else {
-                    out_id[run] = id;
-                    out_fl[run] = 0u;
-                    out_y[run] = x;
-                }
-                run++;
-            }
+        for (uint32_t w = w0 + lane; w < w1; w += 64) c += __popc(rw_pbits[w]);
+        c = rw_wave_sum(c);
+        if (lane == 0) sh.ru[2][wid] = c;
+        rw_bar();
+        uint32_t run = 0;
+        np = 0;
+#pragma unroll
+        for (int w = 0; w < RW_NW; w++) {
+            const uint32_t k = sh.ru[2][w];
+            run += (uint32_t)w < wid ? k : 0u;
+            np += k;
+        }
+        for (uint32_t wb = w0; wb < w1; wb += 64) {
+            const uint32_t w = wb + lane;
+            const uint32_t k = w < w1 ? __popc(rw_pbits[w]) : 0u;
+            const uint32_t inc = rw_wave_scan(k);
+            if (w < w1) rw_pbits[words + w] = run + inc - k;
+            run += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
         }
     }
     np = rw_uni(np);
+    rw_bar();
+    // the list in id order: every patched id with its masked logit
+    each(0, ne, [&](uint32_t, uint32_t id, uint32_t, auto&& x) {
+        const uint32_t k = rw_rank(id, words);
+        if (k < ZS_PATCH_LDS) {
+            sh.pid[k] = id;
+            sh.py[k] = x();
+        } else {
+            out_id[k] = id;
+            out_fl[k] = 0u;
+            out_y[k] = x();
+        }
+    });
     __syncthreads();
     // bans (a banned x~ and y are -inf)
-    for (uint32_t i = t; i < nb; i += RW_NT) {
-        const uint32_t id = b.d_ban_ids[ban0 + i];
-        if (id >= V) continue;
-        const uint32_t k = rw_rank(id, words);
-        SET_FL(k, ZS_PF_BAN);
-        SET_Y(k, -INFINITY);
+    if (nb) {
+        each(0, nb, [&](uint32_t, uint32_t id, uint32_t, auto&&) {
+            const uint32_t k = rw_rank(id, words);
+            SET_FL(k, ZS_PF_BAN);
+            SET_Y(k, -INFINITY);
+        });
+        __syncthreads();
     }
-    __syncthreads();
     // logit_bias (decode_ctrl.rs:108-112): an id met once takes its bias in
     // parallel; the entries of an id met more than once are added by one
     // thread in list order
-    for (uint32_t i = t; i < nbi; i += RW_NT) {
-        const uint32_t id = b.d_bias_ids[bi0 + i];
-        if (id >= V || ((dup[id >> 5] >> (id & 31)) & 1u)) continue;
-        const uint32_t k = rw_rank(id, words);
-        SET_Y(k, Y(k) + b.d_bias_vals[bi0 + i]);
-        SET_FL(k, FL(k) | ZS_PF_Y);
-    }
-    if (t == 0) {
-        for (uint32_t i = 0; i < nbi; i++) {
-            const uint32_t id = b.d_bias_ids[bi0 + i];
-            if (id >= V || !((dup[id >> 5] >> (id & 31)) & 1u)) continue;
+    if (nbi) {
+        each(nb, nb + nbi, [&](uint32_t, uint32_t id, uint32_t v, auto&&) {
+            if ((dup[id >> 5] >> (id & 31)) & 1u) return;
             const uint32_t k = rw_rank(id, words);
-            SET_Y(k, Y(k) + b.d_bias_vals[bi0 + i]);
+            SET_Y(k, Y(k) + zs_u2f(v));
             SET_FL(k, FL(k) | ZS_PF_Y);
+        });
+        if (t == 0) {
+            for (uint32_t i = 0; i < nbi; i++) {
+                const uint32_t id = b.d_bias_ids[bi0 + i];
+                if (id >= V || !((dup[id >> 5] >> (id & 31)) & 1u)) continue;
+                const uint32_t k = rw_rank(id, words);
+                SET_Y(k, Y(k) + b.d_bias_vals[bi0 + i]);
+                SET_FL(k, FL(k) | ZS_PF_Y);
+            }
         }
+        __syncthreads();
     }
-    __syncthreads();
     // penalty (decode_ctrl.rs:113-125): repeat, then frequency * count + presence
     // (the count map holds each id once)
-    for (uint32_t i = t; i < nc; i += RW_NT) {
-        const uint32_t id = b.d_cnt_ids[c0 + i];
-        if (id >= V) continue;
+    each(nb + nbi, ne, [&](uint32_t, uint32_t id, uint32_t cnt, auto&&) {
         const uint32_t k = rw_rank(id, words);
-        const uint32_t cnt = b.d_cnt_vals[c0 + i];
         float y = Y(k);
         if (P.repeat != 1.0f) {
             if (y > 0.0f) y = y / P.repeat;
@@ -292,25 +354,18 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
         y = __fsub_rn(y, pen_v);
         SET_Y(k, y);
         SET_FL(k, FL(k) | ZS_PF_Y);
-    }
+    });
     __syncthreads();
     // the list's head out to row scratch (the later kernels read it there)
-    uint32_t hy = 0;
-    for (uint32_t k = t; k < np; k += RW_NT) {
-        const uint32_t fl = FL(k);
-        hy |= (fl & ZS_PF_Y) ? 1u : 0u;
-        if (wr && k < ZS_PATCH_LDS) {
-            out_id[k] = sh.pid[k] & ((1u << RW_PF_SHIFT) - 1u);
-            out_fl[k] = fl;
-            out_y[k] = sh.py[k];
-        }
+    for (uint32_t k = t; k < min(np, (uint32_t)ZS_PATCH_LDS); k += RW_NT) {
+        out_id[k] = sh.pid[k] & ((1u << RW_PF_SHIFT) - 1u);
+        out_fl[k] = sh.pid[k] >> RW_PF_SHIFT;
+        out_y[k] = sh.py[k];
     }
-    has_y = block_or_u<RW_NT>(hy, sh.ru[1]);
-    if (wr && t == 0) a.p_cnt[r] = np;
+    if (t == 0) a.p_cnt[r] = np;
     // first patch of every 1024-id sub-chunk (read by the sum, big-row and
     // output kernels): the bitmap's prefix count at the sub-chunk start
-    for (uint32_t j = t; wr && j <= nsub; j += RW_NT) psub[j] = j * (ZS_SUB / 32) < words ? rw_pbits[words + j * (ZS_SUB / 32)] : np;
-    __syncthreads();
+    for (uint32_t j = t; j <= nsub; j += RW_NT) psub[j] = j * (ZS_SUB / 32) < words ? rw_pbits[words + j * (ZS_SUB / 32)] : np;
     return (int)np;
 }
 
@@ -477,13 +532,13 @@ struct rw_list {
 // above the first bit where the members' keys differ are skipped; each pass
 // histograms one digit of the members that share the bits above it with the
 // K1-th smallest, and one wave picks the digit where the count reaches K1. It stops once the members up to and including the chosen digit
-// number at most RW_SEL_CAP (always by the last digit: entries are
-// distinct); those are gathered to the front and sorted by one wave.
+// number at most the cap (always by the last digit: entries are distinct;
+// K1 <= RW_SEL_MAX); those are gathered to the front and sorted, by one wave
+// up to RW_SEL_CAP, else by the workgroup.
 #define RW_SEL_CAP 256
+#define RW_SEL_MAX 512
 #define RW_SEL_E (RW_BUF / RW_NT)   // list entries per thread
 static_assert(RW_BUF % RW_NT == 0, "the list is spread evenly over the threads");
-static_assert(RW_PART == ZS_ROW_PART && ZS_OBS_CAND <= RW_PART_S - RW_PART_O && ZS_KS + 1 <= ZS_SMALL_CAP,
-              "the split rows' slots hold the lists");
 
 __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, uint32_t idlim) {
     rw_shared& sh = rw_sh;
@@ -524,10 +579,11 @@ __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, u
     c = rw_uni(c);
     if (c == 0) return 0;   // every thread read buf before the barrier above
     const uint32_t need = min(c, K1);
+    const uint32_t cap = K1 <= RW_SEL_CAP ? RW_SEL_CAP : RW_SEL_MAX;
     // the selected members: (v >> shift) <= (pre >> shift)
     int shift = 0;
     unsigned long long pre = NONE - 1ull;   // every member (ids < 2^32 - 1)
-    if (c > RW_SEL_CAP) {
+    if (c > cap) {
         lo = rw_uni(lo); hi = rw_uni(hi);
         shift = lo != hi ? 32 + ((31 - __clz(lo ^ hi)) & ~7) : 24;
         pre = ((unsigned long long)lo << 32) & ~((2ull << (shift + 7)) - 1ull);   // the bits above the digit
@@ -572,7 +628,7 @@ __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, u
             const uint32_t dg = rw_uni(sh.sel_mm[0][0]), cb = rw_uni(sh.sel_mm[2][0]);
             below = rw_uni(sh.sel_mm[1][0]);
             pre |= (unsigned long long)dg << shift;
-            if (below + cb <= RW_SEL_CAP || shift == 0) break;
+            if (below + cb <= cap || shift == 0) break;
             shift -= 8;
         }
     }
@@ -586,8 +642,15 @@ __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, u
     }
     __syncthreads();
     const uint32_t m = rw_uni(sh.sel_n);
-    if (wid == 0) rw_wave_sort(buf, m);
-    __syncthreads();
+    if (m <= RW_SEL_CAP) {
+        if (wid == 0) rw_wave_sort(buf, m);
+        __syncthreads();
+    } else {
+        static_assert(RW_SEL_MAX == RW_NT, "one entry per thread");
+        if (t >= m) buf[t] = NONE;
+        __syncthreads();
+        block_sort_reg_u64<RW_NT, 1>(buf, RW_SEL_MAX);
+    }
     return c;
 }
 
@@ -654,58 +717,182 @@ __device__ __noinline__ uint32_t rw_gather_allowed(const float* row, const uint3
                                                    float* cx, const uint32_t* gfl, const float* gy) {
     rw_shared& sh = rw_sh;
     const uint32_t t = threadIdx.x, words = (V + 31) / 32;
-    const uint32_t per = (words + RW_NT - 1) / RW_NT, w0 = t * per, w1 = min(w0 + per, words);
+    const uint32_t lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    // each wave its own stretch of words, 64 at a time: the counts of the
+    // waves, then every allowed id to its place in an LDS list, then their
+    // values, all of a thread's loads at once (a loop per thread over its
+    // words with a load per id took 10 us on JSON masks)
+    const uint32_t per = ((words + RW_NT - 1) / RW_NT) * 64u, w0 = wid * per, w1 = min(w0 + per, words);
     auto word = [&](uint32_t w) {
-        uint32_t a = allow[w];
+        uint32_t a = w < w1 ? rw_gload(allow + w) : 0u;
         if (w == words - 1 && (V & 31)) a &= (1u << (V & 31)) - 1u;
         return a;
     };
-    uint32_t c = 0;
-    for (uint32_t w = w0; w < w1; w++) c += __popc(word(w));
-    uint32_t n;
-    uint32_t pos = block_excl_scan_u<RW_NT>(c, sh.ru[4], &n);
+    constexpr uint32_t NWD = 10;   // words a thread keeps in registers
+    uint32_t aw[NWD], c = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < NWD; i++) aw[i] = word(w0 + lane + 64u * i);
+#pragma unroll
+    for (uint32_t i = 0; i < NWD; i++) c += __popc(aw[i]);
+    for (uint32_t wb = w0 + 64u * NWD; wb < w1; wb += 64) c += __popc(word(wb + lane));
+    c = rw_wave_sum(c);
+    if (lane == 0) sh.ru[4][wid] = c;
+    rw_bar();
+    uint32_t n = 0, pos = 0;
+#pragma unroll
+    for (int w = 0; w < RW_NW; w++) {
+        const uint32_t k = sh.ru[4][w];
+        pos += (uint32_t)w < wid ? k : 0u;
+        n += k;
+    }
     n = rw_uni(n);
+    rw_bar();
     if (n == 0 || n > RW_BUF || n > V / 4 || V < 16) return 0;   // V >= 16: 3 round_up(n, 4) + 3 values fit 2 V
     const uint32_t n4 = (n + 3) & ~3u;
     float* cy = cx + n4;
-    for (uint32_t w = w0; w < w1; w++) {
-        uint32_t a = word(w);
+    uint32_t* lid = reinterpret_cast<uint32_t*>(sh.u.b.o);   // RW_BUF ids (the list is built after)
+    auto place = [&](uint32_t a, uint32_t wb) {
+        const uint32_t k = __popc(a), inc = rw_wave_scan(k);
+        uint32_t p = pos + inc - k;
         while (a) {
-            const uint32_t id = w * 32 + (uint32_t)__builtin_ctz(a);
+            lid[p++] = (wb + lane) * 32 + (uint32_t)__builtin_ctz(a);
             a &= a - 1u;
-            float x = row[id], y = x;
-            if (np) {
-                const uint32_t wd = rw_pbits[id >> 5];
-                if ((wd >> (id & 31)) & 1u) {
-                    const uint32_t rank = rw_pbits[words + (id >> 5)] + __popc(wd & ((1u << (id & 31)) - 1u));
-                    const uint32_t fl = rank < ZS_PATCH_LDS ? sh.pid[rank] >> RW_PF_SHIFT : gfl[rank];
-                    if (fl & ZS_PF_BAN) { x = -INFINITY; y = -INFINITY; }
-                    if (fl & ZS_PF_Y) y = rank < ZS_PATCH_LDS ? sh.py[rank] : gy[rank];
-                }
-            }
-            cx[pos] = x;
-            cy[pos] = y;
-            reinterpret_cast<uint32_t*>(cy + n4)[pos] = id;
-            pos++;
         }
+        pos += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    };
+    for (uint32_t i = 0; i < NWD; i++) {
+        if (w0 + 64u * i >= w1) break;   // (uniform)
+        uint32_t a = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < NWD; j++) a = j == i ? aw[j] : a;
+        place(a, w0 + 64u * i);
+    }
+    for (uint32_t wb = w0 + 64u * NWD; wb < w1; wb += 64) place(word(wb + lane), wb);
+    rw_bar();
+    constexpr uint32_t NE = RW_BUF / RW_NT;
+    uint32_t id[NE];
+    float xv[NE];
+#pragma unroll
+    for (uint32_t e = 0; e < NE; e++) {
+        id[e] = lid[min(t + e * RW_NT, n - 1u)];
+        xv[e] = rw_gload(row + id[e]);
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < NE; e++) {
+        const uint32_t i = t + e * RW_NT;
+        if (i >= n) continue;
+        float x = xv[e], y = x;
+        if (np) {
+            const uint32_t wd = rw_pbits[id[e] >> 5];
+            if ((wd >> (id[e] & 31)) & 1u) {
+                const uint32_t rank = rw_pbits[words + (id[e] >> 5)] + __popc(wd & ((1u << (id[e] & 31)) - 1u));
+                const uint32_t fl = rank < ZS_PATCH_LDS ? sh.pid[rank] >> RW_PF_SHIFT : gfl[rank];
+                if (fl & ZS_PF_BAN) { x = -INFINITY; y = -INFINITY; }
+                if (fl & ZS_PF_Y) y = rank < ZS_PATCH_LDS ? sh.py[rank] : gy[rank];
+            }
+        }
+        cx[i] = x;
+        cy[i] = y;
+        reinterpret_cast<uint32_t*>(cy + n4)[i] = id[e];
     }
     if (t < n4 - n) { cx[n + t] = -INFINITY; cy[n + t] = -INFINITY; }
     __syncthreads();
     return n;
 }
 
-// Exact sampling of a small survivor set by wave 0 (token to sh.tok).
-__device__ __noinline__ void rw_small(uint64_t seed, uint64_t counter, uint32_t V, const zs_row_params& P, uint32_t nsv,
-                                      float zmax, rw_shared& sh) {
-    const uint32_t tk = nsv <= 64 ? small_path_wave<1>(seed, counter, V, P, nsv, zmax, sh.sval, sh.sidx)
-                                  : small_path_wave<ZS_SMALL_CAP / 64>(seed, counter, V, P, nsv, zmax, sh.sval, sh.sidx);
-    if (threadIdx.x == 0) sh.tok = tk;
+// Exact sampling of 65 to ZS_SMALL_CAP survivors by the whole workgroup, one
+// survivor per thread: the steps of small_path_wave with the two sorts spread
+// over the waves (the sequential sums stay with wave 0, over LDS copies).
+// One wave with 8 survivors per lane spent 6.4 us on each sort and 35 us in
+// all on 512 survivors, this 18 us. Called by every thread (token to sh.tok).
+__device__ __noinline__ void rw_small_wg(uint64_t seed, uint64_t counter, uint32_t V, float top_p, float min_p, uint32_t n,
+                                         float m) {
+    rw_shared& sh = rw_sh;
+    const uint32_t t = threadIdx.x;
+    unsigned long long* kb = sh.u.b.s;   // (the lists are no longer needed)
+    const bool live = t < n;
+    static_assert(ZS_SMALL_CAP == RW_NT, "one survivor per thread");
+    uint32_t np2 = 128;
+    while (np2 < n) np2 <<= 1;
+    // survivors by index
+    if (t < np2) kb[t] = live ? (((unsigned long long)sh.sidx[t] << 32) | zs_f2u(sh.sval[t])) : ~0ull;
+    __syncthreads();
+    block_sort_reg_u64<RW_NT, 1>(kb, np2);
+    const unsigned long long e0 = live ? kb[t] : 0ull;
+    const uint32_t id = (uint32_t)(e0 >> 32);
+    float p = live ? zs_expf(zs_u2f((uint32_t)e0) - m) : 0.0f;
+    // s0 + v of thread 0 + v of thread 1 + ... (sampler.rs:68, 80, 107), or
+    // the first thread where the sum reaches thresh (to sh.n_surv)
+    auto scan = [&](float v, float s0, float thresh) {
+        if (live) sh.sval[t] = v;
+        __syncthreads();
+        if (t < 64) {
+            float s;
+            const uint32_t i = serial_scan_f(sh.sval, n, s0, thresh, &s);
+            if (t == 0) { sh.fsh = s; sh.n_surv = i; }
+        }
+        __syncthreads();
+    };
+    // softmax (sampler.rs:67-69)
+    scan(p, -0.0f, NAN);
+    p = p / sh.fsh;
+    // min-p (sampler.rs:72-88)
+    if (min_p > 0.0f) {
+        const float pm = block_max_f<RW_NT>(live ? p : 0.0f, sh.rf[0]);
+        if (p < min_p * pm) p = 0.0f;
+        scan(p, 0.0f, NAN);
+        const float kept = sh.fsh;
+        if (kept > 0.0f) p = p / kept;
+    }
+    // top-p (sampler.rs:91-115): cumsum in (p desc, idx asc) order
+    if (top_p < 1.0f) {
+        uint32_t vstar = 0, istar = 0xffffffffu;
+        const bool none = !(top_p > 0.0f);  // cumsum 0 >= top_p: nothing kept
+        if (!none) {
+            if (t < np2) kb[t] = live ? (((unsigned long long)(~zs_f2u(p)) << 32) | id) : ~0ull;
+            __syncthreads();
+            block_sort_reg_u64<RW_NT, 1>(kb, np2);
+            scan(live ? zs_u2f(~(uint32_t)(kb[t] >> 32)) : 0.0f, 0.0f, top_p);
+            const uint32_t i = sh.n_surv;
+            if (i < n) {
+                vstar = ~(uint32_t)(kb[i] >> 32);
+                istar = (uint32_t)kb[i];
+            }
+        }
+        const uint32_t pb = zs_f2u(p);
+        const bool keep = live && !none && (pb > vstar || (pb == vstar && id <= istar));
+        const float f = keep ? p : 0.0f;
+        scan(f, -0.0f, NAN);
+        const float sum = sh.fsh;
+        if (sum > 0.0f) p = f / sum;
+    }
+    // draw (sampler.rs:118-127); r == 0 stops at index 0 whatever its p
+    const float rr = zs_philox_uniform(seed, counter, 0u);
+    scan(p, 0.0f, rr);
+    if (live && t == sh.n_surv) sh.tok = id;
+    if (t == 0) {
+        if (rr <= 0.0f) sh.tok = 0;
+        else if (sh.n_surv >= n) sh.tok = V - 1;
+    }
+}
+
+// Exact sampling of a small survivor set (token to sh.tok): up to 64 by wave
+// 0, more by the workgroup. Called by every thread.
+__device__ __forceinline__ void rw_small(uint64_t seed, uint64_t counter, uint32_t V, const zs_row_params& P, uint32_t nsv,
+                                         float zmax, rw_shared& sh) {
+    if (nsv > 64) {
+        rw_small_wg(seed, counter, V, P.top_p, P.min_p, nsv, zmax);
+    } else if (threadIdx.x < 64) {
+        const uint32_t tk = small_path_wave<1>(seed, counter, V, P, nsv, zmax, sh.sval, sh.sidx);
+        if (threadIdx.x == 0) sh.tok = tk;
+    }
 }
 
 // The row of the j-th row workgroup: the unmasked rows in index order, then
-// the masked ones. Uniform.
-__device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j) {
-    if (!b.d_allow_bits || b.B > 4 * RW_NT) return j;
+// the masked ones, when there are more rows than CUs (a CU holds one of these
+// workgroups; with a CU for each the order changes nothing). Uniform.
+__device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, uint32_t ncu) {
+    if (!b.d_allow_bits || b.B <= ncu || b.B > 4 * RW_NT) return j;
     rw_shared& sh = rw_sh;
     const uint32_t t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
     const uint32_t nchunk = (b.B + RW_NT - 1) / RW_NT;
@@ -750,15 +937,448 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j) 
     return r;
 }
 
+
+// ---------------------------------------------------------------------------
+// P1 from group maxima. zs_k_scan (below) reads the row's logits once over the
+// whole GPU and leaves the key of the largest x~ of every group of 2^gshift
+// consecutive ids (mask applied, bans and biases not). Here the groups holding
+// a patched id are read again and the maxima of x~ and y corrected; then
+//   - with t0 a key that at least K groups reach, the first K entries of the
+//     row by (value desc, id asc) all have keys >= t0, and they lie in the
+//     groups whose maximum reaches t0: a few more than K of them;
+//   - only the ids of those groups are read again and listed.
+// A chain of dependent loads and LDS steps bounds it, not V. The streaming
+// loop with its admissions spent 50 us on half a row of 128256 ids; measured,
+// scan + row kernel against the streaming row kernel (us):
+//   1 x 32000 3 + 24 / 45, 64 x 128256 7 + 32 / 92, 256 x 151936 (half the rows
+//   masked) 23 + 47 / 133, 128 x 151936 masked 11 + 47 / 87.
+// Returns false (uniformly) for rows whose lists would overflow or that hold
+// a NaN: they take the streaming loop of zs_k_row.
+// ---------------------------------------------------------------------------
+#define RW_KWIDE 3072      // largest k whose threshold comes from the lists
+#define RW_WIDE (2 * RW_BUF)   // keys in the sampler list's place
+#define RW_GOBS (RW_BUF / 2)   // observers listed at most; the listed groups (u16) follow them in LDS
+#define RW_GL (RW_BUF * 2)     // listed groups at most
+#define RW_GF 14u              // a listed group: group | list flags << RW_GF
+#define RW_GPT 10          // groups per thread at most (zs_scan_gshift)
+struct rw_gst {
+    float omax, ymax, rejf;
+    unsigned long long gbest;
+    uint32_t n_o, n_s;
+    bool s_over;
+};
+__device__ __forceinline__ uint32_t rw_wave_umax(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));   // row_half_mirror
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));   // row_mirror
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));   // row_bcast:15
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));   // row_bcast:31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// Maximum over the 4, 8 or 16 adjacent lanes of a group (qs = 2, 3, 4; uniform).
+__device__ __forceinline__ uint32_t rw_lanes_umax(uint32_t v, uint32_t qs) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
+    if (qs >= 3) v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));   // row_half_mirror
+    if (qs >= 4) v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));   // row_mirror
+    return v;
+}
+// Key of a group maximum: -0 and +0 alike, a NaN above everything.
+#define RW_KNAN 0xffffffffu
+__device__ __forceinline__ uint32_t rw_gkey(float m, bool nan) { return nan ? RW_KNAN : zs_total_key(m + 0.0f); }
+
+// x~ and y of the 4 ids from idx0 (a multiple of 4; ids >= V read -inf).
+__device__ __forceinline__ void rw_load4(const rw_row& R, uint32_t idx0, const float4& v, uint32_t w, float (&x)[4],
+                                         float (&y)[4], const rw_shared& sh) {
+    const uint32_t aw = (w >> (idx0 & 31)) | R.amask;
+    x[0] = (aw & 1u) ? v.x : -INFINITY;
+    x[1] = (aw & 2u) ? v.y : -INFINITY;
+    x[2] = (aw & 4u) ? v.z : -INFINITY;
+    x[3] = (aw & 8u) ? v.w : -INFINITY;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (idx0 + q >= R.V) x[q] = -INFINITY;
+        y[q] = x[q];
+    }
+    if (R.np) {
+        const uint32_t wd = rw_pbits[min(idx0 >> 5, R.words - 1)];
+        const uint32_t pb = idx0 < R.V ? (wd >> (idx0 & 31)) & 15u : 0u;
+        if (pb) rw_patch4<false>(R, idx0, pb, wd, x, y, sh);
+    }
+}
+__device__ __forceinline__ float4 rw_fetch4(const rw_row& R, uint32_t idx0, uint32_t& w) {
+    typedef float rw_f4 __attribute__((ext_vector_type(4)));
+    const uint32_t ia = min(idx0, R.ldm4);
+    const rw_f4 v = rw_gload(reinterpret_cast<const rw_f4*>(R.row + ia));
+    w = rw_gload(R.allow_or_row + min(ia >> 5, R.wmax));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// The K-th largest of n >= K keys in LDS (radix selection, 8-bit digits): the
+// words from offset `off` of the dynamic LDS (the group maxima), or
+// (off = ~0) of the sampler list's place. Called by every thread; uniform.
+__device__ __noinline__ uint32_t rw_kth_key(uint32_t off, uint32_t n, uint32_t K) {
+    rw_shared& sh = rw_sh;
+    const bool list = off == 0xffffffffu;
+    const uint32_t t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    uint32_t pre = 0, need = K;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+        if (t < 256) sh.sel_hist[0][t] = 0;
+        __syncthreads();
+        for (uint32_t i = t; i < n; i += RW_NT) {
+            const uint32_t k = list ? reinterpret_cast<uint32_t*>(sh.u.b.s)[i] : rw_pbits[off + i];
+            if (shift == 24 || (k >> (shift + 8)) == (pre >> (shift + 8))) atomicAdd(&sh.sel_hist[0][(k >> shift) & 255u], 1u);
+        }
+        __syncthreads();
+        if (wid == 0) {
+            // digits in descending order: lane l holds 255 - 4l .. 252 - 4l
+            uint32_t h[4], s4 = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) { h[q] = sh.sel_hist[0][255u - 4u * lane - (uint32_t)q]; s4 += h[q]; }
+            const uint32_t inc = wave_incl_scan_u(s4);
+            const unsigned long long hit = __ballot(inc >= need);
+            const uint32_t L = (uint32_t)__ffsll((long long)hit) - 1u;   // one exists: n >= K
+            if (lane == L) {
+                uint32_t run = inc - s4;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (run + h[q] >= need) {
+                        sh.sel_st[0] = 255u - 4u * lane - (uint32_t)q;
+                        sh.sel_st[1] = need - run;
+                        break;
+                    }
+                    run += h[q];
+                }
+            }
+        }
+        __syncthreads();
+        pre |= rw_uni(sh.sel_st[0]) << shift;
+        need = rw_uni(sh.sel_st[1]);
+        __syncthreads();
+    }
+    return pre;
+}
+
+__device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const rw_row& R, bool greedy, uint32_t smode,
+                                       uint32_t Ks, uint32_t Ko, rw_gst& G) {
+    rw_shared& sh = rw_sh;
+    const uint32_t t = threadIdx.x, wid = (uint32_t)zs_wid();
+    const uint32_t gs = a.gshift, ng = (R.V + (1u << gs) - 1u) >> gs;
+    uint32_t* gx = rw_pbits + 2 * R.words;   // (the bias bitmaps of rw_patches are no longer needed)
+    uint32_t* gy = gx + ng;
+    const uint32_t* gm = a.gmax + (size_t)r * a.gstride;
+    const uint32_t kinf = zs_total_key(-INFINITY);
+#ifdef ZS_WALK_DEBUG
+    unsigned long long rw_t0 = wall_clock64();
+#endif
+    {
+        uint32_t k[RW_GPT];
+#pragma unroll
+        for (int e = 0; e < RW_GPT; e++) k[e] = rw_gload(gm + min(t + (uint32_t)e * RW_NT, ng - 1u));
+#pragma unroll
+        for (int e = 0; e < RW_GPT; e++) {
+            const uint32_t i = t + (uint32_t)e * RW_NT;
+            if (i < ng) { gx[i] = k[e]; gy[i] = k[e]; }
+        }
+    }
+    if (t == 0) { sh.n_gl = 0; sh.sel_n = 0; sh.sel_st[2] = 0; sh.sel_st[3] = 0; }
+    __syncthreads();
+    // groups with patched ids are read again: the first patch of a group lists
+    // it, then one lane per 4 ids (the lanes of a group adjacent)
+    uint16_t* gl = reinterpret_cast<uint16_t*>(sh.u.b.o + RW_GOBS);
+    static_assert(RW_GL * sizeof(uint16_t) <= (RW_BUF - RW_GOBS) * sizeof(unsigned long long) &&
+                  RW_GPT * RW_NT <= 1u << RW_GF && ZS_PATCH_LDS <= RW_GL, "the listed groups fit");
+    const uint32_t qs = gs - 2u, qm = (1u << qs) - 1u;   // log2 of the lanes per group
+    if (R.np) {
+        for (uint32_t p = t; p < R.np; p += RW_NT) {
+            const uint32_t gp = (sh.pid[p] & ((1u << RW_PF_SHIFT) - 1u)) >> gs;
+            const uint32_t gq = p ? (sh.pid[p - 1] & ((1u << RW_PF_SHIFT) - 1u)) >> gs : 0xffffffffu;
+            if (gp != gq) gl[atomicAdd(&sh.n_gl, 1u)] = (uint16_t)gp;
+        }
+        rw_bar();
+        const uint32_t nit = rw_uni(sh.n_gl) << qs;
+        constexpr int NU = 4;
+        for (uint32_t i0 = 0; i0 < nit; i0 += NU * RW_NT) {
+            float4 v[NU];
+            uint32_t w[NU], idx0[NU];
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const uint32_t i = min(i0 + t + (uint32_t)u * RW_NT, nit - 1u);
+                idx0[u] = ((uint32_t)gl[i >> qs] << gs) + 4u * (i & qm);
+                v[u] = rw_fetch4(R, idx0[u], w[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                if (i0 + (uint32_t)u * RW_NT >= nit) break;
+                float x[4], y[4];
+                rw_load4(R, idx0[u], v[u], w[u], x, y, sh);
+                uint32_t mx = rw_gkey(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                                      __builtin_isunordered(x[0], x[1]) || __builtin_isunordered(x[2], x[3]));
+                uint32_t my = rw_gkey(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])),
+                                      __builtin_isunordered(y[0], y[1]) || __builtin_isunordered(y[2], y[3]));
+                mx = rw_lanes_umax(mx, qs);
+                my = rw_lanes_umax(my, qs);
+                // (the clamped lanes past the last item lie in its group: the same maxima)
+                if ((t & qm) == 0u && i0 + t + (uint32_t)u * RW_NT < nit) {
+                    gx[idx0[u] >> gs] = mx;
+                    gy[idx0[u] >> gs] = my;
+                }
+            }
+        }
+    }
+    rw_bar();
+    if (t == 0) sh.n_gl = 0;
+    RW_T(6);
+    // this thread's groups t, t + RW_NT, ...
+    uint32_t kx[RW_GPT], ky[RW_GPT], mo = 0, ms = 0, fin = 0;
+#pragma unroll
+    for (int e = 0; e < RW_GPT; e++) {
+        const uint32_t i = t + (uint32_t)e * RW_NT, ic = min(i, ng - 1u);
+        kx[e] = gx[ic];
+        ky[e] = gy[ic];
+        if (i >= ng) kx[e] = ky[e] = 0u;
+        mo = max(mo, kx[e]);
+        ms = max(ms, ky[e]);
+        fin += ky[e] > kinf ? 1u : 0u;
+    }
+    // t0: in every wave the c-th largest thread maximum, c = ceil(K / waves),
+    // is reached by c groups of that wave, so the smallest of the waves' is
+    // reached by K groups (k past a wave's width: the K-th largest group
+    // maximum itself)
+    const bool wide = Ks > 64u * RW_NW / 4u;
+    const uint32_t so = wave_sort_u32(mo), ss = wave_sort_u32(ms);
+    const int co = max((int)((Ko + RW_NW - 1) / RW_NW), 1), cs = wide ? 1 : max((int)((Ks + RW_NW - 1) / RW_NW), 1);
+    const uint32_t wo = (uint32_t)__builtin_amdgcn_readlane((int)so, 64 - co);
+    const uint32_t ws = (uint32_t)__builtin_amdgcn_readlane((int)ss, 64 - cs);
+    const uint32_t wf = rw_wave_sum(fin);
+    if (zs_lane() == 63) {
+        sh.ru[0][wid] = wo; sh.ru[1][wid] = ws; sh.ru[2][wid] = wf;
+        sh.ru[3][wid] = so; sh.ru[4][wid] = ss;
+    }
+    __syncthreads();
+    uint32_t to = 0xffffffffu, ts = 0xffffffffu, nfin = 0, kmo = 0, kms = 0;
+#pragma unroll
+    for (int w = 0; w < RW_NW; w++) {
+        to = min(to, sh.ru[0][w]); ts = min(ts, sh.ru[1][w]); nfin += sh.ru[2][w];
+        kmo = max(kmo, sh.ru[3][w]); kms = max(kms, sh.ru[4][w]);
+    }
+    to = rw_uni(to); ts = rw_uni(ts); nfin = rw_uni(nfin); kmo = rw_uni(kmo); kms = rw_uni(kms);
+    if (kmo == RW_KNAN || kms == RW_KNAN) return false;
+    // (too many of a wave's groups at -inf, as under a mask: exactly)
+    if (Ko && to <= kinf) to = rw_kth_key(2 * R.words, ng, Ko);
+    if (smode & 1u) {
+        if (wide && 4u * Ks > 3u * ng) return false;   // too few groups for a close threshold
+        if (wide || ts <= kinf) ts = rw_kth_key(2 * R.words + ng, ng, Ks);
+    } else if (smode == 2) {
+        // every y above -inf, when few enough groups hold one
+        G.s_over = nfin > ZS_SMALL_CAP;
+        ts = kinf + 1u;
+    }
+    const bool sl = (smode & 1u) || (smode == 2 && !G.s_over);   // a sampler list is kept
+    // (-inf is no member of either list here: the observers' -inf entries are
+    // added below, the sampler's survivors are above -inf)
+    to = Ko ? max(to, kinf + 1u) : 0xffffffffu;
+    ts = sl ? max(ts, kinf + 1u) : 0xffffffffu;
+    RW_T(15);
+    // the groups that reach a threshold
+    uint32_t rej = 0;
+#pragma unroll
+    for (int e = 0; e < RW_GPT; e++) {
+        const uint32_t f = (kx[e] >= to ? 1u : 0u) | (ky[e] >= ts ? 2u : 0u);
+        if (!(f & 2u)) rej = max(rej, ky[e]);
+        if (f) {
+            const uint32_t p = atomicAdd(&sh.n_gl, 1u);
+            if (p < RW_GL) gl[p] = (uint16_t)((t + (uint32_t)e * RW_NT) | (f << RW_GF));
+        }
+    }
+    __syncthreads();
+    const uint32_t n_gl = rw_uni(sh.n_gl);
+    if (n_gl > RW_GL) return false;
+    const uint32_t nit = n_gl << qs;
+    uint32_t* wk = reinterpret_cast<uint32_t*>(sh.u.b.s);
+    const uint32_t scap = smode == 3 ? (uint32_t)RW_WIDE : smode == 2 ? (uint32_t)ZS_SMALL_CAP : (uint32_t)RW_BUF;
+    constexpr int NU = 4;
+    for (uint32_t i0 = 0; i0 < nit; i0 += NU * RW_NT) {
+        float4 v[NU];
+        uint32_t w[NU], ge[NU];
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+            const uint32_t i = i0 + t + (uint32_t)u * RW_NT;
+            ge[u] = gl[min(i, nit - 1u) >> qs];
+            if (i >= nit) ge[u] &= (1u << RW_GF) - 1u;
+            v[u] = rw_fetch4(R, ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * (i & qm), w[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+            const uint32_t f = ge[u] >> RW_GF;
+            if (!f) continue;
+            const uint32_t idx0 = ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * ((i0 + t + (uint32_t)u * RW_NT) & qm);
+            float x[4], y[4];
+            rw_load4(R, idx0, v[u], w[u], x, y, sh);
+            // (thresholds are keys of group maxima: compared with -0 as +0, the
+            // sampler's entries themselves in total order as Rust sorts them)
+            uint32_t kxq[4], kyq[4], mo4 = 0, ms4 = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                kxq[q] = zs_total_key(x[q] + 0.0f);
+                kyq[q] = zs_total_key(y[q] + 0.0f);
+                mo4 |= kxq[q] >= to ? 1u << q : 0u;
+                const bool in = kyq[q] >= ts;
+                ms4 |= in ? 1u << q : 0u;
+                if (!in) rej = max(rej, kyq[q]);
+            }
+            if ((f & 1u) && mo4) {
+                uint32_t p = atomicAdd(&sh.sel_st[2], (uint32_t)__popc(mo4));
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (!((mo4 >> q) & 1u)) continue;
+                    if (p < RW_GOBS) sh.u.b.o[p] = ((unsigned long long)(~kxq[q]) << 32) | (idx0 + q);
+                    p++;
+                }
+            }
+            if ((f & 2u) && ms4) {
+                uint32_t p = atomicAdd(&sh.sel_st[3], (uint32_t)__popc(ms4));
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (!((ms4 >> q) & 1u)) continue;
+                    if (p < scap) {
+                        if (smode == 3) wk[p] = kyq[q];
+                        else sh.u.b.s[p] = ((unsigned long long)(~zs_total_key(y[q])) << 32) | (idx0 + q);
+                    }
+                    p++;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t n_o = rw_uni(sh.sel_st[2]);
+    const uint32_t n_s = rw_uni(sh.sel_st[3]);
+    __syncthreads();   // (the count is read before the ids at -inf are added to it)
+    if (n_o > RW_GOBS || ((smode & 1u) && n_s > scap)) return false;
+    if (n_o < Ko) {
+        // fewer than Ko ids above -inf: the smallest ids at -inf follow (at
+        // most Ko of the first 64 ids are above it)
+        static_assert(2 * ZS_OBS_CAND <= 64, "the first 64 ids hold them");
+        if (t < 64) {
+            uint32_t w;
+            const uint32_t idx0 = t & ~3u;
+            const float4 v = rw_fetch4(R, idx0, w);
+            float x[4], y[4];
+            rw_load4(R, idx0, v, w, x, y, sh);
+            const float xi = (t & 3u) == 0 ? x[0] : (t & 3u) == 1 ? x[1] : (t & 3u) == 2 ? x[2] : x[3];
+            if (t < R.V && xi == -INFINITY) sh.u.b.o[atomicAdd(&sh.sel_st[2], 1u)] = ((unsigned long long)(~kinf) << 32) | t;
+        }
+        __syncthreads();
+        n_o = rw_uni(sh.sel_st[2]);
+    }
+    if (greedy) {
+        // the last id whose y equals the maximum: in the last group at it
+        uint32_t lg = 0;
+#pragma unroll
+        for (int e = 0; e < RW_GPT; e++)
+            if (ky[e] == kms && t + (uint32_t)e * RW_NT < ng) lg = t + (uint32_t)e * RW_NT + 1u;
+        lg = rw_wave_umax(lg);
+        if (zs_lane() == 0) sh.ru[5][wid] = lg;
+        __syncthreads();
+        lg = 0;
+#pragma unroll
+        for (int w = 0; w < RW_NW; w++) lg = max(lg, sh.ru[5][w]);
+        const uint32_t idx0 = ((lg - 1u) << gs) + 4u * t;
+        if (4u * t < 1u << gs) {
+            uint32_t w;
+            const float4 v = rw_fetch4(R, idx0, w);
+            float x[4], y[4];
+            rw_load4(R, idx0, v, w, x, y, sh);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (idx0 + q < R.V && zs_total_key(y[q] + 0.0f) == kms)
+                    G.gbest = ((unsigned long long)kms << 32) | (idx0 + q + 1);
+        }
+    }
+    G.omax = zs_key_to_float(kmo);
+    G.ymax = zs_key_to_float(kms);
+    G.rejf = rej > kinf ? zs_key_to_float(rej) : -INFINITY;
+    G.n_o = n_o;
+    G.n_s = n_s;
+    if (smode == 2 && n_s > ZS_SMALL_CAP) G.s_over = true;
+    __syncthreads();
+    return true;
+}
+
+// ---------------------------------------------------------------------------
+// zs_k_scan: the group maxima of every row, over the whole GPU. One read of
+// the logits, 4 16-byte loads in flight per thread; a masked row's loads are
+// skipped where 4 ids in a row are disallowed. HBM-bound: 32.8 MB (64 x 128256)
+// in 7.2 us. (A NaN or few survivors are seen in the maxima: no other statistic
+// is needed.)
+// ---------------------------------------------------------------------------
+#define SC_NT 256
+#define SC_IDS (16 * SC_NT)   // ids per workgroup
+template <int GS>
+__global__ __launch_bounds__(SC_NT) void zs_k_scan(zs_sargs a) {
+    const zs_batch& b = a.b;
+    const uint32_t r = blockIdx.y, V = b.V, lane = (uint32_t)zs_lane();
+    const float* row = b.d_logits + (size_t)r * b.ld;
+    const uint32_t* allow = ((b.d_params[r].flags & ZS_ROW_MASKED) && b.d_allow_bits)
+                                ? b.d_allow_bits + (size_t)r * b.allow_words : nullptr;
+    typedef float sc_f4 __attribute__((ext_vector_type(4)));
+    const uint32_t base = blockIdx.x * SC_IDS + 4u * threadIdx.x;
+    sc_f4 v[4];
+    uint32_t w[4];
+    if (allow) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t id = base + (uint32_t)u * (4u * SC_NT);
+            w[u] = id < V ? allow[id >> 5] >> (id & 31u) & 15u : 0u;
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; u++) w[u] = base + (uint32_t)u * (4u * SC_NT) < V ? 15u : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        v[u] = sc_f4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        if (w[u]) v[u] = *reinterpret_cast<const sc_f4*>(row + base + (uint32_t)u * (4u * SC_NT));
+    }
+    uint32_t k[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t id = base + (uint32_t)u * (4u * SC_NT);
+        if (id + 4u > V) w[u] &= id < V ? (1u << (V - id)) - 1u : 0u;
+        const float x0 = (w[u] & 1u) ? v[u].x : -INFINITY, x1 = (w[u] & 2u) ? v[u].y : -INFINITY;
+        const float x2 = (w[u] & 4u) ? v[u].z : -INFINITY, x3 = (w[u] & 8u) ? v[u].w : -INFINITY;
+        const bool nan = __builtin_isunordered(x0, x1) || __builtin_isunordered(x2, x3);
+        k[u] = rw_gkey(fmaxf(fmaxf(x0, x1), fmaxf(x2, x3)), nan);
+        k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0xB1, 0xf, 0xf, false));
+        k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x4E, 0xf, 0xf, false));
+        if (GS >= 5) k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x141, 0xf, 0xf, false));
+        if (GS >= 6) k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x140, 0xf, 0xf, false));
+    }
+    // lane q of a quad stores load q's group (one store for all four)
+    constexpr uint32_t LG = 1u << (GS - 2);   // lanes per group
+    const uint32_t q = lane & 3u;
+    const uint32_t kq = q == 0 ? k[0] : q == 1 ? k[1] : q == 2 ? k[2] : k[3];
+    const uint32_t g = (blockIdx.x * SC_IDS + q * (4u * SC_NT) + 4u * threadIdx.x) >> GS;
+    if ((lane & (LG - 1u)) < 4u && g < (V + (1u << GS) - 1u) >> GS) a.gmax[(size_t)r * a.gstride + g] = kq;
+}
+
+// Group size of the scan: the row kernel holds the maxima of at most RW_GPT
+// groups per thread; smaller groups mean fewer ids read twice. 0: rows below
+// two of the streaming loop's tiles gain nothing from a second launch.
+uint32_t zs_scan_gshift(uint32_t V) {
+    if (V < 2 * RW_G) return 0;
+    uint32_t gs = 4;
+    while (((V + (1u << gs) - 1u) >> gs) > RW_GPT * RW_NT) gs++;
+    return gs;
+}
+
 // ---------------------------------------------------------------------------
 // zs_k_row
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     const zs_batch& b = a.b;
-    // with a.row_split, workgroups B .. 2B - 1 take the second half of their
-    // row's stream (below)
-    const uint32_t half = (a.row_split && blockIdx.x >= b.B) ? 1u : 0u;
-    const uint32_t r = rw_block_row(b, blockIdx.x - half * b.B);
+    const uint32_t r = rw_block_row(b, blockIdx.x, a.ncu);
     const uint32_t t = threadIdx.x;
     const uint32_t V = b.V;
     rw_shared& sh = rw_sh;
@@ -777,37 +1397,8 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     const bool tinf = T == INFINITY;   // y / inf is NaN for y = +-inf: checked per element
     const uint32_t* allow = ((P.flags & ZS_ROW_MASKED) && b.d_allow_bits) ? b.d_allow_bits + (size_t)r * b.allow_words
                                                                           : nullptr;
-    // A row that streams the whole row (not a masked row taking its lists from
-    // at most RW_BUF gathered ids) may split the stream over two workgroups
-    // when the batch leaves CUs free (a.row_split), unless its patch list may
-    // pass the LDS head (both workgroups build it). Both halves decide alike.
-    const uint32_t ngt = (V + RW_G - 1) / RW_G;
-    bool split = false;
-    if (a.row_split && ngt >= 8) {
-        const uint32_t nb = b.d_ban_off ? b.d_ban_off[r + 1] - b.d_ban_off[r] : 0u;
-        const uint32_t nbi = b.d_bias_off ? b.d_bias_off[r + 1] - b.d_bias_off[r] : 0u;
-        const uint32_t nc = (b.d_cnt_off && zs_penalty_active(P)) ? b.d_cnt_off[r + 1] - b.d_cnt_off[r] : 0u;
-        if (nb + nbi + nc <= ZS_PATCH_LDS) {
-            if (!allow || greedy || tinf) {
-                split = true;
-            } else {
-                const uint32_t words = (V + 31) / 32;
-                uint32_t c = 0;
-                for (uint32_t w = t; w < words; w += RW_NT) {
-                    uint32_t aw = allow[w];
-                    if (w == words - 1 && (V & 31)) aw &= (1u << (V & 31)) - 1u;
-                    c += (uint32_t)__popc(aw);
-                }
-                split = rw_uni(block_sum_u<RW_NT>(c, sh.ru[4])) > RW_BUF;
-            }
-        }
-    }
-    if (half && !split) return;
-
-    // ---------------- P0: patches (the second half builds its own LDS copy
-    // only: the first writes the row's list out)
-    uint32_t has_y = 0;
-    const int np = rw_patches(a, r, P, has_y, sh, half == 0);
+    // ---------------- P0: patches
+    const int np = rw_patches(a, r, P, sh);
     RW_T(0);
     rw_row R;
     R.gfl = a.p_flags + (size_t)r * a.pstride;
@@ -821,12 +1412,9 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     R.allow_or_row = R.allow ? R.allow : reinterpret_cast<const uint32_t*>(R.row);
     R.wmax = R.allow ? R.words - 1 : R.ldm4;
     R.amask = R.allow ? 0u : 15u;
-    // the streamed range: the whole row, or this workgroup's half
-    const uint32_t gmid = ngt / 2;
-    const uint32_t gbeg = (split && half) ? gmid : 0u;
-    R.gend = (split && !half) ? gmid : ngt;
-    R.vend = R.gend == ngt ? V : R.gend * RW_G;
-    R.glast = (R.vend - 1) / RW_G;
+    R.gend = (V + RW_G - 1) / RW_G;
+    R.vend = V;
+    R.glast = (V - 1) / RW_G;
 
     // ---------------- P1: statistics and candidate lists
     // The sampler's z = y / T (sampler.rs:47-51) is not formed per element
@@ -835,9 +1423,13 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     // checked when the threshold is set).
     const bool has_topk = P.top_k > 0 && P.top_k < V;
     // sampler list: 1 = top-k by y (k <= ZS_KS), 2 = every y > -inf (the
-    // small-survivor check when no top-k applies), 0 = none
-    const uint32_t smode = greedy ? 0u : (has_topk ? (P.top_k <= ZS_KS ? 1u : 0u) : 2u);
-    const uint32_t Ks = smode == 1 ? P.top_k : 0u;
+    // small-survivor check when no top-k applies), 0 = none; from the group
+    // maxima also larger k: 1 while the survivors fit the small path, 3 (the
+    // keys only, for the threshold) up to RW_KWIDE
+    const bool has_groups = a.gshift && !tinf && R.np <= ZS_PATCH_LDS;
+    const uint32_t kmax1 = has_groups ? (uint32_t)ZS_SMALL_CAP - 1u : (uint32_t)ZS_KS;
+    uint32_t smode = greedy ? 0u : (!has_topk ? 2u : P.top_k <= kmax1 ? 1u : (has_groups && P.top_k <= RW_KWIDE) ? 3u : 0u);
+    uint32_t Ks = (smode & 1u) ? P.top_k : 0u;
     const uint32_t Ko = want_obs ? (ZS_OBS_CAND < V ? ZS_OBS_CAND : V) : 0u;
     rw_list LO, LS;
     LO.buf = sh.u.b.o; LO.cnt = cnt_o; LO.thr = &thr_o; LO.flag = &flag_o;
@@ -886,7 +1478,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     // values stay live across the stream below)
     bool gath = false;
     if (t == 0) { sh.g_n = 0; sh.g_done = 0; }
-    if (R.allow && !greedy && !tinf && !split) {
+    if (R.allow && !greedy && !tinf) {
         const float* gcx = rw_scratch(a, r);
         const uint32_t gn = rw_gather_allowed(R.row, R.allow, V, R.np, rw_scratch(a, r), R.gfl, R.gy);
         if (t == 0) { sh.g_n = gn; sh.g_done = 1; }
@@ -895,11 +1487,23 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
             for (uint32_t i = t; i < gn; i += RW_NT) nf += gcx[i] > -INFINITY ? 1u : 0u;
             nf = block_sum_u<RW_NT>(nf, sh.ru[4]);
             gath = rw_uni(nf) >= Ko;
+            if (gath && smode == 3) { smode = 0; Ks = 0; }
         }
     }
     RW_T(1);
-    uint32_t g = gbeg;
-    const uint32_t ng = gath ? 0u : R.gend;
+    // ---- the lists from the group maxima of zs_k_scan
+    bool fast = false;
+    if (!gath && a.gshift && !tinf && R.np <= ZS_PATCH_LDS) {
+        rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, false};
+        fast = rw_groups(a, r, R, greedy, smode, Ks, Ko, G);
+        if (fast) {
+            omax = G.omax; ymax = G.ymax; rejf = G.rejf; gbest = G.gbest;
+            n_o = G.n_o; n_s = G.n_s; s_over = G.s_over;
+        }
+    }
+    if (!gath && !fast && has_topk && P.top_k > ZS_KS) { smode = 0; Ks = 0; }
+    uint32_t g = 0;
+    const uint32_t ng = (gath || fast) ? 0u : R.gend;
     const uint32_t Vend = R.vend;
     // the admission thresholds in scalar registers: they change only where
     // the lists are set up (first tile) and compacted (outside the stream)
@@ -1237,86 +1841,24 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
         }
         __syncthreads();
     }
-    if (split) {
-        // This half's lists cut to what the row can need from it: the first
-        // Ko observers, the sampler's first Ks + 1 (the next one counts as
-        // turned away), or its small-survivor list. They go to the half's
-        // slot with its statistics; the half that finishes second merges the
-        // other's slot into its own and goes on alone (no waiting: the first
-        // to finish leaves).
-        uint32_t no = 0, ns = 0;
-        if (Ko) no = min(rw_select(0, min(n_o, (uint32_t)RW_BUF), Ko, 0xffffffffu), Ko);
-        if (smode == 1) {
-            const uint32_t c = rw_select(1, min(n_s, (uint32_t)RW_BUF), Ks + 2, 0xffffffffu);
-            if (c > Ks + 1) rejf = fmaxf(rejf, zs_key_to_float(~(uint32_t)(sh.u.b.s[Ks + 1] >> 32)));
-            ns = min(c, Ks + 1);
-        } else if (smode == 2 && !s_over) {
-            ns = n_s;   // at most ZS_SMALL_CAP
-        }
-        RW_T(15);
-        unsigned long long* mine = a.rw_part + ((size_t)r * 2 + half) * RW_PART;
-        if (t == 0) {
-            mine[0] = (unsigned long long)__float_as_uint(omax) | ((unsigned long long)__float_as_uint(ymax) << 32);
-            mine[1] = (unsigned long long)fl | ((unsigned long long)(uint32_t)last_nan << 32);
-            mine[2] = (unsigned long long)__float_as_uint(rejf) | ((unsigned long long)(s_over ? 1u : 0u) << 32);
-            mine[3] = gbest;
-            mine[4] = (unsigned long long)no | ((unsigned long long)ns << 32);
-        }
-        for (uint32_t i = t; i < no; i += RW_NT) mine[RW_PART_O + i] = sh.u.b.o[i];
-        for (uint32_t i = t; i < ns; i += RW_NT) mine[RW_PART_S + i] = sh.u.b.s[i];
-        // (the barrier completes every wave's stores; one device-scope fence
-        // then publishes them before the count, and one makes the other
-        // half's visible after it)
-        __syncthreads();
-        if (t == 0) {
-            __threadfence();
-            const uint32_t m = atomicAdd(&a.rw_ctr[r], 1u);
-            if (m) {
-                a.rw_ctr[r] = 0u;   // for the next call
-                __threadfence();
-            }
-            sh.merge = m;
-        }
-        __syncthreads();
-        RW_T(6);
-        if (rw_uni(sh.merge) == 0u) return;   // the other half merges
-        const unsigned long long* oth = a.rw_part + ((size_t)r * 2 + (1u - half)) * RW_PART;
-        const unsigned long long h0 = oth[0], h1 = oth[1], h2 = oth[2], h3 = oth[3], h4 = oth[4];
-        omax = fmaxf(omax, __uint_as_float((uint32_t)h0));
-        ymax = fmaxf(ymax, __uint_as_float((uint32_t)(h0 >> 32)));
-        fl |= (uint32_t)h1;
-        last_nan = max(last_nan, (int)(uint32_t)(h1 >> 32));
-        rejf = fmaxf(rejf, __uint_as_float((uint32_t)h2));
-        const bool o_over = (h2 >> 32) != 0ull;
-        gbest = h3 > gbest ? h3 : gbest;
-        const uint32_t ono = (uint32_t)h4, ons = (uint32_t)(h4 >> 32);
-        for (uint32_t i = t; i < ono; i += RW_NT) sh.u.b.o[no + i] = oth[RW_PART_O + i];
-        n_o = no + ono;
-        if (smode == 1) {
-            for (uint32_t i = t; i < ons; i += RW_NT) sh.u.b.s[ns + i] = oth[RW_PART_S + i];
-            n_s = ns + ons;
-        } else if (smode == 2) {
-            s_over = s_over || o_over || ns + ons > ZS_SMALL_CAP;
-            if (!s_over)
-                for (uint32_t i = t; i < ons; i += RW_NT) sh.u.b.s[ns + i] = oth[RW_PART_S + i];
-            n_s = ns + ons;
-        }
-        __syncthreads();
-        // later streams (the greedy fold after a NaN) cover the whole row
-        R.gend = ngt;
-        R.vend = V;
-        R.glast = (V - 1) / RW_G;
-    }
     const float M = rw_unif(omax);
     const float zmax = rw_unif(zs_temper(ymax, T));   // max z = temper(max y): monotone
     const bool special = (fl & ZS_CF_OBS_NAN) || M == INFINITY || M == -INFINITY;
     uint32_t obs_need = 0;
     if (!special && want_obs) obs_need |= ZS_OBS_S;
     if (!special && want_unc) obs_need |= ZS_OBS_H;
+    // short lists are sorted whole, the observers' by wave 0 and the sampler's
+    // by wave 1 at the same time
+    const bool short_o = n_o <= RW_SEL_CAP, short_s = smode == 1 && n_s <= RW_SEL_CAP;
+    if (short_o || short_s) {
+        if (short_o && Ko && t < 64) rw_wave_sort(sh.u.b.o, n_o);
+        if (short_s && t >= 64 && t < 128) rw_wave_sort(sh.u.b.s, n_s);
+        __syncthreads();
+    }
     // observer candidates: the first Ko entries of the sorted list
     uint32_t n_cand = 0;
     if (Ko) {
-        const uint32_t n = rw_select(0, min(n_o, (uint32_t)RW_BUF), Ko, 0xffffffffu);
+        const uint32_t n = short_o ? n_o : rw_select(0, min(n_o, (uint32_t)RW_BUF), Ko, 0xffffffffu);
         n_cand = min(n, Ko);
         if (t < n_cand) {
             sh.cand_id[t] = (uint32_t)sh.u.b.o[t];
@@ -1369,7 +1911,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
         bool small = false;
         uint32_t nsv = 0;
         if (smode == 1) {
-            const uint32_t n = rw_select(1, min(n_s, (uint32_t)RW_BUF), Ks + 1, 0xffffffffu);
+            const uint32_t n = short_s ? n_s : rw_select(1, min(n_s, (uint32_t)RW_BUF), Ks + 1, 0xffffffffu);
             // the k-th largest z is temper(the k-th largest y); a list of
             // fewer than k holds every y above -inf, so the k-th is -inf
             const float yk = n >= Ks ? zs_key_to_float(~(uint32_t)(sh.u.b.s[Ks - 1] >> 32)) : -INFINITY;
@@ -1431,15 +1973,22 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
             __syncthreads();
             nsv = sh.n_surv;
             small = true;
+        } else if (smode == 3) {
+            // the k-th largest key among the listed ones (fewer than k: -inf)
+            const float yk = n_s >= Ks ? zs_key_to_float(rw_kth_key(0xffffffffu, n_s, Ks)) : -INFINITY;
+            thr = zs_temper(yk, T);
+            thr_key = zs_total_key(thr);
+            has_thr = 1;
         } else if (has_topk) {
-            has_thr = 2;   // top_k > ZS_KS: zs_k_big selects the threshold
+            has_thr = 2;   // zs_k_big selects the threshold
         }
         if (small) {
             __syncthreads();
-            if (t < 64) rw_small(b.d_seed[r], b.d_counter[r], V, P, nsv, zmax, sh);
+            rw_small(b.d_seed[r], b.d_counter[r], V, P, rw_uni(nsv), zmax, sh);
             __syncthreads();
             token = sh.tok;
-            status |= ZS_ST_SMALL;
+            // (documented for the sets of at most ZS_KS, or no top-k)
+            if (smode == 2 || Ks <= ZS_KS) status |= ZS_ST_SMALL;
         } else {
             mode = ZS_MODE_BIG;
         }
@@ -1504,7 +2053,16 @@ extern "C" int zs_dbg_row_stats(unsigned long long* out) {
 #endif
 
 extern "C" int zs_row_launch(const zs_sargs& a, hipStream_t stream) {
-    const size_t dyn = 4 * ((a.b.V + 31) / 32) * sizeof(uint32_t);
-    hipLaunchKernelGGL(zs_k_row, dim3(a.row_split ? 2 * a.b.B : a.b.B), dim3(RW_NT), dyn, stream, a);
+    const uint32_t words = (a.b.V + 31) / 32;
+    size_t tail = 2 * words;   // rw_patches' bias bitmaps, then the group maxima
+    if (a.gshift) {
+        const uint32_t ng = (a.b.V + (1u << a.gshift) - 1u) >> a.gshift;
+        const dim3 grid((a.b.V + SC_IDS - 1) / SC_IDS, a.b.B);
+        if (a.gshift == 4) hipLaunchKernelGGL(zs_k_scan<4>, grid, dim3(SC_NT), 0, stream, a);
+        else if (a.gshift == 5) hipLaunchKernelGGL(zs_k_scan<5>, grid, dim3(SC_NT), 0, stream, a);
+        else hipLaunchKernelGGL(zs_k_scan<6>, grid, dim3(SC_NT), 0, stream, a);
+        tail = std::max(tail, (size_t)2 * ng);
+    }
+    hipLaunchKernelGGL(zs_k_row, dim3(a.b.B), dim3(RW_NT), (2 * words + tail) * sizeof(uint32_t), stream, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

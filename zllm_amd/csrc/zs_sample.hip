@@ -7,6 +7,7 @@
 //   logprobs / token_uncertainty on x~    logprobs.rs:34-54, hallucination.rs:129-154
 //
 // Kernels (one launch each, in stream order):
+//   zs_k_scan     (zs_row.hip) the maxima of groups of ids, over the whole GPU.
 //   zs_k_row      (zs_row.hip) one workgroup per row: patch list, candidate
 //                 lists, the sampler's decisions (greedy, non-finite, top-k and
 //                 small survivor sets sampled on chip); the other rows are
@@ -2013,11 +2014,10 @@ extern "C" int zs_sample_launch(zs_ctx* ctx, const zs_batch* bt, hipStream_t str
     a.tp_pre = ctx->tp_pre;
     a.kcnt = ctx->kcnt;
     a.tp_task = ctx->tp_task;
-    a.rw_part = ctx->rw_part;
-    a.rw_ctr = ctx->rw_ctr;
-    // rows split their stream over two workgroups when the batch leaves the
-    // second workgroups CUs of their own
-    a.row_split = 2 * bt->B <= ctx->num_cus ? 1u : 0u;
+    a.ncu = ctx->num_cus;
+    a.gmax = ctx->gmax;
+    a.gstride = ctx->max_vocab / ZS_SCAN_MIN_GROUP + 1;
+    a.gshift = zs_scan_gshift(bt->V);
     a.s_rec = ctx->s_rec;
     a.s_xrec = ctx->s_rec + (size_t)ctx->max_rows * ZS_NSUM * ctx->max_subs;
     a.s_apx = ctx->s_apx;

@@ -34,9 +34,10 @@ struct zs_sargs {
     float* gath;
     float* s_hterm;
     uint32_t pstride;   // entries per row of the merged patch list (p_id, p_flags, p_y): max_vocab
-    uint32_t row_split; // zs_k_row: 2B workgroups, rows may split their stream in two halves
-    unsigned long long* rw_part;
-    uint32_t* rw_ctr;
+    uint32_t gshift;    // zs_k_scan: log2 of the ids per group (0: no scan)
+    uint32_t ncu;       // CUs of the device
+    uint32_t gstride;   // groups per row of gmax
+    uint32_t* gmax;     // [rows][gstride] keys of the group maxima
 };
 
 #define ZS_ST_FALLBACK 0x200u
@@ -44,6 +45,8 @@ struct zs_sargs {
 // zs_row.hip: the per-row front of the step (patches, row statistics,
 // candidates, greedy and small rows)
 extern "C" int zs_row_launch(const zs_sargs& a, hipStream_t stream);
+// log2 of the ids per group of zs_k_scan for rows of V ids (0: no scan)
+uint32_t zs_scan_gshift(uint32_t V);
 // zs_sums.hip: the row sums (the big rows' sampler S; S_obs, then the
 // entropy) spread over the GPU (one kernel per call, `which` 0..7)
 extern "C" int zs_sums_launch(const zs_sargs& a, uint32_t which, hipStream_t stream);
@@ -121,6 +124,21 @@ __device__ __forceinline__ void wave_stage_f(float* buf, const float (&v)[E], ui
 __device__ __forceinline__ uint32_t serial_scan_f(const float* buf, uint32_t n, float s0, float thresh, float* s) {
     float acc = s0;
     uint32_t i = 0;
+    // 32 terms per batch of reads, their latency off the chain of additions
+    // (the terms are probabilities, never negative: a running sum below
+    // thresh after the batch was below it inside); the batch that reaches
+    // thresh is added again below to find the element. 512 terms: 8.6 us one
+    // test and one read of 4 at a time, 3 us so.
+    for (; i + 32 <= n; i += 32) {
+        float4 q8[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) q8[u] = *reinterpret_cast<const float4*>(buf + i + 4 * u);
+        float c = acc;
+#pragma unroll
+        for (int u = 0; u < 8; u++) c = (((c + q8[u].x) + q8[u].y) + q8[u].z) + q8[u].w;
+        if (c >= thresh) break;
+        acc = c;
+    }
     for (; i + 4 <= n; i += 4) {
         const float4 q = *reinterpret_cast<const float4*>(buf + i);
         acc = acc + q.x;
