@@ -233,7 +233,11 @@ __device__ __forceinline__ float sm_walk(const float (&v)[SW_TPT], float s, floa
             for (int q = SW_TPT - 1; q >= 0; q--)
                 if (SW_TPT * t + (uint32_t)q >= pos && v[q] != 0.0f) my = SW_TPT * t + (uint32_t)q;
             const unsigned long long m = __ballot(my != 0xffffffffu);
-            if (lane == 0) sh.first[wid] = m ? (uint32_t)__builtin_amdgcn_readlane((int)my, __ffsll((long long)m) - 1) : 0xffffffffu;
+            // (the lane read stays outside the lane-0 branch: inside it the
+            // compiler may form `my` for lane 0 alone, and the lane that is
+            // read would hold an old value)
+            const uint32_t wf = m ? (uint32_t)__builtin_amdgcn_readlane((int)my, __ffsll((long long)m) - 1) : 0xffffffffu;
+            if (lane == 0) sh.first[wid] = wf;
             sm_bar();
             uint32_t first = 0xffffffffu;
 #pragma unroll
