@@ -105,3 +105,25 @@ def test_zeros_of_both_signs(V):
     print(f"[case] zeros of both signs V={V}", flush=True)
     errs = compare(x, params, run_gpu(x, params))
     assert not errs, "\n".join(errs)
+
+
+@pytest.mark.parametrize("top_p", [1.0, 0.9])
+def test_min_p_kept_lists(top_p):
+    """The kept mass of min-p rows from per-wave lists (zs_k_big): 1 kept
+    value, a stretch of the row (1280 ids) that keeps exactly as many as its
+    list holds (512) and one more, kept values over all stretches, and a row
+    that keeps everything; min_p above 1 keeps nothing."""
+    V = 20000
+    rng = np.random.default_rng(5)
+    x = rng.normal(-12, 1, (7, V)).astype(np.float32)
+    x[0, 17] = 9.0
+    for i, n in ((1, 512), (2, 513)):
+        x[i, 1280 + rng.choice(1280, n, replace=False)] = rng.normal(8, 0.3, n).astype(np.float32)
+    x[3, rng.choice(V, 700, replace=False)] = rng.normal(8, 0.5, 700).astype(np.float32)
+    x[4] = rng.normal(0, 0.1, V).astype(np.float32)
+    x[5, :700] = 3.0
+    params = [dict(temperature=1.1, top_k=0, top_p=top_p, min_p=0.05, seed=i, top_logprobs=3) for i in range(7)]
+    params[6]["min_p"] = 1.5
+    print(f"[case] min-p kept lists top_p={top_p}", flush=True)
+    errs = compare(x, params, run_gpu(x, params))
+    assert not errs, "\n".join(errs)

@@ -537,8 +537,8 @@ __global__ __launch_bounds__(PV_NT) void zs_k_pv(zs_sargs a) {
 //                 widened by a bound on the f32 rounding error, crosses a
 //                 power of two or top_p; the first bucket);
 //   zs_k_tp_inc   (all CUs): per-bucket increment totals on the predicted grid
-//                 and the exact-half (tie) flags; every positive p is gathered
-//                 into the bucket layout; buckets with ties become candidates;
+//                 and the exact-half (tie) flags; every p of a bucket that the
+//                 walk can reach is gathered into the bucket layout; buckets with ties become candidates;
 //   zs_k_tp_sort  (one workgroup per candidate): sorts the bucket in
 //                 descending order and stores the prefix of its increment
 //                 maps on the predicted grid (a parity pair, so ties are
@@ -556,6 +556,7 @@ __global__ __launch_bounds__(PV_NT) void zs_k_pv(zs_sargs a) {
 #define TP_M_TIE1 0x400u
 #define TP_M_SORTED 0x800u
 #define TP_ROW_FAST 1u
+#define TP_ROW_LIM 8        // cl[0] >> TP_ROW_LIM: the first bucket the walk cannot reach
 #define TP_SORT_MAX 4096
 #define TP_SORT_NT 1024
 #define TP_SERIAL_N 512
@@ -587,6 +588,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_plan(zs_sargs a) {
     const double mex = block_excl_scan_d<ZS_BIG_NT>(m[0] + m[1], sd, &mtot);
     const double top_p = (double)P.top_p;
     uint32_t cand[2], meta[2];
+    int rlim = ZS_TP_NB;
 #pragma unroll
     for (int k2 = 0; k2 < 2; k2++) {
         const uint32_t start = cex + (k2 ? c[0] : 0u);
@@ -601,6 +603,10 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_plan(zs_sargs a) {
         const int e0 = zs_grid_exp((float)lo), e1 = zs_grid_exp((float)fmin(hi, top_p));
         const bool cd = c[k2] != 0u && lo < top_p && (P0 == 0.0 || e0 != e1 || hi >= top_p);
         cand[k2] = cd ? 1u : 0u;
+        // (buckets the sum has reached top_p before: their increments and
+        // values are left out by zs_k_tp_inc; a walk that gets there after
+        // all falls back)
+        if (c[k2] && lo >= top_p) rlim = min(rlim, 2 * t + k2);
         meta[k2] = (uint32_t)(cd ? e0 : e1) | (cd ? TP_M_CAND : 0u);
         zs_tp_bucket& B = bk[2 * t + k2];
         B.start = start;
@@ -608,6 +614,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_plan(zs_sargs a) {
         B.meta = meta[k2];
         B.tot = 0ull;
     }
+    rlim = block_min_i<ZS_BIG_NT>(rlim, reinterpret_cast<int*>(su));
     uint32_t ntot;
     const uint32_t pos = block_excl_scan_u<ZS_BIG_NT>(cand[0] + cand[1], su, &ntot);
     if (ntot > ZS_TP_CAND) {
@@ -619,7 +626,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_plan(zs_sargs a) {
     for (int k2 = 0; k2 < 2; k2++)
         if (cand[k2]) cl[2 + q++] = 2 * t + k2;
     if (t == 0) {
-        cl[0] = TP_ROW_FAST;
+        cl[0] = TP_ROW_FAST | ((uint32_t)rlim << TP_ROW_LIM);
         cl[1] = ntot;
         const uint32_t base = ntot ? atomicAdd(&a.tp_task[0], ntot) : 0u;
         for (uint32_t j = 0; j < ntot; j++) a.tp_task[1 + base + j] = (r << 8) | j;
@@ -630,6 +637,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_inc(zs_sargs a) {
     const uint32_t g = blockIdx.x, r = blockIdx.y;
     uint32_t* cl = a.tp_cl + (size_t)r * ZS_TP_CL;
     if (!(cl[0] & TP_ROW_FAST)) return;
+    const uint32_t rlim = cl[0] >> TP_ROW_LIM;
     const uint32_t V = a.b.V;
     const int t = threadIdx.x;
     __shared__ uint32_t lc[ZS_TP_NB];
@@ -646,7 +654,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_inc(zs_sargs a) {
     for (int q = 0; q < 4; q++) {
         rk[q] = bk_rank<0>(pb[q]);
         off[q] = 0u;
-        if (zs_u2f(pb[q]) > 0.0f) {
+        if (rk[q] < rlim && zs_u2f(pb[q]) > 0.0f) {
             const int eg = (int)(bk[rk[q]].meta & TP_M_EG);
             const seq_pair pr = seq_pair_of(zs_u2f(pb[q]), eg);
             off[q] = atomicAdd(&lc[rk[q]], 1u);
@@ -674,7 +682,7 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_inc(zs_sargs a) {
     uint32_t* gv = a.pairs + (size_t)r * a.max_vocab * 2;
 #pragma unroll
     for (int q = 0; q < 4; q++)
-        if (zs_u2f(pb[q]) > 0.0f) gv[lc[rk[q]] + off[q]] = pb[q];
+        if (rk[q] < rlim && zs_u2f(pb[q]) > 0.0f) gv[lc[rk[q]] + off[q]] = pb[q];
 }
 
 // Composition of increment maps over a workgroup, in thread order: exclusive
@@ -881,6 +889,7 @@ extern "C" int zs_dbg_big_stats(unsigned long long* out) {
 
 #define TP_CH 1024   // values per LDS chunk of tp_walk's one-by-one additions
 __device__ __forceinline__ int tp_walk(const zs_sargs& a, uint32_t r, float top_p, walk_out* wo, float* lbuf) {
+    const uint32_t rlim = a.tp_cl[(size_t)r * ZS_TP_CL] >> TP_ROW_LIM;
     const uint32_t lane = (uint32_t)zs_lane();
     const zs_tp_bucket* bk = a.tp_bk + (size_t)r * ZS_TP_NB;
     const uint32_t* gv = a.pairs + (size_t)r * a.max_vocab * 2;
@@ -917,7 +926,7 @@ __device__ __forceinline__ int tp_walk(const zs_sargs& a, uint32_t r, float top_
     grp_ld cur = load(0), nxt = load(64);
     while (b0 < ZS_TP_NB) {
         const uint32_t cnt = lane >= l0 ? cur.cnt : 0u, meta = cur.meta;
-        const bool special = cnt && ((int)(meta & TP_M_EG) != eg || (meta & TP_M_TIE0));
+        const bool special = cnt && ((int)(meta & TP_M_EG) != eg || (meta & TP_M_TIE0) || b0 + lane >= rlim);
         // totals on the grid, saturated: a group is only added whole while the
         // sum stays below the binade end
         const uint32_t inc = (cnt && !special) ? (uint32_t)min(cur.tot, (unsigned long long)ZS_INC_CAP) : 0u;
@@ -1065,6 +1074,65 @@ __device__ __forceinline__ int tp_walk(const zs_sargs& a, uint32_t r, float top_
 }
 
 
+// The min-p kept mass (sampler.rs:80: the sum of the p >= cut in index order,
+// from +0) of a row that keeps few values: every wave lists the kept values of
+// its stretch of the row in LDS (in index order), then one wave adds the lists
+// up one value at a time (the zeros between them add nothing). One pass over
+// p by one workgroup, 12 us on 100003 ids where the sum in groups of 4096 with
+// a workgroup scan each took 95. False (uniform) when a wave keeps more than
+// its list holds: the caller sums the whole row.
+#define BK_KEEP (ZS_SORT_CAP / (ZS_BIG_NT / 64))   // values per wave
+__device__ __forceinline__ bool bk_kept_mass(const uint32_t* pv, uint32_t V, float cut, float& kept, big_shared& sh) {
+    constexpr uint32_t NW = ZS_BIG_NT / 64;
+    const uint32_t t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    const uint32_t seg = (V + 256u * NW - 1u) / (256u * NW) * 256u, w0 = wid * seg, w1 = min(w0 + seg, V);
+    float* list = reinterpret_cast<float*>(sh.sortbuf) + wid * BK_KEEP;
+    uint32_t n = 0;
+    for (uint32_t i0 = w0; i0 < w1; i0 += 256u * BK_U) {
+        uint4 v[BK_U];
+#pragma unroll
+        for (int u = 0; u < BK_U; u++) {
+            const uint32_t idx0 = i0 + 256u * (uint32_t)u + 4u * lane;
+            v[u] = idx0 < w1 ? *reinterpret_cast<const uint4*>(pv + idx0) : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int u = 0; u < BK_U; u++) {
+            const float p4[4] = {zs_u2f(v[u].x), zs_u2f(v[u].y), zs_u2f(v[u].z), zs_u2f(v[u].w)};
+            uint32_t p = n, c = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const unsigned long long m = __ballot(p4[q] >= cut && p4[q] > 0.0f);
+                p = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, p));
+                c += (uint32_t)__popcll(m);
+            }
+            if (c == 0) continue;
+            n += c;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (!(p4[q] >= cut && p4[q] > 0.0f)) continue;
+                if (p < BK_KEEP) list[p] = p4[q];
+                p++;
+            }
+        }
+    }
+    if (lane == 0) sh.hist2[wid] = n;
+    const bool over = __syncthreads_or(n > BK_KEEP);
+    if (over) return false;
+    if (t < 64) {
+        float s = 0.0f;
+        for (uint32_t w = 0; w < NW; w++) {
+            float r;
+            serial_scan_f(reinterpret_cast<float*>(sh.sortbuf) + w * BK_KEEP, sh.hist2[w], s, NAN, &r);
+            s = r;
+        }
+        if (t == 0) sh.s = s;
+    }
+    __syncthreads();
+    kept = sh.s;
+    __syncthreads();
+    return true;
+}
+
 __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_big(zs_sargs a) {
     const uint32_t r = blockIdx.x;
     zs_row_state stt = a.rst[r];
@@ -1159,7 +1227,8 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_big(zs_sargs a) {
     float kept = 0.0f;
     if (big_s_from_rounds(stt)) {
         // pv was filled by zs_k_pv; min-p needs the kept mass
-        if (minp) {
+        if (minp && !bk_kept_mass(pv, V, cut, kept, sh)) {
+            kept = 0.0f;
             for (uint32_t g = 0; g < ng; g++) {
                 const uint32_t idx0 = g * ZS_BIG_G + 4 * t;
                 uint4 v = idx0 < V ? *reinterpret_cast<const uint4*>(pv + idx0) : make_uint4(0u, 0u, 0u, 0u);
