@@ -1,0 +1,38 @@
+"""BTOPK for K <= 64 from group maxima (zs_k_lane_scan, zs_k_btopk_pick): rows
+and widths where groups, thresholds and lists can go wrong, against the
+oracle's WGSL restatement (ids and values bit for bit)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V", [50, 4096, 50257, 81921, 163844])
+@pytest.mark.parametrize("K", [1, 5, 64])
+def test_btopk_from_group_maxima(V, K):
+    from tests.gpu_util import ctx
+    from zllm_amd.engine import lane_topk
+    rng = np.random.default_rng(V + K)
+    x = rng.normal(0, 2, (9, V)).astype(np.float32)
+    x[0].sort()                                     # the top entries adjacent
+    x[1] = 1.5                                      # every key at the threshold
+    x[2] = np.where(rng.random(V) < 0.5, np.float32(0.0), np.float32(-0.0))
+    x[3] = -np.inf                                  # fewer candidates than K
+    x[3, [0, V // 2, V - 1]] = [1.0, np.nan, 2.0]
+    x[4] = np.round(x[4])                           # many ties
+    x[5, -3:] = [9.0, 3.2e38, 10.0]                 # the last, partial group; beyond the candidates' range
+    x[6, V // 3:V // 3 + 2000] = 20.0               # more equal keys than the lists hold
+    x[7, ::2] = np.nan
+    x[8] = np.nan
+    print(f"[case] btopk group maxima V={V} K={K}", flush=True)
+    xs = torch.zeros((9, (V + 3) // 4 * 4), device="cuda")
+    xs[:, :V] = torch.from_numpy(x)
+    vals, idxs = lane_topk(ctx(64, max(151936, V)), xs[:, :V], K)
+    vals, idxs = vals.cpu().numpy(), idxs.cpu().numpy().view(np.uint32)
+    for s in range(9):
+        ov, oi = O.btopk(x[s], K)
+        assert idxs[s].tolist() == oi.tolist(), s
+        assert vals[s].tobytes() == ov.tobytes(), s

@@ -20,13 +20,13 @@ extern "C" int zs_lane_argmax_launch(const float* logits, uint32_t B, uint32_t V
                                      uint32_t* out, hipStream_t stream);
 extern "C" int zs_lane_hash_fill(uint32_t* ih, uint32_t n, hipStream_t stream);
 extern "C" int zs_lane_topk_launch(const float* logits, uint32_t B, uint32_t V, uint64_t ld, uint32_t K,
-                                   float* vals, uint32_t* idxs, unsigned long long* ck, uint32_t* cn,
+                                   float* vals, uint32_t* idxs, uint32_t* gmax, uint32_t gstride,
                                    hipStream_t stream);
 extern "C" int zs_lane_sample_topk_launch(const float* vals, const uint32_t* idxs, uint32_t B, uint32_t K,
                                           const float* temp, const uint32_t* top_k, const float* top_p,
                                           const uint32_t* seed, uint32_t* out, hipStream_t stream);
 extern "C" int zs_lane_topk_draw_launch(const float* logits, uint32_t B, uint32_t V, uint64_t ld, uint32_t K,
-                                        float* vals, uint32_t* idxs, unsigned long long* ck, uint32_t* cn,
+                                        float* vals, uint32_t* idxs, uint32_t* gmax, uint32_t gstride,
                                         const float* temp, const uint32_t* top_k, const float* top_p,
                                         const uint32_t* seed, uint32_t* out, hipStream_t stream);
 extern "C" int zs_dfa_mask_launch(const dm_args& a, bool lds, uint32_t ncu, uint32_t* any_scratch, hipStream_t stream);
@@ -129,7 +129,7 @@ extern "C" void zs_ctx_destroy(zs_ctx* ctx) {
     void* ptrs[] = {ctx->p_cnt, ctx->p_id, ctx->p_flags, ctx->p_y, ctx->rst, ctx->pairs, ctx->pv, ctx->mask_scratch, ctx->spec_chunks,
                     ctx->spec_rows, ctx->p_sub, ctx->k_ap, ctx->k_sum, ctx->s_rec, ctx->s_apx, ctx->gath, ctx->s_hterm, ctx->tp_bk, ctx->tp_cl, ctx->tp_pre, ctx->kcnt, ctx->tp_task, ctx->gmax,
                     ctx->lane_temp, ctx->lane_vals, ctx->lane_ih, ctx->lane_keys,
-                    ctx->lane_idxs, ctx->lane_ck, ctx->lane_cn};
+                    ctx->lane_idxs, ctx->lane_gmax};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     (void)hipSetDevice(dev);
@@ -202,8 +202,7 @@ extern "C" int zs_ctx_create(int device, uint32_t max_rows, uint32_t max_vocab, 
     }
     if (!rc) rc = zs_alloc(ctx, &ctx->lane_vals, R * ZS_LANE_K);
     if (!rc) rc = zs_alloc(ctx, &ctx->lane_idxs, R * ZS_LANE_K);
-    if (!rc) rc = zs_alloc(ctx, &ctx->lane_ck, R * C * ZS_LANE_K);
-    if (!rc) rc = zs_alloc(ctx, &ctx->lane_cn, R * C);
+    if (!rc) rc = zs_alloc(ctx, &ctx->lane_gmax, R * ((size_t)max_vocab / ZS_SCAN_MIN_GROUP + 1));
     if (!rc) rc = zs_alloc(ctx, &ctx->lane_ih, (size_t)ctx->max_vocab + 4);
     if (!rc) rc = zs_alloc(ctx, &ctx->lane_keys, R);
     if (!rc && hipMemset(ctx->lane_keys, 0, R * sizeof(unsigned long long)) != hipSuccess) rc = ZS_EHIP;
@@ -954,8 +953,8 @@ extern "C" int zs_lane_topk(zs_ctx* ctx, const float* d_logits, uint32_t B, uint
     if (B == 0) return ZS_OK;
     int prev = zs_device_guard_begin(ctx);
     const bool fits = B <= ctx->max_rows && V <= ctx->max_vocab;
-    rc = zs_lane_topk_launch(d_logits, B, V, ld, K, d_vals, d_idxs, fits ? ctx->lane_ck : nullptr,
-                             fits ? ctx->lane_cn : nullptr, (hipStream_t)stream);
+    rc = zs_lane_topk_launch(d_logits, B, V, ld, K, d_vals, d_idxs, fits ? ctx->lane_gmax : nullptr,
+                             ctx->max_vocab / ZS_SCAN_MIN_GROUP + 1, (hipStream_t)stream);
     zs_device_guard_end(ctx, prev);
     return rc ? zs_set_error(ctx, ZS_EHIP, "zs_lane_topk: launch failed") : ZS_OK;
 }
@@ -1028,7 +1027,7 @@ extern "C" int zs_lane_step(zs_ctx* ctx, const float* d_logits, uint32_t m, uint
             rc = zs_lane_argmax_launch(d_logits, m, V, ld, ctx->lane_temp, ctx->lane_seed, ctx->lane_ih, ctx->lane_keys, d_out, st);
         else {
             rc = zs_lane_topk_draw_launch(d_logits, m, V, ld, ZS_LANE_K, ctx->lane_vals, ctx->lane_idxs,
-                                          V <= ctx->max_vocab ? ctx->lane_ck : nullptr, ctx->lane_cn, ctx->lane_temp,
+                                          V <= ctx->max_vocab ? ctx->lane_gmax : nullptr, ctx->max_vocab / ZS_SCAN_MIN_GROUP + 1, ctx->lane_temp,
                                           ctx->lane_topk, ctx->lane_topp, ctx->lane_seed, d_out, st);
         }
         if (rc) rc = ZS_EHIP;

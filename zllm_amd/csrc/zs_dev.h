@@ -6,6 +6,17 @@
 #define ZS_WAVE 64
 #define ZS_BIGI 0x7fffffff
 
+// A load through a global-address-space pointer (the host pass of the
+// compiler only parses device code, and has no such address space).
+template <class T>
+__device__ __forceinline__ T zs_gload(const T* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const __attribute__((address_space(1))) T*)p;
+#else
+    return *p;
+#endif
+}
+
 __device__ __forceinline__ int zs_lane() { return (int)(threadIdx.x & 63); }
 __device__ __forceinline__ int zs_wid() { return (int)(threadIdx.x >> 6); }
 

@@ -205,8 +205,7 @@ struct zs_ctx {
     uint32_t* lane_seed;         // [rows]
     float* lane_vals;            // [rows][ZS_LANE_K]
     uint32_t* lane_idxs;         // [rows][ZS_LANE_K]
-    unsigned long long* lane_ck; // [rows][chunks][ZS_LANE_K] chunk top-K lists (two-phase BTOPK)
-    uint32_t* lane_cn;           // [rows][chunks]
+    uint32_t* lane_gmax;         // [rows][max_vocab / ZS_SCAN_MIN_GROUP + 1] group maxima (zs_k_lane_scan)
     uint32_t* lane_ih;           // [max_vocab + 4] hash of every id (the id half of BSAMPLE's uniforms)
     unsigned long long* lane_keys;  // [rows] BSAMPLE's per-row best key (zero between calls)
     uint32_t* lane_host;         // pinned [2][4][rows]: temp, top_k, top_p, seed (two areas, alternating)

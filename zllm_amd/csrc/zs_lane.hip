@@ -276,26 +276,22 @@ __global__ void zs_k_bsample_fin(unsigned long long* keys, uint32_t B, uint32_t*
 __device__ __forceinline__ bool tk_cand(float v) { return v >= -3.0e38f && v < 3.0e38f; }
 __device__ __forceinline__ uint32_t tk_key(float v) { return zs_total_key(v == 0.0f ? 0.0f : v); }
 
-__global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
-                                                     float* vals, uint32_t* idxs) {
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t u[4];
-    __shared__ unsigned long long buf[TK_MAX];
-    __shared__ uint32_t scan_sh[LN_NT / 64];
-    const uint32_t r = blockIdx.x;
+// By an NT-thread workgroup over its row, six passes (buf: KMAX >= K entries).
+template <int NT, int KMAX>
+__device__ __forceinline__ void tk_row_radix(const float* row, uint32_t V, uint32_t K, float* vals, uint32_t* idxs,
+                                             unsigned long long* buf, uint32_t* hist, uint32_t* u, uint32_t* scan_sh) {
     const int t = threadIdx.x;
-    const float* row = logits + (size_t)r * ld;
     // radix select of the K-th largest candidate key
     uint32_t ncand = 0;
-    for (uint32_t i = t; i < V; i += LN_NT) ncand += tk_cand(row[i]) ? 1u : 0u;
-    ncand = block_sum_u<LN_NT>(ncand, scan_sh);
+    for (uint32_t i = t; i < V; i += NT) ncand += tk_cand(row[i]) ? 1u : 0u;
+    ncand = block_sum_u<NT>(ncand, scan_sh);
     const uint32_t KK = ncand < K ? ncand : K;
     uint32_t prefix = 0, mask = 0, need = KK;
     if (KK > 0) {
         for (int shift = 24; shift >= 0; shift -= 8) {
-            if (t < 256) hist[t] = 0;
+            for (int i = t; i < 256; i += NT) hist[i] = 0;
             __syncthreads();
-            for (uint32_t i = t; i < V; i += LN_NT) {
+            for (uint32_t i = t; i < V; i += NT) {
                 float v = row[i];
                 if (!tk_cand(v)) continue;
                 uint32_t k = tk_key(v);
@@ -323,17 +319,17 @@ __global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_
     if (t == 0) u[2] = 0;
     __syncthreads();
     uint32_t carry = 0;
-    for (uint32_t base = 0; base < V && KK > 0; base += LN_NT) {
+    for (uint32_t base = 0; base < V && KK > 0; base += NT) {
         uint32_t i = base + t;
         float v = i < V ? row[i] : NAN;
         bool c = i < V && tk_cand(v);
         uint32_t k = c ? tk_key(v) : 0;
         bool gt = c && k > prefix, eq = c && k == prefix;
         uint32_t tot;
-        uint32_t ex = block_excl_scan_u<LN_NT>(eq ? 1u : 0u, scan_sh, &tot);
+        uint32_t ex = block_excl_scan_u<NT>(eq ? 1u : 0u, scan_sh, &tot);
         if (gt || (eq && carry + ex < need)) {
             uint32_t pos = atomicAdd(&u[2], 1u);
-            if (pos < TK_MAX) buf[pos] = ((unsigned long long)(~k) << 32) | i;
+            if (pos < KMAX) buf[pos] = ((unsigned long long)(~k) << 32) | i;
         }
         carry += tot;
     }
@@ -341,179 +337,81 @@ __global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_
     uint32_t n = KK;
     uint32_t np2 = 1;
     while (np2 < n) np2 <<= 1;
-    for (uint32_t i = n + t; i < np2; i += LN_NT) buf[i] = ~0ull;
+    for (uint32_t i = n + t; i < np2; i += NT) buf[i] = ~0ull;
     __syncthreads();
-    if (np2 > 1) block_sort_u64<LN_NT>(buf, np2);
-    for (uint32_t j = t; j < K; j += LN_NT) {
+    if (np2 > 1) block_sort_u64<NT>(buf, np2);
+    for (uint32_t j = t; j < K; j += NT) {
         if (j < n) {
             uint32_t id = (uint32_t)(buf[j] & 0xffffffffull);
-            vals[(size_t)r * K + j] = row[id];
-            idxs[(size_t)r * K + j] = id;
+            vals[j] = row[id];
+            idxs[j] = id;
         } else {
-            vals[(size_t)r * K + j] = -3.0e38f;
-            idxs[(size_t)r * K + j] = 0xffffffffu;
+            vals[j] = -3.0e38f;
+            idxs[j] = 0xffffffffu;
         }
     }
 }
 
-// Two-phase BTOPK for K <= 64: every 16384-id chunk keeps its own top-K by
-// (key desc, id asc) -- a superset of the row's top-K restricted to the chunk
-// -- and one workgroup per row sorts the chunk lists. Same result as
-// zs_k_btopk; one read of the row over the whole chip instead of six passes
-// by one workgroup.
-#define TC_NT 256
-#define TC_CH 16384
-#define TC_EPT (TC_CH / TC_NT)
-#define TC_SORT 256
-#define TC_K 64
-#define TC_MAXCH 32
-__global__ __launch_bounds__(TC_NT) void zs_k_btopk_chunks(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
-                                                            unsigned long long* ck, uint32_t* cn, uint32_t nch) {
-    __shared__ uint32_t tmax[TC_NT];
-    __shared__ unsigned long long s64[TC_SORT];
+__global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
+                                                     float* vals, uint32_t* idxs) {
     __shared__ uint32_t hist[256];
     __shared__ uint32_t u[4];
-    __shared__ uint32_t scan_sh[TC_NT / 64];
-    const uint32_t c = blockIdx.x, r = blockIdx.y;
-    const int t = threadIdx.x, lane = zs_lane(), wid = zs_wid();
-    const uint32_t base = c * TC_CH;
-    const float* row = logits + (size_t)r * ld;
-    unsigned long long* out = ck + ((size_t)r * nch + c) * TC_K;
-    // keys of the thread's elements: float4 j covers ids base + (j*NT + t)*4 .. +3;
-    // 0 for ids past V and for non-candidates (below every candidate key)
-    uint32_t key[TC_EPT];
-#pragma unroll
-    for (int j = 0; j < TC_EPT / 4; j++) {
-        const uint32_t id = base + (j * TC_NT + t) * 4;
-        float4 v = make_float4(NAN, NAN, NAN, NAN);
-        if (id + 3 < V) v = *reinterpret_cast<const float4*>(row + id);
-        else {
-            if (id < V) v.x = row[id];
-            if (id + 1 < V) v.y = row[id + 1];
-            if (id + 2 < V) v.z = row[id + 2];
-        }
-        const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int q = 0; q < 4; q++) key[4 * j + q] = tk_cand(vv[q]) ? tk_key(vv[q]) : 0u;
-    }
-    auto idx_of = [&](int e) { return base + ((e >> 2) * TC_NT + t) * 4 + (e & 3); };
-    uint32_t tm = 0;
-#pragma unroll
-    for (int e = 0; e < TC_EPT; e++) tm = max(tm, key[e]);
-    // theta: the K-th largest of the 256 thread maxima (maxima of distinct
-    // elements, so at least K keys are >= theta when K threads hold one)
-    const uint32_t srt = wave_sort_u32(tm);
-    tmax[wid * 64 + lane] = srt;
-    __syncthreads();
-    if (t < 64) {
-        uint32_t m = srt;
-#pragma unroll
-        for (int w = 1; w < TC_NT / 64; w++) {
-            m = max(m, tmax[w * 64 + 63 - lane]);
-#pragma unroll
-            for (int j = 32; j > 0; j >>= 1) {
-                const uint32_t o = __shfl_xor(m, j, 64);
-                m = (lane & j) ? max(m, o) : min(m, o);
-            }
-        }
-        if (lane == 64 - (int)K) u[0] = m;
-    }
-    __syncthreads();
-    const uint32_t theta = max(u[0], 1u);
-    uint32_t cnt = 0;
-#pragma unroll
-    for (int e = 0; e < TC_EPT; e++) cnt += key[e] >= theta ? 1u : 0u;
-    uint32_t nsup;
-    uint32_t pos = block_excl_scan_u<TC_NT>(cnt, scan_sh, &nsup);
-    if (nsup <= TC_SORT) {
-#pragma unroll
-        for (int e = 0; e < TC_EPT; e++)
-            if (key[e] >= theta) s64[pos++] = ((unsigned long long)(~key[e]) << 32) | idx_of(e);
-        __syncthreads();
-        const uint32_t n = min(K, nsup);
-        if (nsup <= 64) {
-            if (t < 64) {
-                unsigned long long v = (uint32_t)t < nsup ? s64[t] : ~0ull;
-                v = wave_sort_u64(v);
-                if ((uint32_t)t < n) out[t] = v;
-            }
-        } else {
-            for (uint32_t i = nsup + t; i < TC_SORT; i += TC_NT) s64[i] = ~0ull;
-            __syncthreads();
-            block_sort_u64<TC_NT>(s64, TC_SORT);
-            if ((uint32_t)t < n) out[t] = s64[t];
-        }
-        if (t == 0) cn[(size_t)r * nch + c] = n;
-        return;
-    }
-    // many keys tie near theta: exact K-th key by an 8-bit radix select, then
-    // the keys above it and the lowest ids among the keys equal to it
-    uint32_t ncand = 0;
-#pragma unroll
-    for (int e = 0; e < TC_EPT; e++) ncand += key[e] ? 1u : 0u;
-    ncand = block_sum_u<TC_NT>(ncand, scan_sh);
-    const uint32_t KK = min(K, ncand);
-    uint32_t prefix = 0, mask = 0, need = KK;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        hist[t] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < TC_EPT; e++)
-            if (key[e] && (key[e] & mask) == prefix) atomicAdd(&hist[(key[e] >> shift) & 255u], 1u);
-        __syncthreads();
-        if (t < 64) {
-            uint32_t cc[4], loc = 0;
-            for (int q = 0; q < 4; q++) { cc[q] = hist[255 - 4 * t - q]; loc += cc[q]; }
-            uint32_t inc = wave_incl_scan_u(loc);
-            uint32_t before = inc - loc;
-            for (int q = 0; q < 4; q++) {
-                if (before < need && need <= before + cc[q]) { u[1] = 255 - 4 * t - q; u[2] = need - before; }
-                before += cc[q];
-            }
-        }
-        __syncthreads();
-        prefix |= u[1] << shift;
-        mask |= 0xffu << shift;
-        need = u[2];
-        __syncthreads();
-    }
-    if (t == 0) u[3] = 0;
-    __syncthreads();
-    uint32_t carry = 0;  // the KK chosen keys are gathered in s64, then sorted
-#pragma unroll
-    for (int j = 0; j < TC_EPT / 4; j++) {  // ids ascend with j, then t, then q
-        uint32_t ce = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) ce += key[4 * j + q] == prefix ? 1u : 0u;
-        uint32_t tot;
-        uint32_t rank = carry + block_excl_scan_u<TC_NT>(ce, scan_sh, &tot);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t k = key[4 * j + q];
-            bool take = k && k > prefix;
-            if (k && k == prefix) { take = rank < need; rank++; }
-            if (take) {
-                const uint32_t p = atomicAdd(&u[3], 1u);
-                if (p < TC_K) s64[p] = ((unsigned long long)(~k) << 32) | idx_of(4 * j + q);
-            }
-        }
-        carry += tot;
-    }
-    __syncthreads();
-    if (t < 64) {
-        unsigned long long v = (uint32_t)t < KK ? s64[t] : ~0ull;
-        v = wave_sort_u64(v);
-        if ((uint32_t)t < KK) out[t] = v;
-    }
-    if (t == 0) cn[(size_t)r * nch + c] = KK;
+    __shared__ unsigned long long buf[TK_MAX];
+    __shared__ uint32_t scan_sh[LN_NT / 64];
+    const size_t r = blockIdx.x;
+    tk_row_radix<LN_NT, TK_MAX>(logits + r * ld, V, K, vals + r * K, idxs + r * K, buf, hist, u, scan_sh);
 }
 
-// One wave per row: the chunk lists are sorted (best first), so the row's
-// best K is a running merge -- the elementwise min of the kept list and the
-// reversed next list holds the 64 best of both as a bitonic sequence, which
-// six exchange steps sort.
-#define TM_ROWS 4
-struct tm_draw {   // the nucleus draw after the merge (zs_lane_step's top-K path)
+// BTOPK for K <= 64 from group maxima. zs_k_lane_scan reads the logits once
+// over the whole GPU and leaves the largest candidate key of every group of
+// 2^gshift consecutive ids; zs_k_btopk_pick (one workgroup per row) takes a
+// key that at least K groups reach: the row's first K by (key desc, id asc)
+// lie in the groups whose maximum reaches it, a few more than K, whose ids are
+// read again, listed and sorted. With the draw of zs_lane_step's top-K path
+// in the same kernel. 256 rows of 151936 ids: the scan 24 us (6.5 TB/s), the
+// pick 20 us; chunks of 16384 ids with a top-K each and a merge took 54 + 20.
+#define LS_NT 256
+#define LS_IDS (16 * LS_NT)   // ids per workgroup of the scan
+#define LP_NT 256
+#define LP_GPT 20             // groups per thread of the pick at most
+#define LP_GL 1024            // listed groups at most
+#define LP_LIST 1024          // listed keys at most
+#define TC_K 64
+template <int GS>
+__global__ __launch_bounds__(LS_NT) void zs_k_lane_scan(const float* logits, uint32_t V, uint64_t ld, uint32_t* gmax,
+                                                        uint32_t gstride) {
+    typedef float ls_f4 __attribute__((ext_vector_type(4)));
+    const uint32_t r = blockIdx.y, lane = (uint32_t)zs_lane();
+    const float* row = logits + (size_t)r * ld;
+    const uint32_t base = blockIdx.x * LS_IDS + 4u * threadIdx.x;
+    const uint32_t last4 = (V - 1u) & ~3u;   // (rows are whole multiples of 4 in memory)
+    ls_f4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const ls_f4*>(row + min(base + (uint32_t)u * (4u * LS_NT), last4));
+    uint32_t k[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint32_t id = base + (uint32_t)u * (4u * LS_NT);
+        const float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+        // (non-candidates, NaN among them, count as no value)
+        float m = -INFINITY;
+#pragma unroll
+        for (int q = 0; q < 4; q++) m = fmaxf(m, id + (uint32_t)q < V && tk_cand(x[q]) ? x[q] : -INFINITY);
+        k[u] = tk_cand(m) ? tk_key(m) : 0u;
+        k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
+        k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
+        if (GS >= 5) k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x141, 0xf, 0xf, false));   // row_half_mirror
+        if (GS >= 6) k[u] = max(k[u], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k[u], 0x140, 0xf, 0xf, false));   // row_mirror
+    }
+    // lane q of a quad stores load q's group (one store for all four)
+    constexpr uint32_t LG = 1u << (GS - 2);   // lanes per group
+    const uint32_t q = lane & 3u;
+    const uint32_t kq = q == 0 ? k[0] : q == 1 ? k[1] : q == 2 ? k[2] : k[3];
+    const uint32_t g = (blockIdx.x * LS_IDS + q * (4u * LS_NT) + 4u * threadIdx.x) >> GS;
+    if ((lane & (LG - 1u)) < 4u && g < (V + (1u << GS) - 1u) >> GS) gmax[(size_t)r * gstride + g] = kq;
+}
+
+struct tm_draw {   // the nucleus draw after the pick (zs_lane_step's top-K path)
     const float* temp;
     const uint32_t *top_k;
     const float* top_p;
@@ -523,42 +421,122 @@ struct tm_draw {   // the nucleus draw after the merge (zs_lane_step's top-K pat
 __device__ __forceinline__ uint32_t lane_draw64(float v, uint32_t id, uint32_t K, float T, uint32_t top_k, float tp,
                                                 uint32_t seed);
 template <bool DRAW>
-__global__ __launch_bounds__(64 * TM_ROWS) void zs_k_btopk_merge(const float* logits, uint32_t B, uint64_t ld,
-                                                                  uint32_t K, const unsigned long long* ck,
-                                                                  const uint32_t* cn, uint32_t nch, float* vals,
-                                                                  uint32_t* idxs, tm_draw d) {
-    const uint32_t r = blockIdx.x * TM_ROWS + zs_wid();
-    if (r >= B) return;
-    const int lane = zs_lane();
-    unsigned long long cur = ~0ull;
-    for (uint32_t c = 0; c < nch; c++) {
-        const uint32_t n = cn[(size_t)r * nch + c];
-        unsigned long long b = (uint32_t)lane < n ? ck[((size_t)r * nch + c) * TC_K + lane] : ~0ull;
-        b = __shfl(b, 63 - lane, 64);
-        unsigned long long m = b < cur ? b : cur;
+__global__ __launch_bounds__(LP_NT) void zs_k_btopk_pick(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
+                                                         const uint32_t* gmax, uint32_t gstride, uint32_t gs, float* vals,
+                                                         uint32_t* idxs, tm_draw d) {
+    constexpr uint32_t NW = LP_NT / 64;
+    __shared__ unsigned long long list[LP_LIST];
+    __shared__ uint16_t gl[LP_GL];
+    __shared__ uint32_t hist[256], u[4], scan_sh[NW], wthr[NW];
+    const uint32_t r = blockIdx.x, t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    const float* row = logits + (size_t)r * ld;
+    const uint32_t ng = (V + (1u << gs) - 1u) >> gs, last4 = (V - 1u) & ~3u;
+    const uint32_t* gm = gmax + (size_t)r * gstride;
+    uint32_t k[LP_GPT], tm = 0;
 #pragma unroll
-        for (int j = 32; j > 0; j >>= 1) {
-            const unsigned long long o = __shfl_xor(m, j, 64);
-            m = (lane & j) ? (o > m ? o : m) : (o < m ? o : m);
-        }
-        cur = m;
+    for (int e = 0; e < LP_GPT; e++) k[e] = zs_gload(gm + min(t + (uint32_t)e * LP_NT, ng - 1u));
+#pragma unroll
+    for (int e = 0; e < LP_GPT; e++) {
+        if (t + (uint32_t)e * LP_NT >= ng) k[e] = 0u;
+        tm = max(tm, k[e]);
     }
+    if (t < 2) u[t] = 0;
+    // theta: in every wave the ceil(K / waves)-th largest thread maximum; the
+    // smallest of them is reached by K groups (0: too few hold a candidate;
+    // every candidate is listed then)
+    const uint32_t srt = wave_sort_u32(tm);
+    const uint32_t wt = (uint32_t)__builtin_amdgcn_readlane((int)srt, 64 - (int)((K + NW - 1u) / NW));
+    if (lane == 0) wthr[wid] = wt;
+    __syncthreads();
+    uint32_t theta = wthr[0];
+#pragma unroll
+    for (uint32_t w = 1; w < NW; w++) theta = min(theta, wthr[w]);
+    theta = max(theta, 1u);
+#pragma unroll
+    for (int e = 0; e < LP_GPT; e++) {
+        if (k[e] < theta) continue;
+        const uint32_t p = atomicAdd(&u[0], 1u);
+        if (p < LP_GL) gl[p] = (uint16_t)(t + (uint32_t)e * LP_NT);
+    }
+    __syncthreads();
+    const uint32_t n_gl = u[0], qs = gs - 2u, nit = n_gl << qs;
+    if (n_gl <= LP_GL) {
+        constexpr int NU = 4;
+        for (uint32_t i0 = 0; i0 < nit; i0 += NU * LP_NT) {
+            typedef float ls_f4 __attribute__((ext_vector_type(4)));
+            ls_f4 v[NU];
+            uint32_t id[NU];
+#pragma unroll
+            for (int w = 0; w < NU; w++) {
+                const uint32_t i = i0 + t + (uint32_t)w * LP_NT, ic = min(i, nit - 1u);
+                id[w] = ((uint32_t)gl[ic >> qs] << gs) + 4u * (ic & ((1u << qs) - 1u));
+                v[w] = zs_gload(reinterpret_cast<const ls_f4*>(row + min(id[w], last4)));
+                if (i >= nit) id[w] = V;
+            }
+#pragma unroll
+            for (int w = 0; w < NU; w++) {
+                const float x[4] = {v[w].x, v[w].y, v[w].z, v[w].w};
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (id[w] + (uint32_t)q >= V || !tk_cand(x[q])) continue;
+                    const uint32_t kq = tk_key(x[q]);
+                    if (kq < theta) continue;
+                    const uint32_t p = atomicAdd(&u[1], 1u);
+                    if (p < LP_LIST) list[p] = ((unsigned long long)(~kq) << 32) | (id[w] + (uint32_t)q);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t n = u[1];
     float v = -3.0e38f;
     uint32_t id = 0xffffffffu;
-    if ((uint32_t)lane < K) {
-        if (cur != ~0ull) {
-            id = (uint32_t)(cur & 0xffffffffull);
-            v = logits[(size_t)r * ld + id];
+    if (n_gl <= LP_GL && n <= LP_LIST) {
+        uint32_t np2 = 64;
+        while (np2 < n) np2 <<= 1;
+        for (uint32_t i = n + t; i < np2; i += LP_NT) list[i] = ~0ull;
+        __syncthreads();
+        block_sort_u64<LP_NT>(list, np2);
+        if (t >= 64) return;
+        const unsigned long long e = lane < min(K, n) ? list[lane] : ~0ull;
+        if (e != ~0ull) {
+            id = (uint32_t)e;
+            v = row[id];
         }
-        vals[(size_t)r * K + lane] = v;
-        idxs[(size_t)r * K + lane] = id;
+        if (lane < K) {
+            vals[(size_t)r * K + lane] = v;
+            idxs[(size_t)r * K + lane] = id;
+        }
+    } else {
+        // more equal maxima or more keys than the lists hold
+        tk_row_radix<LP_NT, LP_LIST>(row, V, K, vals + (size_t)r * K, idxs + (size_t)r * K, list, hist, u, scan_sh);
+        __threadfence_block();
+        __syncthreads();
+        if (t >= 64) return;
+        if (lane < K) {
+            v = vals[(size_t)r * K + lane];
+            id = idxs[(size_t)r * K + lane];
+        }
     }
     if (DRAW) {
         // the pool as zs_k_sample_topk64 reads it back
-        const uint32_t res = lane_draw64((uint32_t)lane < K ? v : -INFINITY, (uint32_t)lane < K ? id : 0u, K,
-                                         d.temp[r], d.top_k[r], d.top_p[r], d.seed[r]);
+        const uint32_t res = lane_draw64(lane < K ? v : -INFINITY, lane < K ? id : 0u, K, d.temp[r], d.top_k[r],
+                                         d.top_p[r], d.seed[r]);
         if (lane == 0) d.out[r] = res;
     }
+}
+// Launches the scan and the pick; gmax: B rows of gstride >= ceil(V / 16) keys.
+template <bool DRAW>
+static void lane_topk_groups(const float* logits, uint32_t B, uint32_t V, uint64_t ld, uint32_t K, float* vals,
+                             uint32_t* idxs, uint32_t* gmax, uint32_t gstride, const tm_draw& d, hipStream_t stream) {
+    uint32_t gs = 4;
+    while (((V + (1u << gs) - 1u) >> gs) > LP_GPT * LP_NT) gs++;
+    const dim3 grid((V + LS_IDS - 1) / LS_IDS, B);
+    if (gs == 4) hipLaunchKernelGGL(zs_k_lane_scan<4>, grid, dim3(LS_NT), 0, stream, logits, V, ld, gmax, gstride);
+    else if (gs == 5) hipLaunchKernelGGL(zs_k_lane_scan<5>, grid, dim3(LS_NT), 0, stream, logits, V, ld, gmax, gstride);
+    else hipLaunchKernelGGL(zs_k_lane_scan<6>, grid, dim3(LS_NT), 0, stream, logits, V, ld, gmax, gstride);
+    hipLaunchKernelGGL(zs_k_btopk_pick<DRAW>, dim3(B), dim3(LP_NT), 0, stream, logits, V, ld, K, gmax, gstride, gs, vals,
+                       idxs, d);
 }
 
 // gpu/sampling.rs:24-31
@@ -645,6 +623,7 @@ __device__ __forceinline__ uint32_t lane_draw64(float v, uint32_t id, uint32_t K
     return __shfl(id, (int)pick, 64);
 }
 
+#define TM_ROWS 4
 __global__ __launch_bounds__(64 * TM_ROWS) void zs_k_sample_topk64(const float* vals, const uint32_t* idxs,
                                                                     uint32_t B, uint32_t K, const float* temp,
                                                                     const uint32_t* top_k, const float* top_p,
@@ -672,38 +651,32 @@ extern "C" int zs_lane_argmax_launch(const float* logits, uint32_t B, uint32_t V
     hipLaunchKernelGGL(zs_k_bargmax, dim3(B), dim3(LN_NT), 0, stream, logits, V, ld, out);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
-// ck / cn: scratch of at least B * ceil(V / TC_CH) * 64 keys and B * ceil(V / TC_CH)
-// counts (two-phase path, K <= 64, V <= 32 * TC_CH); nullptr forces one pass
+// gmax: scratch of B rows of gstride >= ceil(V / 16) keys (the path from group
+// maxima, K <= 64, V <= ZS_MAX_VOCAB); nullptr forces the passes by one workgroup
 extern "C" int zs_lane_topk_launch(const float* logits, uint32_t B, uint32_t V, uint64_t ld, uint32_t K,
-                                   float* vals, uint32_t* idxs, unsigned long long* ck, uint32_t* cn,
+                                   float* vals, uint32_t* idxs, uint32_t* gmax, uint32_t gstride,
                                    hipStream_t stream) {
-    const uint32_t nch = (V + TC_CH - 1) / TC_CH;
-    if (ck && cn && K <= TC_K && nch <= TC_MAXCH) {
-        hipLaunchKernelGGL(zs_k_btopk_chunks, dim3(nch, B), dim3(TC_NT), 0, stream, logits, V, ld, K, ck, cn, nch);
-        hipLaunchKernelGGL(zs_k_btopk_merge<false>, dim3((B + TM_ROWS - 1) / TM_ROWS), dim3(64 * TM_ROWS), 0, stream,
-                           logits, B, ld, K, ck, cn, nch, vals, idxs, tm_draw{});
+    if (gmax && K <= TC_K && V <= ZS_MAX_VOCAB) {
+        lane_topk_groups<false>(logits, B, V, ld, K, vals, idxs, gmax, gstride, tm_draw{}, stream);
     } else {
         hipLaunchKernelGGL(zs_k_btopk, dim3(B), dim3(LN_NT), 0, stream, logits, V, ld, K, vals, idxs);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
-// The top-K pool and its nucleus draw: on the two-phase path the merge kernel
+// The top-K pool and its nucleus draw: on the group path the pick kernel
 // draws too (one launch and no read-back of the pool), else the two launches.
 extern "C" int zs_lane_sample_topk_launch(const float* vals, const uint32_t* idxs, uint32_t B, uint32_t K,
                                           const float* temp, const uint32_t* top_k, const float* top_p,
                                           const uint32_t* seed, uint32_t* out, hipStream_t stream);
 extern "C" int zs_lane_topk_draw_launch(const float* logits, uint32_t B, uint32_t V, uint64_t ld, uint32_t K,
-                                        float* vals, uint32_t* idxs, unsigned long long* ck, uint32_t* cn,
+                                        float* vals, uint32_t* idxs, uint32_t* gmax, uint32_t gstride,
                                         const float* temp, const uint32_t* top_k, const float* top_p,
                                         const uint32_t* seed, uint32_t* out, hipStream_t stream) {
-    const uint32_t nch = (V + TC_CH - 1) / TC_CH;
-    if (ck && cn && K <= TC_K && nch <= TC_MAXCH) {
-        hipLaunchKernelGGL(zs_k_btopk_chunks, dim3(nch, B), dim3(TC_NT), 0, stream, logits, V, ld, K, ck, cn, nch);
-        hipLaunchKernelGGL(zs_k_btopk_merge<true>, dim3((B + TM_ROWS - 1) / TM_ROWS), dim3(64 * TM_ROWS), 0, stream,
-                           logits, B, ld, K, ck, cn, nch, vals, idxs, tm_draw{temp, top_k, top_p, seed, out});
+    if (gmax && K <= TC_K && V <= ZS_MAX_VOCAB) {
+        lane_topk_groups<true>(logits, B, V, ld, K, vals, idxs, gmax, gstride, tm_draw{temp, top_k, top_p, seed, out}, stream);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
-    if (zs_lane_topk_launch(logits, B, V, ld, K, vals, idxs, ck, cn, stream)) return -1;
+    if (zs_lane_topk_launch(logits, B, V, ld, K, vals, idxs, gmax, gstride, stream)) return -1;
     return zs_lane_sample_topk_launch(vals, idxs, B, K, temp, top_k, top_p, seed, out, stream);
 }
 extern "C" int zs_lane_sample_topk_launch(const float* vals, const uint32_t* idxs, uint32_t B, uint32_t K,

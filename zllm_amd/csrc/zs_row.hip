@@ -390,16 +390,6 @@ struct rw_raw {
     uint32_t w;   // the allow word holding the 4 ids
     uint32_t pw;  // the patch bitmap word holding them (rows with patches)
 };
-// A load through a global-address-space pointer (the host pass of the
-// compiler only parses device code, and has no such address space).
-template <class T>
-__device__ __forceinline__ T rw_gload(const T* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return *(const __attribute__((address_space(1))) T*)p;
-#else
-    return *p;
-#endif
-}
 // Loads of tile g for this thread, as global-memory loads (a generic pointer
 // would be loaded with flat instructions, whose completion every LDS wait
 // also waits for). Unconditional, from addresses clamped into the row (rows
@@ -409,9 +399,9 @@ __device__ __forceinline__ rw_raw rw_fetch(const rw_row& R, uint32_t g) {
     const uint32_t idx0 = min(g * RW_G + 4 * threadIdx.x, R.ldm4);
     rw_raw o;
     typedef float rw_f4 __attribute__((ext_vector_type(4)));
-    const rw_f4 v = rw_gload(reinterpret_cast<const rw_f4*>(R.row + idx0));
+    const rw_f4 v = zs_gload(reinterpret_cast<const rw_f4*>(R.row + idx0));
     o.v = make_float4(v.x, v.y, v.z, v.w);
-    o.w = rw_gload(R.allow_or_row + min(idx0 >> 5, R.wmax));
+    o.w = zs_gload(R.allow_or_row + min(idx0 >> 5, R.wmax));
     // read with the loads, long before its use
     o.pw = R.np ? rw_pbits[min((g * RW_G + 4 * threadIdx.x) >> 5, R.words - 1)] : 0u;
     return o;
@@ -724,7 +714,7 @@ __device__ __noinline__ uint32_t rw_gather_allowed(const float* row, const uint3
     // words with a load per id took 10 us on JSON masks)
     const uint32_t per = ((words + RW_NT - 1) / RW_NT) * 64u, w0 = wid * per, w1 = min(w0 + per, words);
     auto word = [&](uint32_t w) {
-        uint32_t a = w < w1 ? rw_gload(allow + w) : 0u;
+        uint32_t a = w < w1 ? zs_gload(allow + w) : 0u;
         if (w == words - 1 && (V & 31)) a &= (1u << (V & 31)) - 1u;
         return a;
     };
@@ -775,7 +765,7 @@ __device__ __noinline__ uint32_t rw_gather_allowed(const float* row, const uint3
 #pragma unroll
     for (uint32_t e = 0; e < NE; e++) {
         id[e] = lid[min(t + e * RW_NT, n - 1u)];
-        xv[e] = rw_gload(row + id[e]);
+        xv[e] = zs_gload(row + id[e]);
     }
 #pragma unroll
     for (uint32_t e = 0; e < NE; e++) {
@@ -1010,8 +1000,8 @@ __device__ __forceinline__ void rw_load4(const rw_row& R, uint32_t idx0, const f
 __device__ __forceinline__ float4 rw_fetch4(const rw_row& R, uint32_t idx0, uint32_t& w) {
     typedef float rw_f4 __attribute__((ext_vector_type(4)));
     const uint32_t ia = min(idx0, R.ldm4);
-    const rw_f4 v = rw_gload(reinterpret_cast<const rw_f4*>(R.row + ia));
-    w = rw_gload(R.allow_or_row + min(ia >> 5, R.wmax));
+    const rw_f4 v = zs_gload(reinterpret_cast<const rw_f4*>(R.row + ia));
+    w = zs_gload(R.allow_or_row + min(ia >> 5, R.wmax));
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
@@ -1075,7 +1065,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     {
         uint32_t k[RW_GPT];
 #pragma unroll
-        for (int e = 0; e < RW_GPT; e++) k[e] = rw_gload(gm + min(t + (uint32_t)e * RW_NT, ng - 1u));
+        for (int e = 0; e < RW_GPT; e++) k[e] = zs_gload(gm + min(t + (uint32_t)e * RW_NT, ng - 1u));
 #pragma unroll
         for (int e = 0; e < RW_GPT; e++) {
             const uint32_t i = t + (uint32_t)e * RW_NT;
