@@ -20,30 +20,78 @@ __device__ __forceinline__ T zs_gload(const T* p) {
 __device__ __forceinline__ int zs_lane() { return (int)(threadIdx.x & 63); }
 __device__ __forceinline__ int zs_wid() { return (int)(threadIdx.x >> 6); }
 
-__device__ __forceinline__ float wave_max_f(float v) {
-    for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
+// The value of lane (lane ^ J), J a power of two below 64, by register moves:
+// permutations inside quads, shifts and rotations inside rows of 16 lanes, and
+// the row swaps of gfx950 across them. A lane shuffle goes through the LDS
+// crossbar instead: its latency (and, for the sorts of a full workgroup, its
+// rate) bounded the sorting networks and reductions that used it (zs_k_row on
+// 64 x 128256: 31.9 -> 30.1 us).
+template <int J>
+__device__ __forceinline__ uint32_t zs_lane_xor(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int x = (int)v;
+    if constexpr (J == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true);         // quad_perm [1,0,3,2]
+    else if constexpr (J == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true);    // quad_perm [2,3,0,1]
+    else if constexpr (J == 4) {
+        const int lo = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);                           // row_shl:4, banks 0 and 2
+        return (uint32_t)__builtin_amdgcn_update_dpp(lo, x, 0x114, 0xf, 0xa, false);                        // row_shr:4, banks 1 and 3
+    } else if constexpr (J == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true); // row_ror:8
+    else if constexpr (J == 16) {
+        // odd rows of the first operand swap with even rows of the second
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (zs_lane() & 16) ? r[0] : r[1];
+    } else {
+        static_assert(J == 32, "a power of two below the wave width");
+        // the upper half of the first operand swaps with the lower half of the second
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (zs_lane() & 32) ? r[0] : r[1];
+    }
+#else
     return v;
+#endif
 }
-__device__ __forceinline__ double wave_sum_d(double v) {
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+template <int J>
+__device__ __forceinline__ int zs_lane_xor(int v) { return (int)zs_lane_xor<J>((uint32_t)v); }
+template <int J>
+__device__ __forceinline__ float zs_lane_xor(float v) { return __uint_as_float(zs_lane_xor<J>(__float_as_uint(v))); }
+template <int J>
+__device__ __forceinline__ unsigned long long zs_lane_xor(unsigned long long v) {
+    return ((unsigned long long)zs_lane_xor<J>((uint32_t)(v >> 32)) << 32) | zs_lane_xor<J>((uint32_t)v);
 }
-__device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) {
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+template <int J>
+__device__ __forceinline__ double zs_lane_xor(double v) {
+    return __longlong_as_double((long long)zs_lane_xor<J>((unsigned long long)__double_as_longlong(v)));
 }
-__device__ __forceinline__ int wave_min_i(int v) {
-    for (int d = 32; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
-    return v;
+// The same for a stride that is a constant once its loop is unrolled.
+template <class T>
+__device__ __forceinline__ T zs_lane_xor_by(T v, uint32_t j) {
+    switch (j) {
+        case 1: return zs_lane_xor<1>(v);
+        case 2: return zs_lane_xor<2>(v);
+        case 4: return zs_lane_xor<4>(v);
+        case 8: return zs_lane_xor<8>(v);
+        case 16: return zs_lane_xor<16>(v);
+        default: return zs_lane_xor<32>(v);
+    }
 }
-__device__ __forceinline__ int wave_max_i(int v) {
-    for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    return v;
+// Reduction over the wave, the result on every lane (lanes pair up at
+// distance 32, 16, ... 1).
+template <class T, class F>
+__device__ __forceinline__ T zs_wave_reduce(T v, const F& f) {
+    v = f(v, zs_lane_xor<32>(v));
+    v = f(v, zs_lane_xor<16>(v));
+    v = f(v, zs_lane_xor<8>(v));
+    v = f(v, zs_lane_xor<4>(v));
+    v = f(v, zs_lane_xor<2>(v));
+    return f(v, zs_lane_xor<1>(v));
 }
-__device__ __forceinline__ uint32_t wave_or_u(uint32_t v) {
-    for (int d = 32; d > 0; d >>= 1) v |= __shfl_xor(v, d, 64);
-    return v;
-}
+
+__device__ __forceinline__ float wave_max_f(float v) { return zs_wave_reduce(v, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ double wave_sum_d(double v) { return zs_wave_reduce(v, [](double a, double b) { return a + b; }); }
+__device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) { return zs_wave_reduce(v, [](uint32_t a, uint32_t b) { return a + b; }); }
+__device__ __forceinline__ int wave_min_i(int v) { return zs_wave_reduce(v, [](int a, int b) { return min(a, b); }); }
+__device__ __forceinline__ int wave_max_i(int v) { return zs_wave_reduce(v, [](int a, int b) { return max(a, b); }); }
+__device__ __forceinline__ uint32_t wave_or_u(uint32_t v) { return zs_wave_reduce(v, [](uint32_t a, uint32_t b) { return a | b; }); }
 // Inclusive scan (plain add) over the wave.
 __device__ __forceinline__ uint32_t wave_incl_scan_u(uint32_t x) {
     int lane = zs_lane();
@@ -189,7 +237,7 @@ __device__ __forceinline__ uint32_t wave_sort_u32(uint32_t v) {
     for (int k = 2; k <= 64; k <<= 1) {
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1) {
-            uint32_t o = __shfl_xor(v, j, 64);
+            const uint32_t o = zs_lane_xor_by(v, (uint32_t)j);   // (constant once unrolled)
             bool keep_min = ((lane & j) == 0) == ((lane & k) == 0 || k == 64);
             v = keep_min ? min(v, o) : max(v, o);
         }
@@ -202,7 +250,7 @@ __device__ __forceinline__ unsigned long long wave_sort_u64(unsigned long long v
     for (int k = 2; k <= 64; k <<= 1) {
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1) {
-            unsigned long long o = __shfl_xor(v, j, 64);
+            const unsigned long long o = zs_lane_xor_by(v, (uint32_t)j);
             bool keep_min = ((lane & j) == 0) == ((lane & k) == 0 || k == 64);
             v = keep_min ? (o < v ? o : v) : (o > v ? o : v);
         }
@@ -255,6 +303,8 @@ __device__ void block_sort_reg_u64(unsigned long long* a, uint32_t n) {
             } else {
                 unsigned long long o[E];
                 if (j < 64u * E) {
+                    // (a runtime stride: a branch per stride to the moves of
+                    // zs_lane_xor was slower than the shuffle)
 #pragma unroll
                     for (int e = 0; e < E; e++) o[e] = __shfl_xor(v[e], (int)(j / E), 64);
                 } else {

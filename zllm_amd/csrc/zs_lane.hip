@@ -34,10 +34,7 @@ __device__ __forceinline__ uint32_t wg_key_idx(unsigned long long k) {
 }
 
 __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v, unsigned long long* sh) {
-    for (int d = 32; d > 0; d >>= 1) {
-        unsigned long long o = __shfl_xor(v, d, 64);
-        v = o > v ? o : v;
-    }
+    v = zs_wave_reduce(v, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
     if (zs_lane() == 0) sh[zs_wid()] = v;
     __syncthreads();
     unsigned long long r = 0;
@@ -234,7 +231,7 @@ __global__ __launch_bounds__(BS_NT) void zs_k_bsample(const float* logits, uint3
         }
         const bool near = bb > -INFINITY && ba - bb <= 2.0f * zs_gumbel_band(fmaxf(fabsf(ba), fabsf(bb)));
         float m = ba;
-        for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+        m = wave_max_f(m);
         if (zs_lane() == 0) shf[zs_wid()] = m;
         __syncthreads();
         m = -INFINITY;
@@ -246,10 +243,7 @@ __global__ __launch_bounds__(BS_NT) void zs_k_bsample(const float* logits, uint3
             else best = wg_key(zs_gumbel_exact(bx, inv_t, sd, bi), bi);
         }
     }
-    for (int d = 32; d > 0; d >>= 1) {
-        const unsigned long long o = __shfl_xor(best, d, 64);
-        best = o > best ? o : best;
-    }
+    best = zs_wave_reduce(best, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
     if (zs_lane() == 0) shk[zs_wid()] = best;
     __syncthreads();
     if (threadIdx.x == 0) {

@@ -553,10 +553,8 @@ __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, u
             hi = max(hi, (uint32_t)(v[e] >> 32));
         }
     }
-    for (int d = 32; d > 0; d >>= 1) {
-        lo = min(lo, (uint32_t)__shfl_xor(lo, d, 64));
-        hi = max(hi, (uint32_t)__shfl_xor(hi, d, 64));
-    }
+    lo = zs_wave_reduce(lo, [](uint32_t x, uint32_t y) { return min(x, y); });
+    hi = zs_wave_reduce(hi, [](uint32_t x, uint32_t y) { return max(x, y); });
     if (lane == 0) { sh.sel_mm[0][wid] = c; sh.sel_mm[1][wid] = lo; sh.sel_mm[2][wid] = hi; }
     __syncthreads();
     c = 0; lo = 0xffffffffu; hi = 0;
@@ -1805,15 +1803,12 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     RW_T(2);
     // ---- row statistics (one workgroup reduction)
     {
-        for (int d = 32; d > 0; d >>= 1) {
-            omax = fmaxf(omax, __shfl_xor(omax, d, 64));
-            ymax = fmaxf(ymax, __shfl_xor(ymax, d, 64));
-            fl |= __shfl_xor(fl, d, 64);
-            last_nan = max(last_nan, __shfl_xor(last_nan, d, 64));
-            rejf = fmaxf(rejf, __shfl_xor(rejf, d, 64));
-            const unsigned long long og = __shfl_xor(gbest, d, 64);
-            gbest = og > gbest ? og : gbest;
-        }
+        omax = wave_max_f(omax);
+        ymax = wave_max_f(ymax);
+        fl = wave_or_u(fl);
+        last_nan = wave_max_i(last_nan);
+        rejf = wave_max_f(rejf);
+        gbest = zs_wave_reduce(gbest, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
         if (zs_lane() == 0) {
             sh.rf[0][zs_wid()] = omax; sh.rf[1][zs_wid()] = ymax;
             sh.ru[0][zs_wid()] = fl; sh.rf[2][zs_wid()] = rejf;
@@ -1881,10 +1876,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
                 }
                 return false;
             });
-            for (int d = 32; d > 0; d >>= 1) {
-                const unsigned long long o = __shfl_xor(gb, d, 64);
-                gb = o > gb ? o : gb;
-            }
+            gb = zs_wave_reduce(gb, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
             if (zs_lane() == 0) sh.rl[zs_wid()] = gb;
             __syncthreads();
             gb = 0;

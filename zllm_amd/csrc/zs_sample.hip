@@ -1990,7 +1990,7 @@ __global__ __launch_bounds__(64) void zs_k_final(zs_sargs a) {
                 const unsigned long long at = __ballot(mine && rank == n - 1);
                 lpn = zs_readlane_f(lp, (uint32_t)__ffsll((long long)at) - 1u);
                 float lmin = mine ? lp : INFINITY;
-                for (int d = 32; d > 0; d >>= 1) lmin = fminf(lmin, __shfl_xor(lmin, d, 64));
+                lmin = zs_wave_reduce(lmin, [](float x, float y) { return fminf(x, y); });
                 fill = lpn > -INFINITY && lmin == lpn;
             }
             if (!fill) {

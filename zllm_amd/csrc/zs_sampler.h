@@ -91,7 +91,7 @@ __device__ __forceinline__ void wave_sort_u64_e(unsigned long long (&v)[E]) {
             } else {
 #pragma unroll
                 for (uint32_t e = 0; e < (uint32_t)E; e++) {
-                    const unsigned long long o = __shfl_xor(v[e], (int)(j / E), 64);
+                    const unsigned long long o = zs_lane_xor_by(v[e], j / E);
                     const uint32_t i = lane * E + e;
                     const bool asc = (i & k) == 0u, lower = (i & j) == 0u;
                     v[e] = (lower == asc) ? (o < v[e] ? o : v[e]) : (o > v[e] ? o : v[e]);

@@ -343,8 +343,7 @@ __device__ __forceinline__ void sm_incs(const sm_terms& f, const float (&a)[SM_E
 }
 
 __device__ __forceinline__ float sm_wave_sum_f(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+    v = zs_wave_reduce(v, [](float x, float y) { return x + y; });
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v)));
 }
 
