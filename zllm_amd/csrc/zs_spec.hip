@@ -117,10 +117,7 @@ __global__ __launch_bounds__(SP_NT) void zs_k_spec_chunk(zs_spec_args a) {
         : ((unsigned long long)zs_total_key(bv == 0.0f ? 0.0f : bv) << 32) | (0xffffffffu - sp_id(base, be));
     const float xmax = block_max_f<SP_NT>(bv, fsh);
     fl = block_or_u<SP_NT>(fl, ush);
-    for (int d = 32; d > 0; d >>= 1) {
-        unsigned long long o = __shfl_xor(best, d, 64);
-        best = o > best ? o : best;
-    }
+    best = zs_wave_reduce(best, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
     // chunk sum of the weights relative to the chunk maximum (at most 32
     // weights below 2^25 each per thread)
     const float T = a.temperature[r];
@@ -131,7 +128,7 @@ __global__ __launch_bounds__(SP_NT) void zs_k_spec_chunk(zs_spec_args a) {
 #pragma unroll
         for (int e = 0; e < SP_EPT; e++) s32 += sp_weight(x[e], xmax, cT);
         wsum = s32;
-        for (int d = 32; d > 0; d >>= 1) wsum += __shfl_xor(wsum, d, 64);
+        wsum = zs_wave_reduce(wsum, [](unsigned long long x, unsigned long long y) { return x + y; });
     }
     if (zs_lane() == 0) { gsh[zs_wid()] = best; wsh[zs_wid()] = wsum; }
     __syncthreads();
@@ -214,10 +211,7 @@ __global__ __launch_bounds__(SR_NT) void zs_k_spec_row(zs_spec_args a) {
                 : ((unsigned long long)zs_total_key(bv == 0.0f ? 0.0f : bv) << 32) | (0xffffffffu - sr_id(base, be));
             const float xmax = wave_max_f(bv);
             fl = wave_or_u(fl);
-            for (int d = 32; d > 0; d >>= 1) {
-                unsigned long long o = __shfl_xor(best, d, 64);
-                best = o > best ? o : best;
-            }
+            best = zs_wave_reduce(best, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
             if (lane == 0) { wz[h][wid] = xmax; wf[c][wid] = fl; wb[c][wid] = best; }
         }
         __syncthreads();
@@ -235,7 +229,7 @@ __global__ __launch_bounds__(SR_NT) void zs_k_spec_row(zs_spec_args a) {
 #pragma unroll
                 for (int e = 0; e < SR_EPT; e++) s32 += sp_weight(x[h][e], m, cT);
                 s = s32;
-                for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+                s = zs_wave_reduce(s, [](unsigned long long x, unsigned long long y) { return x + y; });
             }
             if (lane == 0) ws[c][wid] = s;
         }
@@ -265,122 +259,7 @@ __device__ __forceinline__ int sp_bitlen(u128 v) {
     const unsigned long long hi = (unsigned long long)(v >> 64), lo = (unsigned long long)v;
     return hi ? 128 - __clzll((long long)hi) : (lo ? 64 - __clzll((long long)lo) : 0);
 }
-// sum of a row's weights, sum_c F_c * S_c, by one wave (lanes over chunks);
-// every lane gets it
-__device__ __forceinline__ u128 sp_row_sum(const zs_spec_chunk* cs, uint32_t nch, float M, float cT) {
-    u128 s = 0;
-    for (uint32_t c = (uint32_t)zs_lane(); c < nch; c += 64)
-        s += (u128)((unsigned long long)sp_weight(cs[c].xmax, M, cT) * cs[c].wsum);
-    for (int d = 32; d > 0; d >>= 1) {
-        const unsigned long long lo = __shfl_xor((unsigned long long)s, d, 64);
-        const unsigned long long hi = __shfl_xor((unsigned long long)(s >> 64), d, 64);
-        s += ((u128)hi << 64) | lo;
-    }
-    return s;
-}
-
-// pass 2: one wave per row -- accept / reject decisions (lanes over chunks)
-// and the sums of the final draw
-__global__ __launch_bounds__(64) void zs_k_spec_decide(zs_spec_args a) {
-    const uint32_t r = blockIdx.x;
-    const int lane = zs_lane();
-    const uint32_t k = a.k, V = a.V;
-    const uint32_t nch = (V + SP_CH - 1) / SP_CH;
-    const uint32_t npos = a.draft ? 2 * k + 1 : k + 1;
-    const float T = a.temperature[r];
-    zs_spec_row out;
-    out.m_t = out.m_d = 0.f;
-    out.ps = out.qs = 0;
-    out.sum_lo = out.sum_hi = 0;
-    bool degenerate = !(T > 0.0f) || !a.draft;
-    float mpos[2 * ZS_SPEC_KMAX + 1];
-    uint32_t apos[ZS_SPEC_KMAX + 1];
-    auto cst = [&](uint32_t p) { return a.cst + ((size_t)r * a.npos_max + p) * a.nch; };
-    for (uint32_t p = 0; p < npos; p++) {
-        const zs_spec_chunk* cs = cst(p);
-        float m = -INFINITY;
-        uint32_t fl = 0;
-        unsigned long long best = 0;  // (value key, ~id) of the first maximum
-        for (uint32_t c = lane; c < nch; c += 64) {
-            const zs_spec_chunk q = cs[c];
-            m = fmaxf(m, q.xmax);
-            fl |= q.flags;
-            if (q.amax_idx != 0xffffffffu) {
-                const unsigned long long key = ((unsigned long long)zs_total_key(q.amax_val) << 32) | (0xffffffffu - q.amax_idx);
-                best = key > best ? key : best;
-            }
-        }
-        m = wave_max_f(m);
-        fl = wave_or_u(fl);
-        for (int d = 32; d > 0; d >>= 1) {
-            unsigned long long o = __shfl_xor(best, d, 64);
-            best = o > best ? o : best;
-        }
-        if (fl || m == -INFINITY) degenerate = true;
-        if (p <= k) apos[p] = best ? 0xffffffffu - (uint32_t)(best & 0xffffffffull) : 0u;
-        mpos[p] = m;
-    }
-    const uint32_t* drafts = a.draft_ids + (size_t)r * k;
-    if (degenerate) {
-        if (lane != 0) return;
-        uint32_t acc = 0, bonus = apos[k];
-        for (uint32_t i = 0; i < k; i++) {
-            if (apos[i] == drafts[i]) acc++;
-            else { bonus = apos[i]; break; }
-        }
-        a.accepted[r] = acc;
-        a.next[r] = bonus;
-        out.mode = 0;
-        a.rs[r] = out;
-        return;
-    }
-    const float cT = sp_c(T);
-    // P_d = w_d * F_c of the chunk holding d
-    auto weight_at = [&](uint32_t p, uint32_t d) -> unsigned long long {
-        const float mc = cst(p)[d / SP_CH].xmax;
-        return (unsigned long long)sp_weight(sp_row(a, r, p)[d], mc, cT) * sp_weight(mc, mpos[p], cT);
-    };
-    uint32_t i = 0;
-    u128 sp = 0, sq = 0;
-    int sh = 0;
-    for (; i < k; i++) {
-        sp = sp_row_sum(cst(i), nch, mpos[i], cT);
-        sq = sp_row_sum(cst(k + 1 + i), nch, mpos[k + 1 + i], cT);
-        sh = max(0, sp_bitlen(sp | sq) - 40);
-        const uint32_t d = drafts[i];
-        if (d >= V) break;
-        const unsigned long long Ps = (unsigned long long)(sp >> sh), Qs = (unsigned long long)(sq >> sh);
-        const unsigned long long P = weight_at(i, d), Q = weight_at(k + 1 + i, d);
-        const uint32_t U = zs_philox_u32(a.seed[r], a.counter[r], 1u + i);
-        const u128 lhs = ((u128)U * Q) * Ps;  // < 2^122
-        const u128 rhs = ((u128)P * Qs) << 32;                      // < 2^122
-        if (!(lhs <= rhs)) break;
-    }
-    out.mode = 1;
-    out.pos = i;
-    if (i == k) {
-        const u128 st = sp_row_sum(cst(k), nch, mpos[k], cT);
-        out.residual = 0;
-        out.m_t = mpos[k];
-        out.sum_lo = (unsigned long long)st;
-        out.sum_hi = (unsigned long long)(st >> 64);
-        out.word = zs_philox_u32(a.seed[r], a.counter[r], 1u + 2 * k);
-    } else {
-        out.residual = 1;
-        out.m_t = mpos[i];
-        out.m_d = mpos[k + 1 + i];
-        out.ps = (unsigned long long)(sp >> sh);
-        out.qs = (unsigned long long)(sq >> sh);
-        out.sum_lo = (unsigned long long)sp;  // the target's sum: the draw when R is all 0
-        out.sum_hi = (unsigned long long)(sp >> 64);
-        out.word = zs_philox_u32(a.seed[r], a.counter[r], 1u + k + i);
-    }
-    if (lane != 0) return;
-    a.accepted[r] = i;
-    a.rs[r] = out;
-}
-
-// u128 helpers for the workgroup scan
+// u128 helpers
 struct u128p { unsigned long long lo, hi; };
 __device__ __forceinline__ u128 u128_of(u128p v) { return ((u128)v.hi << 64) | v.lo; }
 __device__ __forceinline__ u128p u128p_of(u128 v) { return {(unsigned long long)v, (unsigned long long)(v >> 64)}; }
@@ -390,11 +269,163 @@ __device__ __forceinline__ u128 shfl_up_u128(u128 v, int d) {
     p.hi = __shfl_up(p.hi, d, 64);
     return u128_of(p);
 }
-__device__ __forceinline__ u128 shfl_xor_u128(u128 v, int d) {
+template <int J>
+__device__ __forceinline__ u128 xor_add_u128(u128 v) {
     u128p p = u128p_of(v);
-    p.lo = __shfl_xor(p.lo, d, 64);
-    p.hi = __shfl_xor(p.hi, d, 64);
-    return u128_of(p);
+    p.lo = zs_lane_xor<J>(p.lo);
+    p.hi = zs_lane_xor<J>(p.hi);
+    return v + u128_of(p);
+}
+__device__ __forceinline__ u128 wave_sum_u128(u128 v) {
+    return xor_add_u128<1>(xor_add_u128<2>(xor_add_u128<4>(xor_add_u128<8>(xor_add_u128<16>(xor_add_u128<32>(v))))));
+}
+
+// pass 2: accept / reject decisions of a row and the sums of its draw, by an
+// SP_NT-thread workgroup: the waves take the positions in turn (maximum, first
+// argmax, weight sum and the draft id's weight of a position in one visit to
+// its chunk records), then one lane per draft makes its accept test and the
+// first rejection decides. Every workgroup of zs_k_spec_rsum makes it for
+// itself (one wave per row visiting the positions one after the other, and the
+// drafts' tests one after the other, took a launch of 18 us on 64 rows of 9
+// positions; the residual pass with it in front takes 5 us more than without).
+#define SP_NPOS (2 * ZS_SPEC_KMAX + 1)
+struct sp_decision {
+    zs_spec_row row;
+    uint32_t accepted, next;   // next: greedy rows (row.mode 0) only
+    unsigned long long slo[SP_NPOS], shi[SP_NPOS];   // weight sums
+    unsigned long long wt[SP_NPOS];                  // weight of the draft id at its target / draft position
+    float m[SP_NPOS];
+    uint32_t am[SP_NPOS], fl[SP_NPOS];
+};
+__device__ __forceinline__ void sp_decide(const zs_spec_args& a, uint32_t r, sp_decision& S) {
+    const uint32_t k = a.k, V = a.V, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    const uint32_t nch = (V + SP_CH - 1) / SP_CH;
+    const uint32_t npos = a.draft ? 2 * k + 1 : k + 1;
+    const float T = a.temperature[r];
+    const bool weights = T > 0.0f && a.draft;
+    const float cT = weights ? sp_c(T) : 0.0f;
+    const uint32_t* drafts = a.draft_ids + (size_t)r * k;
+    constexpr uint32_t PU = 3;   // positions of a wave with their first loads in flight
+    for (uint32_t p0 = wid; p0 < npos; p0 += PU * (SP_NT / 64)) {
+        zs_spec_chunk q[PU];
+        uint32_t d[PU];
+        float xd[PU], xm[PU];   // the draft id's logit and its chunk's maximum
+#pragma unroll
+        for (uint32_t u = 0; u < PU; u++) {
+            const uint32_t p = p0 + u * (SP_NT / 64);
+            q[u].xmax = -INFINITY; q[u].flags = 0; q[u].amax_val = -INFINITY; q[u].amax_idx = 0xffffffffu; q[u].wsum = 0;
+            d[u] = 0xffffffffu;
+            if (p >= npos) continue;
+            if (lane < nch) q[u] = a.cst[((size_t)r * a.npos_max + p) * a.nch + lane];
+            if (weights && p != k) d[u] = drafts[p < k ? p : p - k - 1];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < PU; u++) {
+            const uint32_t p = p0 + u * (SP_NT / 64);
+            xd[u] = xm[u] = 0.0f;
+            if (p < npos && d[u] < V) {
+                xd[u] = sp_row(a, r, p)[d[u]];
+                xm[u] = a.cst[((size_t)r * a.npos_max + p) * a.nch + d[u] / SP_CH].xmax;
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < PU; u++) {
+            const uint32_t p = p0 + u * (SP_NT / 64);
+            if (p >= npos) continue;
+            const zs_spec_chunk* cs = a.cst + ((size_t)r * a.npos_max + p) * a.nch;
+            auto key = [](const zs_spec_chunk& c) -> unsigned long long {   // (value key, ~id) of the first maximum
+                return c.amax_idx == 0xffffffffu ? 0ull : ((unsigned long long)zs_total_key(c.amax_val) << 32) | (0xffffffffu - c.amax_idx);
+            };
+            float m = q[u].xmax;
+            uint32_t fl = q[u].flags;
+            unsigned long long best = key(q[u]);
+            for (uint32_t c = lane + 64; c < nch; c += 64) {
+                const zs_spec_chunk w = cs[c];
+                m = fmaxf(m, w.xmax);
+                fl |= w.flags;
+                const unsigned long long kw = key(w);
+                best = kw > best ? kw : best;
+            }
+            m = wave_max_f(m);
+            fl = wave_or_u(fl);
+            best = zs_wave_reduce(best, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
+            u128 s = 0;
+            unsigned long long wt = 0;
+            if (weights && !fl && m > -INFINITY) {
+                // sum_c F_c * S_c, and P_d = w_d * F_c of the chunk holding d
+                if (lane < nch) s = (u128)((unsigned long long)sp_weight(q[u].xmax, m, cT) * q[u].wsum);
+                for (uint32_t c = lane + 64; c < nch; c += 64) s += (u128)((unsigned long long)sp_weight(cs[c].xmax, m, cT) * cs[c].wsum);
+                s = wave_sum_u128(s);
+                if (d[u] < V) wt = (unsigned long long)sp_weight(xd[u], xm[u], cT) * sp_weight(xm[u], m, cT);
+            }
+            if (lane == 0) {
+                S.m[p] = m;
+                S.fl[p] = (fl || m == -INFINITY) ? 1u : 0u;
+                S.am[p] = best ? 0xffffffffu - (uint32_t)best : 0u;
+                S.slo[p] = (unsigned long long)s;
+                S.shi[p] = (unsigned long long)(s >> 64);
+                S.wt[p] = wt;
+            }
+        }
+    }
+    __syncthreads();
+    if (wid == 0) {
+        bool bad = !weights;
+        for (uint32_t p = lane; p < npos; p += 64) bad |= S.fl[p] != 0u;
+        const bool degenerate = __ballot(bad) != 0ull;
+        const uint32_t dr = lane < k ? drafts[lane] : 0u;
+        // lane i: whether draft i is turned away
+        bool rej = false;
+        u128 sp = 0, sq = 0;
+        int sh = 0;
+        if (lane < k) {
+            if (degenerate) {
+                rej = S.am[lane] != dr;
+            } else {
+                sp = ((u128)S.shi[lane] << 64) | S.slo[lane];
+                sq = ((u128)S.shi[k + 1 + lane] << 64) | S.slo[k + 1 + lane];
+                sh = max(0, sp_bitlen(sp | sq) - 40);
+                const unsigned long long Ps = (unsigned long long)(sp >> sh), Qs = (unsigned long long)(sq >> sh);
+                const uint32_t U = zs_philox_u32(a.seed[r], a.counter[r], 1u + lane);
+                const u128 lhs = ((u128)U * S.wt[k + 1 + lane]) * Ps;  // < 2^122
+                const u128 rhs = ((u128)S.wt[lane] * Qs) << 32;       // < 2^122
+                rej = dr >= V || !(lhs <= rhs);
+            }
+        }
+        const unsigned long long rm = __ballot(rej);
+        const uint32_t i = rm ? (uint32_t)__ffsll((long long)rm) - 1u : k;
+        if (degenerate) {
+            if (lane == 0) {
+                S.accepted = i;
+                S.next = S.am[i];
+                S.row.mode = 0;
+            }
+        } else if (lane == (i < k ? i : 0u)) {
+            zs_spec_row o;
+            o.mode = 1;
+            o.pos = i;
+            o.m_t = S.m[i];
+            o.m_d = 0.f;
+            o.ps = o.qs = 0;
+            if (i == k) {
+                o.residual = 0;
+                o.sum_lo = S.slo[k];
+                o.sum_hi = S.shi[k];
+                o.word = zs_philox_u32(a.seed[r], a.counter[r], 1u + 2 * k);
+            } else {
+                o.residual = 1;
+                o.m_d = S.m[k + 1 + i];
+                o.ps = (unsigned long long)(sp >> sh);
+                o.qs = (unsigned long long)(sq >> sh);
+                o.sum_lo = S.slo[i];  // the target's sum: the draw when R is all 0
+                o.sum_hi = S.shi[i];
+                o.word = zs_philox_u32(a.seed[r], a.counter[r], 1u + k + i);
+            }
+            S.accepted = i;
+            S.row = o;
+        }
+    }
+    __syncthreads();
 }
 
 // Draw weight of id v (given its target / draft logits and its chunk's maxima
@@ -426,12 +457,21 @@ __device__ __forceinline__ u128 spd_weight2(const zs_spec_row& s, const sp_chunk
     return pp > qq ? pp - qq : 0;
 }
 
-// pass 3: chunk sums of the residual weights (rows that rejected a draft)
+// pass 3: the decision, and chunk sums of the residual weights (rows that
+// rejected a draft). Chunk 0's workgroup stores the decision; without draft
+// logits every row is verified greedily and it is the only one launched.
 __global__ __launch_bounds__(SP_NT) void zs_k_spec_rsum(zs_spec_args a) {
     const uint32_t c = blockIdx.x, r = blockIdx.y;
     const uint32_t base = c * SP_CH;
     if (base >= a.V) return;
-    const zs_spec_row s = a.rs[r];
+    __shared__ sp_decision S;
+    sp_decide(a, r, S);
+    const zs_spec_row s = S.row;
+    if (c == 0 && threadIdx.x == 0) {
+        a.accepted[r] = S.accepted;
+        if (s.mode == 0) a.next[r] = S.next;
+        a.rs[r] = s;
+    }
     if (s.mode != 1 || !s.residual) return;
     __shared__ unsigned long long lo[SP_NT / 64], hi[SP_NT / 64];
     const float cT = sp_c(a.temperature[r]);
@@ -443,7 +483,7 @@ __global__ __launch_bounds__(SP_NT) void zs_k_spec_rsum(zs_spec_args a) {
 #pragma unroll
     for (int e = 0; e < SP_EPT; e++)
         acc += spd_weight2(s, cw, cT, xt[e], xd[e]);
-    for (int d = 32; d > 0; d >>= 1) acc += shfl_xor_u128(acc, d);
+    acc = wave_sum_u128(acc);
     if (zs_lane() == 0) { lo[zs_wid()] = (unsigned long long)acc; hi[zs_wid()] = (unsigned long long)(acc >> 64); }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -477,7 +517,7 @@ __global__ __launch_bounds__(SP_BIG_NT) void zs_k_spec_draw(zs_spec_args a) {
         u128 rt = 0;
         if (s.residual)
             for (uint32_t c = t; c < nch; c += 64) rt += ((u128)c0[c].rhi << 64) | c0[c].rlo;
-        for (int d = 32; d > 0; d >>= 1) rt += shfl_xor_u128(rt, d);
+        rt = wave_sum_u128(rt);
         const bool resid = s.residual && rt != 0;
         const u128 total = resid ? rt : (((u128)s.sum_hi << 64) | s.sum_lo);
         // floor(word * total / 2^32) without overflow: total < 2^108
@@ -589,9 +629,8 @@ extern "C" int zs_spec_launch(const zs_spec_args& a, const zs_prof& prof, hipStr
     hipLaunchKernelGGL(zs_k_spec_chunk, grid, dim3(SP_NT), 0, stream, a);
     mark("zs_k_spec_chunk");
     }
-    hipLaunchKernelGGL(zs_k_spec_decide, dim3(a.B), dim3(64), 0, stream, a);
-    hipLaunchKernelGGL(zs_k_spec_rsum, dim3(nch, a.B), dim3(SP_NT), 0, stream, a);
-    hipLaunchKernelGGL(zs_k_spec_draw, dim3(a.B), dim3(SP_BIG_NT), 0, stream, a);
+    hipLaunchKernelGGL(zs_k_spec_rsum, dim3(a.draft ? nch : 1, a.B), dim3(SP_NT), 0, stream, a);
+    if (a.draft) hipLaunchKernelGGL(zs_k_spec_draw, dim3(a.B), dim3(SP_BIG_NT), 0, stream, a);
     mark("zs_k_spec_draw");
     if (prof.on) *prof.n = ev - 1;
     return hipGetLastError() == hipSuccess ? 0 : -1;
