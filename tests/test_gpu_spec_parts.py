@@ -1,0 +1,35 @@
+"""A verification of more workgroups than one launch takes: every row against
+the oracle, the last launch's rows and a last launch that is not full included."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from zllm_amd.engine import Context, verify_drafts
+
+pytestmark = pytest.mark.gpu
+
+
+# 33 positions of one chunk a row (24576 workgroups a launch: 744 rows of one): one full launch, two, three
+@pytest.mark.parametrize("B", [744, 745, 1500])
+def test_rows_of_every_launch(B):
+    print(f"[case] spec parts B={B}", flush=True)
+    k, V, ld = 16, 37, 40
+    rng = np.random.default_rng(B)
+    target = rng.normal(0, 2.0, (B, k + 1, ld)).astype(np.float32)
+    draft = (target[:, :k] + rng.normal(0, 0.3, (B, k, ld))).astype(np.float32)
+    ids = rng.integers(0, V, (B, k)).astype(np.uint32)
+    sure = rng.random((B, k)) < 0.9
+    ids = np.where(sure, np.argmax(draft[:, :, :V], axis=2), ids).astype(np.uint32)
+    temp = np.where(np.arange(B) % 3 == 0, 0.0, 0.8).astype(np.float32)
+    seeds = np.arange(B, dtype=np.uint64) + 5
+    ctr = np.full(B, 2, np.uint64)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    c = Context(max_rows=B, max_vocab=64)
+    acc, nxt = verify_drafts(c, t(target)[:, :, :V], t(ids.view(np.int32)), t(temp), t(seeds.view(np.int64)),
+                             t(ctr.view(np.int64)), t(draft)[:, :, :V])
+    acc, nxt = acc.cpu().numpy(), nxt.cpu().numpy().view(np.uint32)
+    c.close()
+    for b in range(B):
+        want = O.spec_verify(target[b, :, :V], draft[b, :, :V], ids[b].tolist(), float(temp[b]), int(seeds[b]), int(ctr[b]))
+        assert (int(acc[b]), int(nxt[b])) == want, (b, (acc[b], nxt[b]), want)

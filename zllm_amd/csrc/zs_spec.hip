@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 #include "zs_internal.h"
 #include "zs_dev.h"
+#include <algorithm>
 #include <mutex>
 
 #define SP_NT 256
@@ -66,13 +67,19 @@ __device__ __forceinline__ uint32_t sp_weight(float x, float m, float c) {
 __device__ __forceinline__ bool sp_live(float xc, float m, float c) {
     return __fmul_rn(__fsub_rn(xc, m), c) >= SP_ZERO_T;
 }
-// the chunk's elements of thread t: float4 j covers ids base + (j*SP_NT + t)*4 .. +3
+// the chunk's elements of thread t: float4 j covers ids base + (j*SP_NT + t)*4
+// .. +3. Non-temporal: a verification reads each of its rows once (the residual
+// pass one pair a row again), and its gigabytes would push the sampler's rows,
+// which the kernels beside it read several times, out of the caches (256 rows
+// of 9 positions of 151936 ids beside the sampler: 697 -> 682 us; alone, 64
+// rows of 128256, 88 us either way).
+typedef float sp_f4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void sp_load(const float* row, uint32_t base, uint32_t V, float (&x)[SP_EPT]) {
 #pragma unroll
     for (int j = 0; j < SP_EPT / 4; j++) {
         const uint32_t id = base + (j * SP_NT + threadIdx.x) * 4;
-        float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        if (id < V) v = *reinterpret_cast<const float4*>(row + id);
+        sp_f4 v = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        if (id < V) v = __builtin_nontemporal_load(reinterpret_cast<const sp_f4*>(row + id));
         x[4 * j] = v.x; x[4 * j + 1] = v.y; x[4 * j + 2] = v.z; x[4 * j + 3] = v.w;
     }
     if (base + SP_CH > V) {  // ids past V read as -inf (neutral in every pass)
@@ -87,9 +94,19 @@ __device__ __forceinline__ uint32_t sp_id(uint32_t base, int e) {
 
 // One pass per chunk: the chunk maximum, flags, the first strict maximum of x
 // (greedy verification) and, once the chunk maximum is known, the chunk sum of
-// the weights w_v = W((x_v - m_c) c).
-__global__ __launch_bounds__(SP_NT) void zs_k_spec_chunk(zs_spec_args a) {
-    const uint32_t c = blockIdx.x, pos = blockIdx.y, r = blockIdx.z;
+// the weights w_v = W((x_v - m_c) c). The rows from r0 on.
+//
+// Bound by HBM. A workgroup is small and needs few registers, so a launch of
+// many holds every slot that one of its own gives up, and a kernel beside it on
+// another stream that needs much of a CU (zs_k_row: 168 registers of 8 waves
+// and 149 KB of LDS at 151936 ids) waits for its end: 190 us instead of 47 beside
+// 43776 workgroups. So the rows go in equal launches of at most SP_PART
+// workgroups: between two of them the CUs come free. Full step of 256 rows (9
+// positions of 151936 ids beside the sampler): one launch 677 us, two 638, three
+// 645, five 651, ten 658; alone each further launch adds about 8 us.
+#define SP_PART 24576u
+__global__ __launch_bounds__(SP_NT) void zs_k_spec_chunk(zs_spec_args a, uint32_t r0) {
+    const uint32_t c = blockIdx.x, pos = blockIdx.y, r = r0 + blockIdx.z;
     const uint32_t npos = a.draft ? 2 * a.k + 1 : a.k + 1;
     if (pos >= npos) return;
     const uint32_t base = c * SP_CH;
@@ -620,14 +637,16 @@ extern "C" int zs_spec_launch(const zs_spec_args& a, const zs_prof& prof, hipStr
         (void)hipEventRecord((hipEvent_t)prof.events[ev], stream);
         ev++;
     };
-    dim3 grid(nch, npos, a.B);
     mark(nullptr);
     if (a.background) {
         hipLaunchKernelGGL(zs_k_spec_row, dim3(npos, a.B), dim3(SR_NT), SR_LDS_HOLD, stream, a);
         mark("zs_k_spec_row");
     } else {
-    hipLaunchKernelGGL(zs_k_spec_chunk, grid, dim3(SP_NT), 0, stream, a);
-    mark("zs_k_spec_chunk");
+        const uint64_t parts = ((uint64_t)nch * npos * a.B + SP_PART - 1) / SP_PART;
+        const uint32_t per = (uint32_t)((a.B + parts - 1) / parts);
+        for (uint32_t r0 = 0; r0 < a.B; r0 += per)
+            hipLaunchKernelGGL(zs_k_spec_chunk, dim3(nch, npos, std::min(per, a.B - r0)), dim3(SP_NT), 0, stream, a, r0);
+        mark("zs_k_spec_chunk");
     }
     hipLaunchKernelGGL(zs_k_spec_rsum, dim3(a.draft ? nch : 1, a.B), dim3(SP_NT), 0, stream, a);
     if (a.draft) hipLaunchKernelGGL(zs_k_spec_draw, dim3(a.B), dim3(SP_BIG_NT), 0, stream, a);
