@@ -150,6 +150,9 @@ extern "C" int zs_ctx_create(int device, uint32_t max_rows, uint32_t max_vocab, 
     ctx->max_vocab = max_vocab;
     ctx->max_chunks = (max_vocab + ZS_P1_CH - 1) / ZS_P1_CH;
     ctx->max_subs = ctx->max_chunks * ZS_SUBS_PER_CHUNK;
+    // the scratch rows' stride: 16-byte stores at a row's end stay in the row
+    max_vocab = (max_vocab + 3u) & ~3u;
+    ctx->row_stride = max_vocab;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || device < 0 || device >= ndev) {
         free(ctx);

@@ -160,6 +160,7 @@ struct zs_ctx {
     int device;
     uint32_t num_cus;
     uint32_t max_rows, max_vocab, max_chunks;
+    uint32_t row_stride;   // entries of a scratch row: max_vocab rounded up to 4 (the areas below, where they say max_vocab)
     char err[512];
     // device scratch
     uint32_t* p_cnt;

@@ -2071,7 +2071,7 @@ extern "C" int zs_sample_launch(zs_ctx* ctx, const zs_batch* bt, hipStream_t str
     a.rst = ctx->rst;
     a.pairs = ctx->pairs;
     a.nch = ctx->max_chunks;
-    a.max_vocab = ctx->max_vocab;
+    a.max_vocab = ctx->row_stride;
     a.pv = ctx->pv;
     a.p_sub = ctx->p_sub;
     a.max_subs = ctx->max_subs;
@@ -2091,7 +2091,7 @@ extern "C" int zs_sample_launch(zs_ctx* ctx, const zs_batch* bt, hipStream_t str
     a.s_xrec = ctx->s_rec + (size_t)ctx->max_rows * ZS_NSUM * ctx->max_subs;
     a.s_apx = ctx->s_apx;
     a.gath = ctx->gath;
-    a.pstride = ctx->max_vocab;
+    a.pstride = ctx->row_stride;
     a.s_hterm = ctx->s_hterm;
     const uint32_t B = bt->B;
     const bool prof = ctx->profiling != 0;

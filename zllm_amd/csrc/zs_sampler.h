@@ -17,7 +17,7 @@ struct zs_sargs {
     uint32_t* pairs;
     uint32_t* pv;
     uint32_t nch;
-    uint32_t max_vocab;
+    uint32_t max_vocab;   // stride of the scratch rows: the context's max_vocab rounded up to 4
     uint32_t* p_sub;
     uint32_t max_subs;
     double* k_ap;
@@ -33,7 +33,7 @@ struct zs_sargs {
     float* s_apx;
     float* gath;
     float* s_hterm;
-    uint32_t pstride;   // entries per row of the merged patch list (p_id, p_flags, p_y): max_vocab
+    uint32_t pstride;   // entries per row of the merged patch list (p_id, p_flags, p_y): the same stride
     uint32_t gshift;    // zs_k_scan: log2 of the ids per group (0: no scan)
     uint32_t ncu;       // CUs of the device
     uint32_t gstride;   // groups per row of gmax
