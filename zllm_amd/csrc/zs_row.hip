@@ -1152,6 +1152,9 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         kmo = max(kmo, sh.ru[3][w]); kms = max(kms, sh.ru[4][w]);
     }
     to = rw_uni(to); ts = rw_uni(ts); nfin = rw_uni(nfin); kmo = rw_uni(kmo); kms = rw_uni(kms);
+    // (every wave has read sh.ru before a row leaves for the streaming loop,
+    // whose first tile writes there)
+    rw_bar();
     if (kmo == RW_KNAN || kms == RW_KNAN) return false;
     // (too many of a wave's groups at -inf, as under a mask: exactly)
     if (Ko && to <= kinf) to = rw_kth_key(2 * R.words, ng, Ko);
