@@ -88,8 +88,19 @@ struct rw_shared {
 // address it directly).
 __shared__ rw_shared rw_sh;
 // Bitmap of the row's patched ids, ceil(V / 32) words, followed by the number
-// of patched ids before each word (dynamic LDS).
+// of patched ids before each word (dynamic LDS); behind them rw_patches' two
+// bias bitmaps, then rw_groups' maxima in the same place.
 extern __shared__ uint32_t rw_pbits[];
+// Words of dynamic LDS: a CU's 160 KB less rw_shared and what the kernel's
+// other functions declare (below 1 KB).
+#define RW_DYN_WORDS ((163840u - (uint32_t)sizeof(rw_shared) - 1024u) / 4u)
+// Words of each bias bitmap: the whole row up to about 180000 ids; the bias
+// lists of wider rows are taken in windows of as many ids as fit.
+__host__ __device__ __forceinline__ uint32_t rw_bias_words(uint32_t words) {
+    const uint32_t fit = (RW_DYN_WORDS - 2u * words) / 2u;
+    return words < fit ? words : fit;
+}
+static_assert(2u * (ZS_MAX_VOCAB / 32u) + 2048u <= RW_DYN_WORDS, "the widest row's bitmap, counts and bias windows fit");
 
 #define RW_PF_SHIFT 30u
 
@@ -184,8 +195,9 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
     const zs_batch& b = a.b;
     const uint32_t t = threadIdx.x, V = b.V;
     const uint32_t words = (V + 31) / 32;
+    const uint32_t bw = rw_bias_words(words);
     uint32_t* seen = rw_pbits + 2 * words;   // bias ids met once, and more than once
-    uint32_t* dup = rw_pbits + 3 * words;
+    uint32_t* dup = seen + bw;
     const uint32_t ban0 = b.d_ban_off ? b.d_ban_off[r] : 0, ban1 = b.d_ban_off ? b.d_ban_off[r + 1] : 0;
     const uint32_t bi0 = b.d_bias_off ? b.d_bias_off[r] : 0, bi1 = b.d_bias_off ? b.d_bias_off[r + 1] : 0;
     uint32_t c0 = b.d_cnt_off ? b.d_cnt_off[r] : 0, c1 = b.d_cnt_off ? b.d_cnt_off[r + 1] : 0;
@@ -228,10 +240,7 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
         eid[u] = i < ne ? id_of(i) : 0xffffffffu;
         ev[u] = i < ne ? val_of(i) : 0u;
     }
-    for (uint32_t i = t; i < words; i += RW_NT) {
-        rw_pbits[i] = 0u;
-        if (nbi) { seen[i] = 0u; dup[i] = 0u; }
-    }
+    for (uint32_t i = t; i < words; i += RW_NT) rw_pbits[i] = 0u;
 #pragma unroll
     for (int u = 0; u < RW_PE; u++) ex[u] = eid[u] < V ? x_of(eid[u]) : 0.0f;
     // calls f(i, id, value, x) for this thread's entries of [i0, i1) with an id
@@ -261,12 +270,8 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
         else out_y[k] = y;
     };
     rw_bar();
-    // the patched ids, and the bias ids that occur more than once
-    each(0, ne, [&](uint32_t i, uint32_t id, uint32_t, auto&&) {
-        const uint32_t bit = 1u << (id & 31);
-        atomicOr(&rw_pbits[id >> 5], bit);
-        if (i >= nb && i < nb + nbi && (atomicOr(&seen[id >> 5], bit) & bit)) atomicOr(&dup[id >> 5], bit);
-    });
+    // the patched ids
+    each(0, ne, [&](uint32_t, uint32_t id, uint32_t, auto&&) { atomicOr(&rw_pbits[id >> 5], 1u << (id & 31)); });
     rw_bar();
     // per-word prefix counts of the bitmap: each wave its own stretch of
     // words, 64 at a time
@@ -321,18 +326,27 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
     }
     // logit_bias (decode_ctrl.rs:108-112): an id met once takes its bias in
     // parallel; the entries of an id met more than once are added by one
-    // thread in list order
-    if (nbi) {
+    // thread in list order. By windows of the ids (one window up to about
+    // 180000 ids): word w of the row is word w - b0 of a window.
+    for (uint32_t b0 = 0; nbi && b0 < words; b0 += bw) {
+        for (uint32_t i = t; i < 2 * bw; i += RW_NT) seen[i] = 0u;   // (dup follows seen)
+        rw_bar();
+        each(nb, nb + nbi, [&](uint32_t, uint32_t id, uint32_t, auto&&) {
+            const uint32_t w = (id >> 5) - b0, bit = 1u << (id & 31);
+            if (w < bw && (atomicOr(&seen[w], bit) & bit)) atomicOr(&dup[w], bit);
+        });
+        rw_bar();
         each(nb, nb + nbi, [&](uint32_t, uint32_t id, uint32_t v, auto&&) {
-            if ((dup[id >> 5] >> (id & 31)) & 1u) return;
+            const uint32_t w = (id >> 5) - b0;
+            if (w >= bw || ((dup[w] >> (id & 31)) & 1u)) return;
             const uint32_t k = rw_rank(id, words);
             SET_Y(k, Y(k) + zs_u2f(v));
             SET_FL(k, FL(k) | ZS_PF_Y);
         });
         if (t == 0) {
             for (uint32_t i = 0; i < nbi; i++) {
-                const uint32_t id = b.d_bias_ids[bi0 + i];
-                if (id >= V || !((dup[id >> 5] >> (id & 31)) & 1u)) continue;
+                const uint32_t id = b.d_bias_ids[bi0 + i], w = (id >> 5) - b0;
+                if (id >= V || w >= bw || !((dup[w] >> (id & 31)) & 1u)) continue;
                 const uint32_t k = rw_rank(id, words);
                 SET_Y(k, Y(k) + b.d_bias_vals[bi0 + i]);
                 SET_FL(k, FL(k) | ZS_PF_Y);
@@ -1356,13 +1370,16 @@ __global__ __launch_bounds__(SC_NT) void zs_k_scan(zs_sargs a) {
 
 // Group size of the scan: the row kernel holds the maxima of at most RW_GPT
 // groups per thread; smaller groups mean fewer ids read twice. 0: rows below
-// two of the streaming loop's tiles gain nothing from a second launch.
+// two of the streaming loop's tiles gain nothing from a second launch, and the
+// maxima of rows past about 240000 ids do not fit the LDS beside the bitmap.
 uint32_t zs_scan_gshift(uint32_t V) {
     if (V < 2 * RW_G) return 0;
     uint32_t gs = 4;
     while (((V + (1u << gs) - 1u) >> gs) > RW_GPT * RW_NT) gs++;
-    return gs;
+    if (2u * ((V + 31u) / 32u) + 2u * ((V + (1u << gs) - 1u) >> gs) > RW_DYN_WORDS) return 0;
+    return gs;   // at most 6: V <= ZS_MAX_VOCAB
 }
+static_assert((ZS_MAX_VOCAB >> 6) <= RW_GPT * RW_NT, "groups of 64 ids serve the widest row");
 
 // ---------------------------------------------------------------------------
 // zs_k_row
@@ -2039,7 +2056,7 @@ extern "C" int zs_dbg_row_stats(unsigned long long* out) {
 
 extern "C" int zs_row_launch(const zs_sargs& a, hipStream_t stream) {
     const uint32_t words = (a.b.V + 31) / 32;
-    size_t tail = 2 * words;   // rw_patches' bias bitmaps, then the group maxima
+    size_t tail = 2 * rw_bias_words(words);   // rw_patches' bias bitmaps, then the group maxima
     if (a.gshift) {
         const uint32_t ng = (a.b.V + (1u << a.gshift) - 1u) >> a.gshift;
         const dim3 grid((a.b.V + SC_IDS - 1) / SC_IDS, a.b.B);
