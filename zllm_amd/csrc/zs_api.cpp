@@ -823,6 +823,8 @@ extern "C" int zs_sample(zs_ctx* ctx, const zs_batch* b, void* stream) {
     int prev = 0;
     (void)hipGetDevice(&prev);
     if (prev != ctx->device) (void)hipSetDevice(ctx->device);
+    __atomic_store_n(&ctx->sample_stream, (const void*)stream, __ATOMIC_RELAXED);
+    __atomic_store_n(&ctx->sampled, 1u, __ATOMIC_RELAXED);
     int rc = zs_sample_launch(ctx, b, (hipStream_t)stream);
     if (prev != ctx->device) (void)hipSetDevice(prev);
     return rc;
@@ -908,6 +910,10 @@ extern "C" int zs_spec_verify(zs_ctx* ctx, const zs_spec_batch* b, void* stream)
     if (b->flags & ~(uint32_t)ZS_SPEC_BACKGROUND)
         return zs_set_error(ctx, ZS_EINVAL, "zs_spec_verify: unknown flags %#x", b->flags);
     a.background = (b->flags & ZS_SPEC_BACKGROUND) ? 1u : 0u;
+    // on the sampler's own stream nothing of the sampler runs meanwhile (which
+    // launches are made, not what they compute, hangs on this)
+    a.beside = __atomic_load_n(&ctx->sampled, __ATOMIC_RELAXED) &&
+               __atomic_load_n(&ctx->sample_stream, __ATOMIC_RELAXED) != (const void*)stream;
     int prev = zs_device_guard_begin(ctx);
     zs_prof prof{ctx->profiling, ctx->spec_events, ctx->spec_names, &ctx->n_spec_timed};
     int rc = zs_spec_launch(a, prof, (hipStream_t)stream);

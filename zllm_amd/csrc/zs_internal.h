@@ -154,6 +154,7 @@ struct zs_spec_args {
     zs_spec_row* rs;            // scratch [B]
     uint32_t nch, npos_max;
     uint32_t background;        // ZS_SPEC_BACKGROUND: the fused one-workgroup-per-CU passes
+    uint32_t beside;            // a sampler may run on another stream meanwhile: launches of bounded size
 };
 
 struct zs_ctx {
@@ -212,6 +213,10 @@ struct zs_ctx {
     uint32_t* lane_host;         // pinned [2][4][rows]: temp, top_k, top_p, seed (two areas, alternating)
     void* lane_event[2];         // hipEvent_t: the staging copy from each area done
     uint32_t lane_slot;          // the area the next call fills
+    // the stream of the context's last zs_sample (compared, never used; the
+    // verification may be called from another thread): null before the first
+    const void* sample_stream;
+    uint32_t sampled;
     int n_spec_timed;      // the same for the last zs_spec_verify call
     void* spec_events[8];
     const char* spec_names[8];

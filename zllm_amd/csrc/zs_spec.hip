@@ -100,10 +100,12 @@ __device__ __forceinline__ uint32_t sp_id(uint32_t base, int e) {
 // many holds every slot that one of its own gives up, and a kernel beside it on
 // another stream that needs much of a CU (zs_k_row: 168 registers of 8 waves
 // and 149 KB of LDS at 151936 ids) waits for its end: 190 us instead of 47 beside
-// 43776 workgroups. So the rows go in equal launches of at most SP_PART
-// workgroups: between two of them the CUs come free. Full step of 256 rows (9
-// positions of 151936 ids beside the sampler): one launch 677 us, two 638, three
-// 645, five 651, ten 658; alone each further launch adds about 8 us.
+// 43776 workgroups. So where a sampler may run beside it (zs_spec_args.beside)
+// the rows go in equal launches of at most SP_PART workgroups: between two of
+// them the CUs come free. Full step of 256 rows (9 positions of 151936 ids
+// beside the sampler; one batch of logits): one launch 677 us, two 638, three
+// 645, five 651, ten 658; other batches, one and two: 680 and 656. Alone each
+// further launch adds about 10 us (302 and 316), so it is one launch there.
 #define SP_PART 24576u
 __global__ __launch_bounds__(SP_NT) void zs_k_spec_chunk(zs_spec_args a, uint32_t r0) {
     const uint32_t c = blockIdx.x, pos = blockIdx.y, r = r0 + blockIdx.z;
@@ -301,10 +303,11 @@ __device__ __forceinline__ u128 wave_sum_u128(u128 v) {
 // SP_NT-thread workgroup: the waves take the positions in turn (maximum, first
 // argmax, weight sum and the draft id's weight of a position in one visit to
 // its chunk records), then one lane per draft makes its accept test and the
-// first rejection decides. Every workgroup of zs_k_spec_rsum makes it for
-// itself (one wave per row visiting the positions one after the other, and the
-// drafts' tests one after the other, took a launch of 18 us on 64 rows of 9
-// positions; the residual pass with it in front takes 5 us more than without).
+// first rejection decides (one wave per row visiting the positions one after
+// the other, and the drafts' tests one after the other, took a launch of 18 us
+// on 64 rows of 9 positions). In a launch of its own (zs_k_spec_decide), or, of
+// at most SP_DECIDE_WGS workgroups, by every workgroup of the residual pass for
+// itself: that saves the launch but repeats the work once a chunk.
 #define SP_NPOS (2 * ZS_SPEC_KMAX + 1)
 struct sp_decision {
     zs_spec_row row;
@@ -474,20 +477,37 @@ __device__ __forceinline__ u128 spd_weight2(const zs_spec_row& s, const sp_chunk
     return pp > qq ? pp - qq : 0;
 }
 
-// pass 3: the decision, and chunk sums of the residual weights (rows that
-// rejected a draft). Chunk 0's workgroup stores the decision; without draft
-// logits every row is verified greedily and it is the only one launched.
+__device__ __forceinline__ void sp_store(const zs_spec_args& a, uint32_t r, const sp_decision& S) {
+    if (threadIdx.x != 0) return;
+    a.accepted[r] = S.accepted;
+    if (S.row.mode == 0) a.next[r] = S.next;
+    a.rs[r] = S.row;
+}
+__global__ __launch_bounds__(SP_NT) void zs_k_spec_decide(zs_spec_args a) {
+    __shared__ sp_decision S;
+    sp_decide(a, blockIdx.x, S);
+    sp_store(a, blockIdx.x, S);
+}
+
+// pass 3: chunk sums of the residual weights (rows that rejected a draft);
+// DECIDE: the decision in front, stored by chunk 0's workgroup. Rejection
+// sampling alone, in a launch of its own / in front (us a call, 9 positions):
+// 32 x 151936 (608 workgroups) 68 / 67, 64 x 128256 (1024) 91 / 90, 128 x
+// 151936 (2432) 172 / 179, 256 x 151936 (4864) 302 / 323.
+#define SP_DECIDE_WGS 2048u
+template <bool DECIDE>
 __global__ __launch_bounds__(SP_NT) void zs_k_spec_rsum(zs_spec_args a) {
     const uint32_t c = blockIdx.x, r = blockIdx.y;
     const uint32_t base = c * SP_CH;
     if (base >= a.V) return;
-    __shared__ sp_decision S;
-    sp_decide(a, r, S);
-    const zs_spec_row s = S.row;
-    if (c == 0 && threadIdx.x == 0) {
-        a.accepted[r] = S.accepted;
-        if (s.mode == 0) a.next[r] = S.next;
-        a.rs[r] = s;
+    zs_spec_row s;
+    if constexpr (DECIDE) {
+        __shared__ sp_decision S;
+        sp_decide(a, r, S);
+        s = S.row;
+        if (c == 0) sp_store(a, r, S);
+    } else {
+        s = a.rs[r];
     }
     if (s.mode != 1 || !s.residual) return;
     __shared__ unsigned long long lo[SP_NT / 64], hi[SP_NT / 64];
@@ -642,13 +662,19 @@ extern "C" int zs_spec_launch(const zs_spec_args& a, const zs_prof& prof, hipStr
         hipLaunchKernelGGL(zs_k_spec_row, dim3(npos, a.B), dim3(SR_NT), SR_LDS_HOLD, stream, a);
         mark("zs_k_spec_row");
     } else {
-        const uint64_t parts = ((uint64_t)nch * npos * a.B + SP_PART - 1) / SP_PART;
+        const uint64_t parts = a.beside ? ((uint64_t)nch * npos * a.B + SP_PART - 1) / SP_PART : 1;
         const uint32_t per = (uint32_t)((a.B + parts - 1) / parts);
         for (uint32_t r0 = 0; r0 < a.B; r0 += per)
             hipLaunchKernelGGL(zs_k_spec_chunk, dim3(nch, npos, std::min(per, a.B - r0)), dim3(SP_NT), 0, stream, a, r0);
         mark("zs_k_spec_chunk");
     }
-    hipLaunchKernelGGL(zs_k_spec_rsum, dim3(a.draft ? nch : 1, a.B), dim3(SP_NT), 0, stream, a);
+    // (without draft logits every row is verified greedily: the decision is all)
+    if (a.draft && (uint64_t)nch * a.B <= SP_DECIDE_WGS) {
+        hipLaunchKernelGGL(zs_k_spec_rsum<true>, dim3(nch, a.B), dim3(SP_NT), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL(zs_k_spec_decide, dim3(a.B), dim3(SP_NT), 0, stream, a);
+        if (a.draft) hipLaunchKernelGGL(zs_k_spec_rsum<false>, dim3(nch, a.B), dim3(SP_NT), 0, stream, a);
+    }
     if (a.draft) hipLaunchKernelGGL(zs_k_spec_draw, dim3(a.B), dim3(SP_BIG_NT), 0, stream, a);
     mark("zs_k_spec_draw");
     if (prof.on) *prof.n = ev - 1;
