@@ -81,3 +81,22 @@ def test_walk_masked_rows():
     params = [dict(temperature=float(t), top_k=0, top_p=float(tp), seed=30 + i, masked=True, top_logprobs=2)
               for i, (t, tp) in enumerate([(1.0, 0.9), (1.3, 0.8), (0.9, 0.95), (1.1, 0.99), (1.5, 0.7), (1.0, 0.6)])]
     _run(x, params, allow_bits=bits, allow=allow)
+
+
+def test_walk_buckets_past_top_p():
+    """A bucket of one value the sum cannot reach, then one of 4000 values
+    whose margin (it grows with the count) reaches back below top_p: neither
+    belongs to the walk, which stops inside the top values."""
+    n, W = 6, 40000
+    rng = np.random.default_rng(53)
+    x = np.full((n, W), -30.0, np.float32)
+    for i in range(n):
+        ids = rng.permutation(W)
+        top = 0.900005 + 5e-6 * i
+        p = np.concatenate([np.full(9, top / 9), [3e-5], rng.uniform(2.30e-5, 2.40e-5, 4000)])
+        rest = 1.0 - p.sum()
+        p = np.concatenate([p, np.full(2000, rest / 2000)])
+        x[i, ids[:len(p)]] = np.log(p).astype(np.float32)
+    params = [dict(temperature=1.0, top_k=0, top_p=0.9, seed=i, counter=i, top_logprobs=5) for i in range(n)]
+    out = _run(x, params)
+    assert not any(out["status"] & 4)

@@ -615,6 +615,11 @@ __global__ __launch_bounds__(ZS_BIG_NT) void zs_k_tp_plan(zs_sargs a) {
         B.tot = 0ull;
     }
     rlim = block_min_i<ZS_BIG_NT>(rlim, reinterpret_cast<int*>(su));
+    // (lo does not grow with every bucket: one past rlim may still look like a
+    // candidate, but holds no values to sort)
+#pragma unroll
+    for (int k2 = 0; k2 < 2; k2++)
+        if (2 * t + k2 >= rlim) cand[k2] = 0u;
     uint32_t ntot;
     const uint32_t pos = block_excl_scan_u<ZS_BIG_NT>(cand[0] + cand[1], su, &ntot);
     if (ntot > ZS_TP_CAND) {
