@@ -36,3 +36,20 @@ def test_btopk_from_group_maxima(V, K):
         ov, oi = O.btopk(x[s], K)
         assert idxs[s].tolist() == oi.tolist(), s
         assert vals[s].tobytes() == ov.tobytes(), s
+
+
+def test_btopk_of_no_ids():
+    """Rows of no ids: refused on the group path before anything is launched
+    (its kernels index the maxima of the last group), all sentinels past it."""
+    from tests.gpu_util import ctx
+    from zllm_amd._lib import lib
+    c = ctx()
+    x = torch.zeros(4, device="cuda")
+    vals, idxs = torch.zeros((2, 65), device="cuda"), torch.zeros((2, 65), dtype=torch.int32, device="cuda")
+    call = lambda K: lib().zs_lane_topk(c.h, x.data_ptr(), 2, 0, 0, K, vals.data_ptr(), idxs.data_ptr(), None)
+    assert call(64) == -1   # ZS_EINVAL
+    torch.cuda.synchronize()
+    assert not vals.any() and not idxs.any()
+    assert call(65) == 0
+    torch.cuda.synchronize()
+    assert (idxs == -1).all() and (vals < -2.9e38).all()

@@ -960,8 +960,9 @@ extern "C" int zs_lane_topk(zs_ctx* ctx, const float* d_logits, uint32_t B, uint
     if (!d_vals || !d_idxs) return zs_set_error(ctx, ZS_EINVAL, "zs_lane_topk: null output");
     if (K == 0 || K > 1024) return zs_set_error(ctx, ZS_ELIMIT, "zs_lane_topk: K=%u outside 1..1024", K);
     if (B == 0) return ZS_OK;
-    int prev = zs_device_guard_begin(ctx);
     const bool fits = B <= ctx->max_rows && V <= ctx->max_vocab;
+    if (V == 0 && fits && K <= 64) return zs_set_error(ctx, ZS_EINVAL, "zs_lane_topk: V == 0");   // no groups to take
+    int prev = zs_device_guard_begin(ctx);
     rc = zs_lane_topk_launch(d_logits, B, V, ld, K, d_vals, d_idxs, fits ? ctx->lane_gmax : nullptr,
                              ctx->max_vocab / ZS_SCAN_MIN_GROUP + 1, (hipStream_t)stream);
     zs_device_guard_end(ctx, prev);
