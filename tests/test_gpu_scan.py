@@ -127,3 +127,34 @@ def test_min_p_kept_lists(top_p):
     print(f"[case] min-p kept lists top_p={top_p}", flush=True)
     errs = compare(x, params, run_gpu(x, params))
     assert not errs, "\n".join(errs)
+
+
+# per width: three quarters of the groups and one more, and the largest k whose
+# ids are expected to fit the list and one more
+@pytest.mark.parametrize("V,ks", [(4096, (129, 192, 193, 511)), (20000, (511, 512, 937, 938, 1200)), (32000, (1500, 1501)),
+                                  (100003, (2304, 2305, 2400)), (128256, (2500, 2594, 2595, 3073))])
+def test_wide_top_k(V, ks):
+    rng = np.random.default_rng(V)
+    x = rng.normal(0, 2, (2 * len(ks), V)).astype(np.float32)
+    params = [dict(temperature=1.1, top_k=k, top_p=0.98, min_p=0.01 * (i % 2), top_logprobs=20, seed=i)
+              for i, k in enumerate(np.repeat(ks, 2).tolist())]
+    print(f"[case] wide top-k V={V}", flush=True)
+    errs = compare(x, params, _run_padded(x, params))
+    assert not errs, "\n".join(errs[:20])
+
+
+def test_wide_top_k_lists_that_overflow():
+    """More values at the threshold than the sampler's list holds, with the
+    observers' candidates above them: k up to 128 streams the row, larger k keep
+    the observers' list alone; without observers nothing else is listed."""
+    V = 50257
+    rng = np.random.default_rng(8)
+    P = [dict(temperature=1.0, top_k=k, top_p=0.9, top_logprobs=20, seed=i) for i, k in enumerate((100, 300, 511, 700, 300))]
+    P[4].update(logprobs=False, detect_hallucination=False, top_logprobs=0)
+    x = rng.normal(0, 1, (len(P), V)).astype(np.float32)
+    for i in range(len(P)):
+        x[i, 16 * 1000:16 * 1400] = 9.0                       # 400 groups of 16 equal values
+        x[i, rng.choice(16000, 60, replace=False)] = rng.uniform(10, 12, 60).astype(np.float32)
+    print("[case] wide top-k overflow", flush=True)
+    errs = compare(x, P, _run_padded(x, P))
+    assert not errs, "\n".join(errs)

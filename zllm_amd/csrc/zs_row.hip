@@ -957,7 +957,6 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 // Returns false (uniformly) for rows whose lists would overflow or that hold
 // a NaN: they take the streaming loop of zs_k_row.
 // ---------------------------------------------------------------------------
-#define RW_KWIDE 3072      // largest k whose threshold comes from the lists
 #define RW_WIDE (2 * RW_BUF)   // keys in the sampler list's place
 #define RW_GOBS (RW_BUF / 2)   // observers listed at most; the listed groups (u16) follow them in LDS
 #define RW_GL (RW_BUF * 2)     // listed groups at most
@@ -968,7 +967,22 @@ struct rw_gst {
     unsigned long long gbest;
     uint32_t n_o, n_s;
     bool s_over;
+    bool s_drop;   // the sampler's list did not fit and is not kept (k > ZS_KS)
 };
+// Whether the groups give a threshold close to the k-th of k > ZS_KS: at most
+// three quarters of them reach it, and the ids expected at or above it fit
+// their list. With ids in no order a group holds Poisson(m) of them, m = -ln(1
+// - k / groups), which is ng * m in all (of 128256 ids, k = 2594 lists 4176 and
+// k = 3000 5540); a list that overflows costs a fifth of what one
+// that fits saves, so the line lies 2% past its length (1.6% are one standard
+// deviation). zs_k_big selects the threshold of the others. 8 rows, us a call,
+// by lists / by zs_k_big: k = 2000 of 100003 ids 220 / 574, k = 2500 of 151936
+// 280 / 765.
+__device__ __forceinline__ bool rw_wide_fits(uint32_t k, uint32_t ng) {
+    if (4u * k > 3u * ng) return false;
+    const float n = (float)ng;
+    return -n * __logf(1.0f - (float)k / n) <= 1.02f * (float)RW_WIDE;
+}
 __device__ __forceinline__ uint32_t rw_wave_umax(uint32_t v) {
     v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
     v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
@@ -1148,7 +1162,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     // is reached by c groups of that wave, so the smallest of the waves' is
     // reached by K groups (k past a wave's width: the K-th largest group
     // maximum itself)
-    const bool wide = Ks > 64u * RW_NW / 4u;
+    const bool wide = Ks > ZS_KS;   // (a quarter of the threads)
     const uint32_t so = wave_sort_u32(mo), ss = wave_sort_u32(ms);
     const int co = max((int)((Ko + RW_NW - 1) / RW_NW), 1), cs = wide ? 1 : max((int)((Ks + RW_NW - 1) / RW_NW), 1);
     const uint32_t wo = (uint32_t)__builtin_amdgcn_readlane((int)so, 64 - co);
@@ -1173,7 +1187,6 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     // (too many of a wave's groups at -inf, as under a mask: exactly)
     if (Ko && to <= kinf) to = rw_kth_key(2 * R.words, ng, Ko);
     if (smode & 1u) {
-        if (wide && 4u * Ks > 3u * ng) return false;   // too few groups for a close threshold
         if (wide || ts <= kinf) ts = rw_kth_key(2 * R.words + ng, ng, Ks);
     } else if (smode == 2) {
         // every y above -inf, when few enough groups hold one
@@ -1258,9 +1271,15 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     }
     __syncthreads();
     uint32_t n_o = rw_uni(sh.sel_st[2]);
-    const uint32_t n_s = rw_uni(sh.sel_st[3]);
+    uint32_t n_s = rw_uni(sh.sel_st[3]);
     __syncthreads();   // (the count is read before the ids at -inf are added to it)
-    if (n_o > RW_GOBS || ((smode & 1u) && n_s > scap)) return false;
+    if (n_o > RW_GOBS) return false;
+    if ((smode & 1u) && n_s > scap) {
+        // (the streaming loop would list no k > ZS_KS either)
+        if (Ks <= ZS_KS) return false;
+        G.s_drop = true;
+        n_s = 0;
+    }
     if (n_o < Ko) {
         // fewer than Ko ids above -inf: the smallest ids at -inf follow (at
         // most Ko of the first 64 ids are above it)
@@ -1433,10 +1452,10 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     // sampler list: 1 = top-k by y (k <= ZS_KS), 2 = every y > -inf (the
     // small-survivor check when no top-k applies), 0 = none; from the group
     // maxima also larger k: 1 while the survivors fit the small path, 3 (the
-    // keys only, for the threshold) up to RW_KWIDE
+    // keys only, for the threshold) as far as rw_wide_fits
     const bool has_groups = a.gshift && !tinf && R.np <= ZS_PATCH_LDS;
     const uint32_t kmax1 = has_groups ? (uint32_t)ZS_SMALL_CAP - 1u : (uint32_t)ZS_KS;
-    uint32_t smode = greedy ? 0u : (!has_topk ? 2u : P.top_k <= kmax1 ? 1u : (has_groups && P.top_k <= RW_KWIDE) ? 3u : 0u);
+    uint32_t smode = greedy ? 0u : (!has_topk ? 2u : P.top_k <= kmax1 ? 1u : has_groups ? 3u : 0u);
     uint32_t Ks = (smode & 1u) ? P.top_k : 0u;
     const uint32_t Ko = want_obs ? (ZS_OBS_CAND < V ? ZS_OBS_CAND : V) : 0u;
     rw_list LO, LS;
@@ -1501,15 +1520,16 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     RW_T(1);
     // ---- the lists from the group maxima of zs_k_scan
     bool fast = false;
-    if (!gath && a.gshift && !tinf && R.np <= ZS_PATCH_LDS) {
-        rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, false};
+    if (!gath && has_groups) {
+        if (Ks > ZS_KS && !rw_wide_fits(Ks, (V + (1u << a.gshift) - 1u) >> a.gshift)) { smode = 0; Ks = 0; }
+        rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, false, false};
         fast = rw_groups(a, r, R, greedy, smode, Ks, Ko, G);
         if (fast) {
             omax = G.omax; ymax = G.ymax; rejf = G.rejf; gbest = G.gbest;
             n_o = G.n_o; n_s = G.n_s; s_over = G.s_over;
         }
+        if ((!fast && Ks > ZS_KS) || G.s_drop) { smode = 0; Ks = 0; }
     }
-    if (!gath && !fast && has_topk && P.top_k > ZS_KS) { smode = 0; Ks = 0; }
     uint32_t g = 0;
     const uint32_t ng = (gath || fast) ? 0u : R.gend;
     const uint32_t Vend = R.vend;
