@@ -158,3 +158,40 @@ def test_wide_top_k_lists_that_overflow():
     print("[case] wide top-k overflow", flush=True)
     errs = compare(x, P, _run_padded(x, P))
     assert not errs, "\n".join(errs)
+
+
+@pytest.mark.parametrize("V", [20001, 50257, 128256, 163844])
+def test_many_groups_at_a_threshold(V):
+    """Rows of few distinct values, where most groups reach a threshold: the
+    observers' ties by id, the sampler's k-th value at, above and below the
+    tied value, k of every kind of list, ties under masks, bans and counts."""
+    rng = np.random.default_rng(V)
+    B = 22
+    x = np.full((B, V), 1.5, np.float32)
+    P = [dict(temperature=0.9, top_k=40, top_p=0.95, top_logprobs=20, seed=i) for i in range(B)]
+    allow = np.ones((B, V), bool)
+    for i, k in ((1, 1), (2, 128), (3, 300), (4, 511), (5, 600), (6, 900), (7, 0)):
+        P[i].update(top_k=k)
+    for i, n in ((8, 10), (9, 39), (10, 40), (11, 41), (12, 200)):
+        x[i, rng.choice(V, n, replace=False)] = rng.uniform(2, 5, n).astype(np.float32)   # above the tied value
+    x[13] = rng.integers(0, 3, V).astype(np.float32)                  # three values, the largest in most groups
+    x[14] = np.where(rng.random(V) < 0.5, 0.0, -0.0).astype(np.float32)
+    x[14, ::16] = 1.0                                                 # one id per group of 16
+    x[15, :V // 2] = -np.inf                                          # ties in the second half alone
+    P[16].update(ban=rng.choice(V, 700, replace=False).tolist(), counts=[(int(t), 2) for t in rng.choice(V, 900, replace=False)],
+                 presence=0.5)
+    P[17].update(temperature=0.0)                                     # greedy: the last id
+    P[18].update(masked=True)
+    allow[18] = rng.random(V) < 0.5
+    P[19].update(masked=True, top_k=600)
+    allow[19] = rng.random(V) < 0.9
+    allow[19, :V // 3] = False
+    x[20] = -np.finfo(np.float32).max                                 # the value next to -inf
+    P[21].update(logprobs=False, detect_hallucination=False, top_logprobs=0)
+    bits = np.zeros((B, (V + 31) // 32), np.uint32)
+    for i in range(B):
+        bits[i] = np.packbits(np.pad(allow[i], (0, -V % 32)), bitorder="little").view(np.uint32)
+    print(f"[case] ties V={V}", flush=True)
+    refs = [oracle_row(x[i], P[i], allow[i] if P[i].get("masked") else None) for i in range(B)]
+    errs = compare(x, P, _run_padded(x, P, bits.view(np.int32)), refs=refs)
+    assert not errs, "\n".join(errs[:20])

@@ -961,6 +961,7 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 #define RW_GOBS (RW_BUF / 2)   // observers listed at most; the listed groups (u16) follow them in LDS
 #define RW_GL (RW_BUF * 2)     // listed groups at most
 #define RW_GF 14u              // a listed group: group | list flags << RW_GF
+#define RW_GTIES 1024          // groups listed beyond k at most without a look at the ties among them
 #define RW_GPT 10          // groups per thread at most (zs_scan_gshift)
 struct rw_gst {
     float omax, ymax, rejf;
@@ -973,11 +974,11 @@ struct rw_gst {
 // three quarters of them reach it, and the ids expected at or above it fit
 // their list. With ids in no order a group holds Poisson(m) of them, m = -ln(1
 // - k / groups), which is ng * m in all (of 128256 ids, k = 2594 lists 4176 and
-// k = 3000 5540); a list that overflows costs a fifth of what one
+// k = 3000 5540); a list that overflows costs a sixth of what one
 // that fits saves, so the line lies 2% past its length (1.6% are one standard
 // deviation). zs_k_big selects the threshold of the others. 8 rows, us a call,
-// by lists / by zs_k_big: k = 2000 of 100003 ids 220 / 574, k = 2500 of 151936
-// 280 / 765.
+// by lists / by zs_k_big: k = 2250 of 100003 ids 214 / 573, k = 2550 of 128256
+// 222 / 682.
 __device__ __forceinline__ bool rw_wide_fits(uint32_t k, uint32_t ng) {
     if (4u * k > 3u * ng) return false;
     const float n = (float)ng;
@@ -1003,6 +1004,23 @@ __device__ __forceinline__ uint32_t rw_lanes_umax(uint32_t v, uint32_t qs) {
 // Key of a group maximum: -0 and +0 alike, a NaN above everything.
 #define RW_KNAN 0xffffffffu
 __device__ __forceinline__ uint32_t rw_gkey(float m, bool nan) { return nan ? RW_KNAN : zs_total_key(m + 0.0f); }
+
+// Places behind a counter for the lanes' entries, one atomic per wave (one per
+// lane is served lane by lane: a row of equal values spent 350 us on 64 K of
+// them). Called by whole waves.
+__device__ __forceinline__ uint32_t rw_wave_reserve(uint32_t* ctr, bool one) {
+    const unsigned long long m = __ballot(one);
+    uint32_t p = 0;
+    if (m && zs_lane() == 0) p = atomicAdd(ctr, (uint32_t)__popcll(m));
+    p = (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, p));
+}
+__device__ __forceinline__ uint32_t rw_wave_reserve_n(uint32_t* ctr, uint32_t n) {
+    const uint32_t inc = rw_wave_scan(n);
+    uint32_t p = 0;
+    if (zs_lane() == 63) p = atomicAdd(ctr, inc);
+    return (uint32_t)__builtin_amdgcn_readlane((int)p, 63) + inc - n;
+}
 
 // x~ and y of the 4 ids from idx0 (a multiple of 4; ids >= V read -inf).
 __device__ __forceinline__ void rw_load4(const rw_row& R, uint32_t idx0, const float4& v, uint32_t w, float (&x)[4],
@@ -1200,18 +1218,51 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     ts = sl ? max(ts, kinf + 1u) : 0xffffffffu;
     RW_T(15);
     // the groups that reach a threshold
-    uint32_t rej = 0;
+    uint32_t rej = 0, n_gl, keep = ~0u, pad = 0u;   // keep: bit e, the observers of group e are listed
+    for (bool cut = false;; cut = true) {
+        rej = 0;
 #pragma unroll
-    for (int e = 0; e < RW_GPT; e++) {
-        const uint32_t f = (kx[e] >= to ? 1u : 0u) | (ky[e] >= ts ? 2u : 0u);
-        if (!(f & 2u)) rej = max(rej, ky[e]);
-        if (f) {
-            const uint32_t p = atomicAdd(&sh.n_gl, 1u);
-            if (p < RW_GL) gl[p] = (uint16_t)((t + (uint32_t)e * RW_NT) | (f << RW_GF));
+        for (int e = 0; e < RW_GPT; e++) {
+            const uint32_t f = (kx[e] >= to && (keep >> e & 1u) ? 1u : 0u) | (ky[e] >= ts ? 2u : 0u);
+            if (!(f & 2u)) rej = max(rej, ky[e]);
+            const uint32_t p = rw_wave_reserve(&sh.n_gl, f != 0u);
+            if (f && p < RW_GL) gl[p] = (uint16_t)((t + (uint32_t)e * RW_NT) | (f << RW_GF));
         }
+        __syncthreads();
+        n_gl = rw_uni(sh.n_gl);
+        if (cut || n_gl <= RW_GTIES + Ks) break;
+        // Many groups at a threshold: a row of few distinct values. Of the
+        // observers' groups at theirs only the first Ko are needed (each holds
+        // an id at it, and the smallest ids come first); the sampler's list
+        // takes the entries above its own and, for the k-th value, Ks places
+        // at it (the others count as turned away).
+        if (Ko) {
+#pragma unroll
+            for (int e = 0; e < RW_GPT; e++) {
+                const uint32_t c = (uint32_t)__popcll(__ballot(kx[e] == to));
+                if (zs_lane() == 0) sh.sel_hist[0][(uint32_t)e * RW_NW + wid] = c;
+            }
+            rw_bar();
+            uint32_t run = 0;
+            keep = 0;
+#pragma unroll
+            for (int e = 0; e < RW_GPT; e++) {
+                const unsigned long long m = __ballot(kx[e] == to);
+                uint32_t before = run;
+                for (uint32_t w = 0; w < RW_NW; w++) {
+                    const uint32_t c = sh.sel_hist[0][(uint32_t)e * RW_NW + w];
+                    before += w < wid ? c : 0u;
+                    run += c;
+                }
+                before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, before));
+                if (kx[e] != to || before < Ko) keep |= 1u << e;
+            }
+        }
+        if ((smode & 1u) && ts > kinf + 1u) pad = ts++;
+        __syncthreads();
+        if (t == 0) sh.n_gl = 0;
+        rw_bar();
     }
-    __syncthreads();
-    const uint32_t n_gl = rw_uni(sh.n_gl);
     if (n_gl > RW_GL) return false;
     const uint32_t nit = n_gl << qs;
     uint32_t* wk = reinterpret_cast<uint32_t*>(sh.u.b.s);
@@ -1230,7 +1281,6 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
 #pragma unroll
         for (int u = 0; u < NU; u++) {
             const uint32_t f = ge[u] >> RW_GF;
-            if (!f) continue;
             const uint32_t idx0 = ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * ((i0 + t + (uint32_t)u * RW_NT) & qm);
             float x[4], y[4];
             rw_load4(R, idx0, v[u], w[u], x, y, sh);
@@ -1241,13 +1291,13 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
             for (int q = 0; q < 4; q++) {
                 kxq[q] = zs_total_key(x[q] + 0.0f);
                 kyq[q] = zs_total_key(y[q] + 0.0f);
-                mo4 |= kxq[q] >= to ? 1u << q : 0u;
-                const bool in = kyq[q] >= ts;
+                mo4 |= (f & 1u) && kxq[q] >= to ? 1u << q : 0u;
+                const bool in = (f & 2u) && kyq[q] >= ts;
                 ms4 |= in ? 1u << q : 0u;
-                if (!in) rej = max(rej, kyq[q]);
+                if (f && !in) rej = max(rej, kyq[q]);
             }
-            if ((f & 1u) && mo4) {
-                uint32_t p = atomicAdd(&sh.sel_st[2], (uint32_t)__popc(mo4));
+            if (__ballot(mo4 != 0u)) {
+                uint32_t p = rw_wave_reserve_n(&sh.sel_st[2], (uint32_t)__popc(mo4));
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     if (!((mo4 >> q) & 1u)) continue;
@@ -1255,8 +1305,8 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
                     p++;
                 }
             }
-            if ((f & 2u) && ms4) {
-                uint32_t p = atomicAdd(&sh.sel_st[3], (uint32_t)__popc(ms4));
+            if (__ballot(ms4 != 0u)) {
+                uint32_t p = rw_wave_reserve_n(&sh.sel_st[3], (uint32_t)__popc(ms4));
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     if (!((ms4 >> q) & 1u)) continue;
@@ -1274,11 +1324,18 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     uint32_t n_s = rw_uni(sh.sel_st[3]);
     __syncthreads();   // (the count is read before the ids at -inf are added to it)
     if (n_o > RW_GOBS) return false;
-    if ((smode & 1u) && n_s > scap) {
+    if ((smode & 1u) && n_s + (pad ? Ks : 0u) > scap) {
         // (the streaming loop would list no k > ZS_KS either)
         if (Ks <= ZS_KS) return false;
         G.s_drop = true;
         n_s = 0;
+    } else if (pad) {
+        for (uint32_t i = t; i < Ks; i += RW_NT) {
+            if (smode == 3) wk[n_s + i] = pad;
+            else sh.u.b.s[n_s + i] = ((unsigned long long)(~pad) << 32) | i;
+        }
+        n_s += Ks;
+        rej = max(rej, pad);
     }
     if (n_o < Ko) {
         // fewer than Ko ids above -inf: the smallest ids at -inf follow (at
