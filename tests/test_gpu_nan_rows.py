@@ -1,6 +1,5 @@
 """NaN rows in one batch with masked rows, rows of a wide top-k and greedy
-rows, while a verification runs on a second stream: a NaN row leaves the row
-kernel's group path where its neighbours stay in it. Every pass against the
+rows, while a verification runs on a second stream. Every pass against the
 oracle (tokens and top ids bit for bit, floats within gpu_util.compare's
 1e-5) and the same in every pass."""
 import numpy as np

@@ -36,7 +36,7 @@ def _case(V):
     x[15, [5, V // 3, V - 2]] = 30.0               # greedy: the last of the equal maxima
     P[15].update(temperature=0.0)
     x[16] = np.where(rng.random(V) < 0.5, np.float32(0.0), np.float32(-0.0))   # zeros of both signs at the threshold
-    x[17, 11] = np.nan                             # streamed: NaN
+    x[17, 11] = np.nan                             # a NaN
     x[18, V // 2] = np.inf
     P[19].update(temperature=0.0, counts=[(int(np.argmax(x[19])), 1)], presence=50.0)   # greedy, the maximum penalised
     return x, P
@@ -192,6 +192,50 @@ def test_many_groups_at_a_threshold(V):
     for i in range(B):
         bits[i] = np.packbits(np.pad(allow[i], (0, -V % 32)), bitorder="little").view(np.uint32)
     print(f"[case] ties V={V}", flush=True)
+    refs = [oracle_row(x[i], P[i], allow[i] if P[i].get("masked") else None) for i in range(B)]
+    errs = compare(x, P, _run_padded(x, P, bits.view(np.int32)), refs=refs)
+    assert not errs, "\n".join(errs[:20])
+
+
+@pytest.mark.parametrize("V", [4096, 50257, 128256, 163841])
+def test_nan_in_a_group(V):
+    """The greedy fold after the last NaN, which lies first, last, in the middle
+    and next to others in its group, in the last group, at a penalised or
+    biased id, under a mask or a ban (no NaN then), before values at -inf, ties
+    and larger values in front of it; sampled rows beside them."""
+    rng = np.random.default_rng(V)
+    gs = 16 if V <= 81920 else 32 if V <= 163840 else 64
+    g0 = V // 2 // gs * gs                                            # a group's first id
+    at = [[g0], [g0 + gs - 1], [g0 + 5], [g0, g0 + 3, g0 + 9], [V - 1], [V - 2], [0], list(range(g0, g0 + gs)),
+          [3, g0 + 2], [g0 + 4], [g0 + 4], [g0 + 4], [g0 + 4], [g0 + 4], [g0 + 4], [g0 + 4, V - 9]]
+    B = 2 * len(at)
+    x = rng.normal(0, 2, (B, V)).astype(np.float32)
+    P = [dict(temperature=0.0 if i < len(at) else 0.9, top_k=[40, 0, 700][i % 3], top_p=0.95, top_logprobs=5, seed=i) for i in range(B)]
+    allow = np.ones((B, V), bool)
+    for i in range(B):
+        k = i % len(at)
+        x[i, at[k]] = np.nan
+        if k == 9:
+            x[i, g0 + 5:] = -np.inf                                   # nothing above -inf follows
+        elif k == 10:
+            x[i, g0 + 5:] = np.where(rng.random(V - g0 - 5) < 0.5, 0.0, -0.0)   # ties of both zeros follow
+        elif k == 11:
+            P[i].update(counts=[(g0 + 4, 2), (g0 + 6, 1), (V - 1, 1)], presence=0.5, bias=[(g0 + 7, 20.0), (g0 + 4, 1.0)])
+        elif k == 12:
+            P[i].update(ban=[g0 + 4, g0 + 5])                         # a banned NaN is none
+        elif k == 13:
+            P[i].update(masked=True)
+            allow[i] = rng.random(V) < 0.5
+            allow[i, g0 + 4] = i >= len(at)                           # masked out, and not
+        elif k == 14:
+            x[i, g0 + 4] = np.inf                                     # inf - inf: NaN in y alone
+            P[i].update(bias=[(g0 + 4, -np.inf)])
+        elif k == 15:
+            x[i, :V - 9] += 40.0                                      # larger values in front of it
+    bits = np.zeros((B, (V + 31) // 32), np.uint32)
+    for i in range(B):
+        bits[i] = np.packbits(np.pad(allow[i], (0, -V % 32)), bitorder="little").view(np.uint32)
+    print(f"[case] NaN in a group V={V}", flush=True)
     refs = [oracle_row(x[i], P[i], allow[i] if P[i].get("masked") else None) for i in range(B)]
     errs = compare(x, P, _run_padded(x, P, bits.view(np.int32)), refs=refs)
     assert not errs, "\n".join(errs[:20])

@@ -22,7 +22,7 @@
 //       every finite z when no top-k applies and at most ZS_SMALL_CAP are
 //       finite) from the group maxima that zs_k_scan took over the whole GPU
 //       (rw_groups), or from a masked row's gathered ids. Rows these cannot
-//       serve (narrow rows, T = inf, NaN, lists that would overflow) read
+//       serve (narrow rows, T = inf, lists that would overflow) read
 //       their logits here, keeping the lists in LDS behind a rising
 //       threshold (greedy argmax: the last maximal element, a NaN restarts
 //       the fold, sampler.rs:35-43);
@@ -954,8 +954,8 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 // scan + row kernel against the streaming row kernel (us):
 //   1 x 32000 3 + 24 / 45, 64 x 128256 7 + 32 / 92, 256 x 151936 (half the rows
 //   masked) 23 + 47 / 133, 128 x 151936 masked 11 + 47 / 87.
-// Returns false (uniformly) for rows whose lists would overflow or that hold
-// a NaN: they take the streaming loop of zs_k_row.
+// Returns false (uniformly) for rows whose lists would overflow: they take
+// the streaming loop of zs_k_row.
 // ---------------------------------------------------------------------------
 #define RW_WIDE (2 * RW_BUF)   // keys in the sampler list's place
 #define RW_GOBS (RW_BUF / 2)   // observers listed at most; the listed groups (u16) follow them in LDS
@@ -966,7 +966,7 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 struct rw_gst {
     float omax, ymax, rejf;
     unsigned long long gbest;
-    uint32_t n_o, n_s;
+    uint32_t n_o, n_s, fl;
     bool s_over;
     bool s_drop;   // the sampler's list did not fit and is not kept (k > ZS_KS)
 };
@@ -1198,24 +1198,24 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         kmo = max(kmo, sh.ru[3][w]); kms = max(kms, sh.ru[4][w]);
     }
     to = rw_uni(to); ts = rw_uni(ts); nfin = rw_uni(nfin); kmo = rw_uni(kmo); kms = rw_uni(kms);
-    // (every wave has read sh.ru before a row leaves for the streaming loop,
-    // whose first tile writes there)
-    rw_bar();
-    if (kmo == RW_KNAN || kms == RW_KNAN) return false;
+    // (a NaN in x~ or in y: the observers' or the sampler's list is not needed)
+    const bool xnan = kmo == RW_KNAN, ynan = kms == RW_KNAN;
+    G.fl = (xnan ? ZS_CF_OBS_NAN : 0u) | (ynan ? ZS_CF_Z_NAN : 0u);
+    const bool ol = Ko && !xnan;
     // (too many of a wave's groups at -inf, as under a mask: exactly)
-    if (Ko && to <= kinf) to = rw_kth_key(2 * R.words, ng, Ko);
-    if (smode & 1u) {
+    if (ol && to <= kinf) to = rw_kth_key(2 * R.words, ng, Ko);
+    if ((smode & 1u) && !ynan) {
         if (wide || ts <= kinf) ts = rw_kth_key(2 * R.words + ng, ng, Ks);
     } else if (smode == 2) {
         // every y above -inf, when few enough groups hold one
         G.s_over = nfin > ZS_SMALL_CAP;
         ts = kinf + 1u;
     }
-    const bool sl = (smode & 1u) || (smode == 2 && !G.s_over);   // a sampler list is kept
+    const bool sl = !ynan && ((smode & 1u) || (smode == 2 && !G.s_over));   // a sampler list is kept
     // (-inf is no member of either list here: the observers' -inf entries are
     // added below, the sampler's survivors are above -inf)
-    to = Ko ? max(to, kinf + 1u) : 0xffffffffu;
-    ts = sl ? max(ts, kinf + 1u) : 0xffffffffu;
+    to = max(to, kinf + 1u);
+    ts = max(ts, kinf + 1u);
     RW_T(15);
     // the groups that reach a threshold
     uint32_t rej = 0, n_gl, keep = ~0u, pad = 0u;   // keep: bit e, the observers of group e are listed
@@ -1223,7 +1223,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         rej = 0;
 #pragma unroll
         for (int e = 0; e < RW_GPT; e++) {
-            const uint32_t f = (kx[e] >= to && (keep >> e & 1u) ? 1u : 0u) | (ky[e] >= ts ? 2u : 0u);
+            const uint32_t f = (ol && kx[e] >= to && (keep >> e & 1u) ? 1u : 0u) | (sl && ky[e] >= ts ? 2u : 0u);
             if (!(f & 2u)) rej = max(rej, ky[e]);
             const uint32_t p = rw_wave_reserve(&sh.n_gl, f != 0u);
             if (f && p < RW_GL) gl[p] = (uint16_t)((t + (uint32_t)e * RW_NT) | (f << RW_GF));
@@ -1236,7 +1236,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         // an id at it, and the smallest ids come first); the sampler's list
         // takes the entries above its own and, for the k-th value, Ks places
         // at it (the others count as turned away).
-        if (Ko) {
+        if (ol) {
 #pragma unroll
             for (int e = 0; e < RW_GPT; e++) {
                 const uint32_t c = (uint32_t)__popcll(__ballot(kx[e] == to));
@@ -1258,7 +1258,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
                 if (kx[e] != to || before < Ko) keep |= 1u << e;
             }
         }
-        if ((smode & 1u) && ts > kinf + 1u) pad = ts++;
+        if (sl && (smode & 1u) && ts > kinf + 1u) pad = ts++;
         __syncthreads();
         if (t == 0) sh.n_gl = 0;
         rw_bar();
@@ -1337,7 +1337,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         n_s += Ks;
         rej = max(rej, pad);
     }
-    if (n_o < Ko) {
+    if (ol && n_o < Ko) {
         // fewer than Ko ids above -inf: the smallest ids at -inf follow (at
         // most Ko of the first 64 ids are above it)
         static_assert(2 * ZS_OBS_CAND <= 64, "the first 64 ids hold them");
@@ -1354,31 +1354,68 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         n_o = rw_uni(sh.sel_st[2]);
     }
     if (greedy) {
-        // the last id whose y equals the maximum: in the last group at it
-        uint32_t lg = 0;
+        // the last id whose y equals the maximum: in the last group at it. A
+        // NaN restarts the fold (sampler.rs:35-43): then of the ids after the
+        // last one, in the rest of its group and in the groups past it
+        uint32_t nl = 0;   // the last group with a NaN, plus one
+        if (ynan) {
 #pragma unroll
-        for (int e = 0; e < RW_GPT; e++)
-            if (ky[e] == kms && t + (uint32_t)e * RW_NT < ng) lg = t + (uint32_t)e * RW_NT + 1u;
-        lg = rw_wave_umax(lg);
-        if (zs_lane() == 0) sh.ru[5][wid] = lg;
+            for (int e = 0; e < RW_GPT; e++)
+                if (ky[e] == RW_KNAN) nl = t + (uint32_t)e * RW_NT + 1u;
+            nl = rw_wave_umax(nl);
+            if (zs_lane() == 0) sh.ru[5][wid] = nl;
+            __syncthreads();
+            nl = 0;
+#pragma unroll
+            for (int w = 0; w < RW_NW; w++) nl = max(nl, sh.ru[5][w]);
+            if (wid == 0) {
+                uint32_t w;
+                const uint32_t idx0 = ((nl - 1u) << gs) + 4u * (t & qm);
+                const float4 v = rw_fetch4(R, idx0, w);
+                float x[4], y[4];
+                rw_load4(R, idx0, v, w, x, y, sh);
+                uint32_t L = 0;   // the last NaN's id, plus one
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (y[q] != y[q]) L = idx0 + (uint32_t)q + 1u;
+                L = rw_wave_umax(L);
+                G.gbest = L;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (idx0 + q < L || idx0 + q >= R.V) continue;
+                    const unsigned long long c = ((unsigned long long)zs_total_key(y[q] + 0.0f) << 32) | (idx0 + q + 1);
+                    G.gbest = c > G.gbest ? c : G.gbest;
+                }
+            }
+        }
+        unsigned long long gk = 0;   // the largest maximum of the groups from nl on, and the last group at it, plus one
+#pragma unroll
+        for (int e = 0; e < RW_GPT; e++) {
+            const uint32_t i = t + (uint32_t)e * RW_NT;
+            const unsigned long long c = ((unsigned long long)ky[e] << 32) | (i + 1u);
+            if (i >= nl && i < ng) gk = c > gk ? c : gk;
+        }
+        gk = zs_wave_reduce(gk, [](unsigned long long x, unsigned long long y) { return x > y ? x : y; });
+        if (zs_lane() == 0) sh.rl[wid] = gk;
         __syncthreads();
-        lg = 0;
+        gk = 0;
 #pragma unroll
-        for (int w = 0; w < RW_NW; w++) lg = max(lg, sh.ru[5][w]);
-        const uint32_t idx0 = ((lg - 1u) << gs) + 4u * t;
-        if (4u * t < 1u << gs) {
+        for (int w = 0; w < RW_NW; w++) gk = sh.rl[w] > gk ? sh.rl[w] : gk;
+        if (gk && t <= qm) {
+            const uint32_t idx0 = (((uint32_t)gk - 1u) << gs) + 4u * t;
             uint32_t w;
             const float4 v = rw_fetch4(R, idx0, w);
             float x[4], y[4];
             rw_load4(R, idx0, v, w, x, y, sh);
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (idx0 + q < R.V && zs_total_key(y[q] + 0.0f) == kms)
-                    G.gbest = ((unsigned long long)kms << 32) | (idx0 + q + 1);
+            for (int q = 0; q < 4; q++) {
+                const unsigned long long c = (gk & 0xffffffff00000000ull) | (idx0 + q + 1);
+                if (idx0 + q < R.V && zs_total_key(y[q] + 0.0f) == (uint32_t)(gk >> 32)) G.gbest = c > G.gbest ? c : G.gbest;
+            }
         }
     }
-    G.omax = zs_key_to_float(kmo);
-    G.ymax = zs_key_to_float(kms);
+    G.omax = xnan ? -INFINITY : zs_key_to_float(kmo);
+    G.ymax = ynan ? -INFINITY : zs_key_to_float(kms);
     G.rejf = rej > kinf ? zs_key_to_float(rej) : -INFINITY;
     G.n_o = n_o;
     G.n_s = n_s;
@@ -1579,11 +1616,11 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     bool fast = false;
     if (!gath && has_groups) {
         if (Ks > ZS_KS && !rw_wide_fits(Ks, (V + (1u << a.gshift) - 1u) >> a.gshift)) { smode = 0; Ks = 0; }
-        rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, false, false};
+        rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, 0u, false, false};
         fast = rw_groups(a, r, R, greedy, smode, Ks, Ko, G);
         if (fast) {
             omax = G.omax; ymax = G.ymax; rejf = G.rejf; gbest = G.gbest;
-            n_o = G.n_o; n_s = G.n_s; s_over = G.s_over;
+            n_o = G.n_o; n_s = G.n_s; fl = G.fl; s_over = G.s_over;
         }
         if ((!fast && Ks > ZS_KS) || G.s_drop) { smode = 0; Ks = 0; }
     }
