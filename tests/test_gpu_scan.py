@@ -239,3 +239,35 @@ def test_nan_in_a_group(V):
     refs = [oracle_row(x[i], P[i], allow[i] if P[i].get("masked") else None) for i in range(B)]
     errs = compare(x, P, _run_padded(x, P, bits.view(np.int32)), refs=refs)
     assert not errs, "\n".join(errs[:20])
+
+
+@pytest.mark.parametrize("V", [4096, 8193, 50257, 128256])
+def test_infinite_temperature(V):
+    """y / inf is 0 of a finite y and NaN of an infinite one, wherever in the
+    row it lies: none, one at either end, in a masked, banned, biased or
+    unbanned place; k of every kind of list."""
+    rng = np.random.default_rng(V)
+    B = 18
+    x = rng.normal(0, 2, (B, V)).astype(np.float32)
+    P = [dict(temperature=float("inf"), top_k=k, top_p=0.9, top_logprobs=5, seed=i)
+         for i, k in enumerate([0, 1, 40, 128, 300, 600, V // 5, V - 1] + [40] * (B - 8))]
+    allow = np.ones((B, V), bool)
+    x[8, V - 1] = -np.inf
+    x[9, 0] = -np.inf
+    x[10, V // 2] = np.inf
+    P[11].update(masked=True)                                         # masked, every id allowed
+    P[12].update(masked=True)
+    allow[12, V - 2] = False
+    P[13].update(ban=[V // 3])
+    P[14].update(bias=[(V // 3, -np.inf)], top_k=0)
+    x[15, 7] = np.inf
+    P[15].update(bias=[(7, -np.inf)])                                 # inf - inf
+    P[16].update(counts=[(int(t), 2) for t in rng.choice(V, 300, replace=False)], repeat=1.2)
+    x[17] = -1.0
+    bits = np.zeros((B, (V + 31) // 32), np.uint32)
+    for i in range(B):
+        bits[i] = np.packbits(np.pad(allow[i], (0, -V % 32)), bitorder="little").view(np.uint32)
+    print(f"[case] T = inf V={V}", flush=True)
+    refs = [oracle_row(x[i], P[i], allow[i] if P[i].get("masked") else None) for i in range(B)]
+    errs = compare(x, P, _run_padded(x, P, bits.view(np.int32)), refs=refs)
+    assert not errs, "\n".join(errs[:20])

@@ -22,7 +22,7 @@
 //       every finite z when no top-k applies and at most ZS_SMALL_CAP are
 //       finite) from the group maxima that zs_k_scan took over the whole GPU
 //       (rw_groups), or from a masked row's gathered ids. Rows these cannot
-//       serve (narrow rows, T = inf, lists that would overflow) read
+//       serve (narrow rows, long patch lists, lists that would overflow) read
 //       their logits here, keeping the lists in LDS behind a rising
 //       threshold (greedy argmax: the last maximal element, a NaN restarts
 //       the fold, sampler.rs:35-43);
@@ -1094,8 +1094,8 @@ __device__ __noinline__ uint32_t rw_kth_key(uint32_t off, uint32_t n, uint32_t K
     return pre;
 }
 
-__device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const rw_row& R, bool greedy, uint32_t smode,
-                                       uint32_t Ks, uint32_t Ko, rw_gst& G) {
+__device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const rw_row& R, bool greedy, bool tinf,
+                                          uint32_t smode, uint32_t Ks, uint32_t Ko, rw_gst& G) {
     rw_shared& sh = rw_sh;
     const uint32_t t = threadIdx.x, wid = (uint32_t)zs_wid();
     const uint32_t gs = a.gshift, ng = (R.V + (1u << gs) - 1u) >> gs;
@@ -1414,6 +1414,26 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
             }
         }
     }
+    if (tinf) {
+        // y / inf is NaN for y = +-inf, which the maxima do not tell: one more
+        // read of the row, without lists
+        bool bad = false;
+        for (uint32_t i0 = 4u * t; i0 < R.V; i0 += NU * 4u * RW_NT) {
+            float4 v[NU];
+            uint32_t w[NU];
+#pragma unroll
+            for (int u = 0; u < NU; u++) v[u] = rw_fetch4(R, i0 + (uint32_t)u * 4u * RW_NT, w[u]);
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const uint32_t idx0 = i0 + (uint32_t)u * 4u * RW_NT;
+                float x[4], y[4];
+                rw_load4(R, idx0, v[u], w[u], x, y, sh);
+#pragma unroll
+                for (int q = 0; q < 4; q++) bad |= idx0 + q < R.V && (y[q] == INFINITY || y[q] == -INFINITY);
+            }
+        }
+        if (bad) G.fl |= ZS_CF_Z_NAN;
+    }
     G.omax = xnan ? -INFINITY : zs_key_to_float(kmo);
     G.ymax = ynan ? -INFINITY : zs_key_to_float(kms);
     G.rejf = rej > kinf ? zs_key_to_float(rej) : -INFINITY;
@@ -1547,7 +1567,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     // small-survivor check when no top-k applies), 0 = none; from the group
     // maxima also larger k: 1 while the survivors fit the small path, 3 (the
     // keys only, for the threshold) as far as rw_wide_fits
-    const bool has_groups = a.gshift && !tinf && R.np <= ZS_PATCH_LDS;
+    const bool has_groups = a.gshift && R.np <= ZS_PATCH_LDS;
     const uint32_t kmax1 = has_groups ? (uint32_t)ZS_SMALL_CAP - 1u : (uint32_t)ZS_KS;
     uint32_t smode = greedy ? 0u : (!has_topk ? 2u : P.top_k <= kmax1 ? 1u : has_groups ? 3u : 0u);
     uint32_t Ks = (smode & 1u) ? P.top_k : 0u;
@@ -1617,7 +1637,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     if (!gath && has_groups) {
         if (Ks > ZS_KS && !rw_wide_fits(Ks, (V + (1u << a.gshift) - 1u) >> a.gshift)) { smode = 0; Ks = 0; }
         rw_gst G = {omax, ymax, rejf, 0ull, 0u, 0u, 0u, false, false};
-        fast = rw_groups(a, r, R, greedy, smode, Ks, Ko, G);
+        fast = rw_groups(a, r, R, greedy, tinf, smode, Ks, Ko, G);
         if (fast) {
             omax = G.omax; ymax = G.ymax; rejf = G.rejf; gbest = G.gbest;
             n_o = G.n_o; n_s = G.n_s; fl = G.fl; s_over = G.s_over;
