@@ -145,16 +145,19 @@ def test_wide_top_k(V, ks):
 
 def test_wide_top_k_lists_that_overflow():
     """More values at the threshold than the sampler's list holds, with the
-    observers' candidates above them: k up to 128 streams the row, larger k keep
-    the observers' list alone; without observers nothing else is listed."""
+    observers' candidates above them (rows 0 to 4) or among them: k up to 128
+    takes the ones above and the k-th, larger k keep the observers' list alone;
+    without observers nothing else is listed."""
     V = 50257
     rng = np.random.default_rng(8)
-    P = [dict(temperature=1.0, top_k=k, top_p=0.9, top_logprobs=20, seed=i) for i, k in enumerate((100, 300, 511, 700, 300))]
+    P = [dict(temperature=1.0, top_k=k, top_p=0.9, top_logprobs=20, seed=i)
+         for i, k in enumerate((100, 300, 511, 700, 300, 60, 61, 20, 128))]
     P[4].update(logprobs=False, detect_hallucination=False, top_logprobs=0)
     x = rng.normal(0, 1, (len(P), V)).astype(np.float32)
     for i in range(len(P)):
         x[i, 16 * 1000:16 * 1400] = 9.0                       # 400 groups of 16 equal values
-        x[i, rng.choice(16000, 60, replace=False)] = rng.uniform(10, 12, 60).astype(np.float32)
+        n = 60 if i < 7 else 5
+        x[i, rng.choice(16000, n, replace=False)] = rng.uniform(10, 12, n).astype(np.float32)
     print("[case] wide top-k overflow", flush=True)
     errs = compare(x, P, _run_padded(x, P))
     assert not errs, "\n".join(errs)

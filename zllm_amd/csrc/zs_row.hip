@@ -961,7 +961,7 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 #define RW_GOBS (RW_BUF / 2)   // observers listed at most; the listed groups (u16) follow them in LDS
 #define RW_GL (RW_BUF * 2)     // listed groups at most
 #define RW_GF 14u              // a listed group: group | list flags << RW_GF
-#define RW_GTIES 1024          // groups listed beyond k at most without a look at the ties among them
+#define RW_GTIES 1024          // groups listed beyond k at most without a cut of the ties among them
 #define RW_GPT 10          // groups per thread at most (zs_scan_gshift)
 struct rw_gst {
     float omax, ymax, rejf;
@@ -1217,9 +1217,12 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     to = max(to, kinf + 1u);
     ts = max(ts, kinf + 1u);
     RW_T(15);
-    // the groups that reach a threshold
-    uint32_t rej = 0, n_gl, keep = ~0u, pad = 0u;   // keep: bit e, the observers of group e are listed
+    uint32_t* wk = reinterpret_cast<uint32_t*>(sh.u.b.s);
+    const uint32_t scap = smode == 3 ? (uint32_t)RW_WIDE : smode == 2 ? (uint32_t)ZS_SMALL_CAP : (uint32_t)RW_BUF;
+    constexpr int NU = 4;
+    uint32_t rej, n_gl, n_o, n_s, keep = ~0u, pad = 0u;   // keep: bit e, the observers of group e are listed
     for (bool cut = false;; cut = true) {
+        // the groups that reach a threshold
         rej = 0;
 #pragma unroll
         for (int e = 0; e < RW_GPT; e++) {
@@ -1230,13 +1233,72 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         }
         __syncthreads();
         n_gl = rw_uni(sh.n_gl);
-        if (cut || n_gl <= RW_GTIES + Ks) break;
-        // Many groups at a threshold: a row of few distinct values. Of the
-        // observers' groups at theirs only the first Ko are needed (each holds
-        // an id at it, and the smallest ids come first); the sampler's list
-        // takes the entries above its own and, for the k-th value, Ks places
-        // at it (the others count as turned away).
+        const uint32_t nit = cut || n_gl <= RW_GTIES + Ks ? min(n_gl, (uint32_t)RW_GL) << qs : 0u;
+        for (uint32_t i0 = 0; i0 < nit; i0 += NU * RW_NT) {
+            float4 v[NU];
+            uint32_t w[NU], ge[NU];
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const uint32_t i = i0 + t + (uint32_t)u * RW_NT;
+                ge[u] = gl[min(i, nit - 1u) >> qs];
+                if (i >= nit) ge[u] &= (1u << RW_GF) - 1u;
+                v[u] = rw_fetch4(R, ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * (i & qm), w[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const uint32_t f = ge[u] >> RW_GF;
+                const uint32_t idx0 = ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * ((i0 + t + (uint32_t)u * RW_NT) & qm);
+                float x[4], y[4];
+                rw_load4(R, idx0, v[u], w[u], x, y, sh);
+                // (thresholds are keys of group maxima: compared with -0 as +0, the
+                // sampler's entries themselves in total order as Rust sorts them)
+                uint32_t kxq[4], kyq[4], mo4 = 0, ms4 = 0;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    kxq[q] = zs_total_key(x[q] + 0.0f);
+                    kyq[q] = zs_total_key(y[q] + 0.0f);
+                    mo4 |= (f & 1u) && kxq[q] >= to ? 1u << q : 0u;
+                    const bool in = (f & 2u) && kyq[q] >= ts;
+                    ms4 |= in ? 1u << q : 0u;
+                    if (f && !in) rej = max(rej, kyq[q]);
+                }
+                if (__ballot(mo4 != 0u)) {
+                    uint32_t p = rw_wave_reserve_n(&sh.sel_st[2], (uint32_t)__popc(mo4));
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        if (!((mo4 >> q) & 1u)) continue;
+                        if (p < RW_GOBS) sh.u.b.o[p] = ((unsigned long long)(~kxq[q]) << 32) | (idx0 + q);
+                        p++;
+                    }
+                }
+                if (__ballot(ms4 != 0u)) {
+                    uint32_t p = rw_wave_reserve_n(&sh.sel_st[3], (uint32_t)__popc(ms4));
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        if (!((ms4 >> q) & 1u)) continue;
+                        if (p < scap) {
+                            if (smode == 3) wk[p] = kyq[q];
+                            else sh.u.b.s[p] = ((unsigned long long)(~zs_total_key(y[q])) << 32) | (idx0 + q);
+                        }
+                        p++;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        n_o = rw_uni(sh.sel_st[2]);
+        n_s = rw_uni(sh.sel_st[3]);
+        __syncthreads();   // (the counts are read before they change below)
+        const bool many = n_gl > RW_GTIES + Ks || (smode == 1 && Ks <= ZS_KS && n_s > scap);
+        if (cut || !(many || n_o > RW_GOBS)) break;
+        // Many groups, or many ids, from a threshold on: a row of few distinct
+        // values or with a run of equal ones. The thresholds are taken exactly
+        // then. Of the observers' groups at theirs only the first Ko are
+        // needed (each holds an id at it, and the smallest ids come first);
+        // the sampler's list takes the entries above its own and, for the
+        // k-th value, Ks places at it (the others count as turned away).
         if (ol) {
+            to = max(rw_kth_key(2 * R.words, ng, Ko), kinf + 1u);
 #pragma unroll
             for (int e = 0; e < RW_GPT; e++) {
                 const uint32_t c = (uint32_t)__popcll(__ballot(kx[e] == to));
@@ -1258,72 +1320,15 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
                 if (kx[e] != to || before < Ko) keep |= 1u << e;
             }
         }
-        if (sl && (smode & 1u) && ts > kinf + 1u) pad = ts++;
+        if (many && sl && (smode & 1u)) {
+            ts = max(rw_kth_key(2 * R.words + ng, ng, Ks), kinf + 1u);
+            if (ts > kinf + 1u) pad = ts++;
+        }
         __syncthreads();
-        if (t == 0) sh.n_gl = 0;
+        if (t == 0) { sh.n_gl = 0; sh.sel_st[2] = 0; sh.sel_st[3] = 0; }
         rw_bar();
     }
-    if (n_gl > RW_GL) return false;
-    const uint32_t nit = n_gl << qs;
-    uint32_t* wk = reinterpret_cast<uint32_t*>(sh.u.b.s);
-    const uint32_t scap = smode == 3 ? (uint32_t)RW_WIDE : smode == 2 ? (uint32_t)ZS_SMALL_CAP : (uint32_t)RW_BUF;
-    constexpr int NU = 4;
-    for (uint32_t i0 = 0; i0 < nit; i0 += NU * RW_NT) {
-        float4 v[NU];
-        uint32_t w[NU], ge[NU];
-#pragma unroll
-        for (int u = 0; u < NU; u++) {
-            const uint32_t i = i0 + t + (uint32_t)u * RW_NT;
-            ge[u] = gl[min(i, nit - 1u) >> qs];
-            if (i >= nit) ge[u] &= (1u << RW_GF) - 1u;
-            v[u] = rw_fetch4(R, ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * (i & qm), w[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < NU; u++) {
-            const uint32_t f = ge[u] >> RW_GF;
-            const uint32_t idx0 = ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * ((i0 + t + (uint32_t)u * RW_NT) & qm);
-            float x[4], y[4];
-            rw_load4(R, idx0, v[u], w[u], x, y, sh);
-            // (thresholds are keys of group maxima: compared with -0 as +0, the
-            // sampler's entries themselves in total order as Rust sorts them)
-            uint32_t kxq[4], kyq[4], mo4 = 0, ms4 = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                kxq[q] = zs_total_key(x[q] + 0.0f);
-                kyq[q] = zs_total_key(y[q] + 0.0f);
-                mo4 |= (f & 1u) && kxq[q] >= to ? 1u << q : 0u;
-                const bool in = (f & 2u) && kyq[q] >= ts;
-                ms4 |= in ? 1u << q : 0u;
-                if (f && !in) rej = max(rej, kyq[q]);
-            }
-            if (__ballot(mo4 != 0u)) {
-                uint32_t p = rw_wave_reserve_n(&sh.sel_st[2], (uint32_t)__popc(mo4));
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    if (!((mo4 >> q) & 1u)) continue;
-                    if (p < RW_GOBS) sh.u.b.o[p] = ((unsigned long long)(~kxq[q]) << 32) | (idx0 + q);
-                    p++;
-                }
-            }
-            if (__ballot(ms4 != 0u)) {
-                uint32_t p = rw_wave_reserve_n(&sh.sel_st[3], (uint32_t)__popc(ms4));
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    if (!((ms4 >> q) & 1u)) continue;
-                    if (p < scap) {
-                        if (smode == 3) wk[p] = kyq[q];
-                        else sh.u.b.s[p] = ((unsigned long long)(~zs_total_key(y[q])) << 32) | (idx0 + q);
-                    }
-                    p++;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    uint32_t n_o = rw_uni(sh.sel_st[2]);
-    uint32_t n_s = rw_uni(sh.sel_st[3]);
-    __syncthreads();   // (the count is read before the ids at -inf are added to it)
-    if (n_o > RW_GOBS) return false;
+    if (n_gl > RW_GL || n_o > RW_GOBS) return false;
     if ((smode & 1u) && n_s + (pad ? Ks : 0u) > scap) {
         // (the streaming loop would list no k > ZS_KS either)
         if (Ks <= ZS_KS) return false;
