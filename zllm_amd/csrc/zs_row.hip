@@ -72,10 +72,10 @@ struct rw_shared {
     float fthr[2];                  // candidate thresholds as values
     float fcut[2];                  // largest values cut from the lists
     unsigned long long rl[RW_NW];
+    unsigned long long n_os;        // rw_groups: entries of the observers' list | of the sampler's << 32
     uint32_t n_surv, tok;
     uint32_t n_gl;                  // groups listed by rw_groups
     uint32_t ovf[3];                // first tile that lost a list entry, per group slot
-    uint32_t thr_o, thr_s;          // candidate admission thresholds (keys)
     float fsh;
     uint32_t sel_hist[2][256];      // list selection: digit histogram (double buffered)
     uint32_t sel_mm[3][RW_NW];      // list selection: per-wave member count, key min / max
@@ -1005,21 +1005,22 @@ __device__ __forceinline__ uint32_t rw_lanes_umax(uint32_t v, uint32_t qs) {
 #define RW_KNAN 0xffffffffu
 __device__ __forceinline__ uint32_t rw_gkey(float m, bool nan) { return nan ? RW_KNAN : zs_total_key(m + 0.0f); }
 
-// Places behind a counter for the lanes' entries, one atomic per wave (one per
-// lane is served lane by lane: a row of equal values spent 350 us on 64 K of
-// them). Called by whole waves.
-__device__ __forceinline__ uint32_t rw_wave_reserve(uint32_t* ctr, bool one) {
-    const unsigned long long m = __ballot(one);
-    uint32_t p = 0;
-    if (m && zs_lane() == 0) p = atomicAdd(ctr, (uint32_t)__popcll(m));
-    p = (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, p));
-}
-__device__ __forceinline__ uint32_t rw_wave_reserve_n(uint32_t* ctr, uint32_t n) {
+// Places behind a counter for n entries of each lane, one atomic per wave (one
+// per lane is served lane by lane: a row of equal values spent 350 us on 64 K
+// of them). Called by whole waves.
+__device__ __forceinline__ uint32_t rw_wave_reserve(uint32_t* ctr, uint32_t n) {
     const uint32_t inc = rw_wave_scan(n);
     uint32_t p = 0;
     if (zs_lane() == 63) p = atomicAdd(ctr, inc);
     return (uint32_t)__builtin_amdgcn_readlane((int)p, 63) + inc - n;
+}
+// The same behind both halves of a counter, for at most 64 K entries of a wave each.
+__device__ __forceinline__ void rw_wave_reserve2(unsigned long long* ctr, uint32_t n0, uint32_t n1, uint32_t& p0, uint32_t& p1) {
+    const uint32_t n = n0 | (n1 << 16), inc = rw_wave_scan(n);
+    unsigned long long p = 0;
+    if (zs_lane() == 63) p = atomicAdd(ctr, (unsigned long long)(inc & 0xffffu) | ((unsigned long long)(inc >> 16) << 32));
+    p0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)p, 63) + (inc & 0xffffu) - n0;
+    p1 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(p >> 32), 63) + (inc >> 16) - n1;
 }
 
 // x~ and y of the 4 ids from idx0 (a multiple of 4; ids >= V read -inf).
@@ -1094,6 +1095,37 @@ __device__ __noinline__ uint32_t rw_kth_key(uint32_t off, uint32_t n, uint32_t K
     return pre;
 }
 
+// Of the n group maxima at offset `off` of the dynamic LDS, this thread's
+// (t, t + RW_NT, ...: bit e) that are not `key` or among the first K equal to
+// it. Called by every thread.
+__device__ __noinline__ uint32_t rw_first_ties(uint32_t off, uint32_t n, uint32_t key, uint32_t K) {
+    rw_shared& sh = rw_sh;
+    const uint32_t t = threadIdx.x, wid = (uint32_t)zs_wid();
+    auto tied = [&](uint32_t e) {
+        const uint32_t i = t + e * RW_NT;
+        return __ballot(i < n && rw_pbits[off + min(i, n - 1u)] == key);
+    };
+    for (uint32_t e = 0; e < RW_GPT; e++) {
+        const uint32_t c = (uint32_t)__popcll(tied(e));
+        if (zs_lane() == 0) sh.sel_hist[0][e * RW_NW + wid] = c;
+    }
+    rw_bar();
+    uint32_t run = 0, keep = ~0u;
+    for (uint32_t e = 0; e < RW_GPT; e++) {
+        const unsigned long long m = tied(e);
+        uint32_t before = run;
+        for (uint32_t w = 0; w < RW_NW; w++) {
+            const uint32_t c = sh.sel_hist[0][e * RW_NW + w];
+            before += w < wid ? c : 0u;
+            run += c;
+        }
+        before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, before));
+        if ((m >> zs_lane() & 1ull) && before >= K) keep &= ~(1u << e);
+    }
+    rw_bar();
+    return keep;
+}
+
 __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const rw_row& R, bool greedy, bool tinf,
                                           uint32_t smode, uint32_t Ks, uint32_t Ko, rw_gst& G) {
     rw_shared& sh = rw_sh;
@@ -1116,7 +1148,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
             if (i < ng) { gx[i] = k[e]; gy[i] = k[e]; }
         }
     }
-    if (t == 0) { sh.n_gl = 0; sh.sel_n = 0; sh.sel_st[2] = 0; sh.sel_st[3] = 0; }
+    if (t == 0) { sh.n_gl = 0; sh.n_os = 0; }
     __syncthreads();
     // groups with patched ids are read again: the first patch of a group lists
     // it, then one lane per 4 ids (the lanes of a group adjacent)
@@ -1166,12 +1198,18 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     RW_T(6);
     // this thread's groups t, t + RW_NT, ...
     uint32_t kx[RW_GPT], ky[RW_GPT], mo = 0, ms = 0, fin = 0;
+    auto load_groups = [&]() {
+#pragma unroll
+        for (int e = 0; e < RW_GPT; e++) {
+            const uint32_t i = t + (uint32_t)e * RW_NT, ic = min(i, ng - 1u);
+            kx[e] = gx[ic];
+            ky[e] = gy[ic];
+            if (i >= ng) kx[e] = ky[e] = 0u;
+        }
+    };
+    load_groups();
 #pragma unroll
     for (int e = 0; e < RW_GPT; e++) {
-        const uint32_t i = t + (uint32_t)e * RW_NT, ic = min(i, ng - 1u);
-        kx[e] = gx[ic];
-        ky[e] = gy[ic];
-        if (i >= ng) kx[e] = ky[e] = 0u;
         mo = max(mo, kx[e]);
         ms = max(ms, ky[e]);
         fin += ky[e] > kinf ? 1u : 0u;
@@ -1223,13 +1261,21 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
     uint32_t rej, n_gl, n_o, n_s, keep = ~0u, pad = 0u;   // keep: bit e, the observers of group e are listed
     for (bool cut = false;; cut = true) {
         // the groups that reach a threshold
+        uint32_t fl2 = 0, n = 0;
         rej = 0;
+        static_assert(2 * RW_GPT <= 32, "two bits per group of a thread");
 #pragma unroll
         for (int e = 0; e < RW_GPT; e++) {
             const uint32_t f = (ol && kx[e] >= to && (keep >> e & 1u) ? 1u : 0u) | (sl && ky[e] >= ts ? 2u : 0u);
             if (!(f & 2u)) rej = max(rej, ky[e]);
-            const uint32_t p = rw_wave_reserve(&sh.n_gl, f != 0u);
-            if (f && p < RW_GL) gl[p] = (uint16_t)((t + (uint32_t)e * RW_NT) | (f << RW_GF));
+            fl2 |= f << (2 * e);
+            n += f ? 1u : 0u;
+        }
+        uint32_t p = rw_wave_reserve(&sh.n_gl, n);
+        for (; fl2; p++) {
+            const uint32_t e = (uint32_t)__builtin_ctz(fl2) >> 1, f = fl2 >> (2 * e) & 3u;
+            fl2 &= ~(3u << (2 * e));
+            if (p < RW_GL) gl[p] = (uint16_t)((t + e * RW_NT) | (f << RW_GF));
         }
         __syncthreads();
         n_gl = rw_uni(sh.n_gl);
@@ -1247,6 +1293,7 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
 #pragma unroll
             for (int u = 0; u < NU; u++) {
                 const uint32_t f = ge[u] >> RW_GF;
+                if (!__ballot(f != 0u)) continue;   // (past the last item)
                 const uint32_t idx0 = ((ge[u] & ((1u << RW_GF) - 1u)) << gs) + 4u * ((i0 + t + (uint32_t)u * RW_NT) & qm);
                 float x[4], y[4];
                 rw_load4(R, idx0, v[u], w[u], x, y, sh);
@@ -1262,32 +1309,28 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
                     ms4 |= in ? 1u << q : 0u;
                     if (f && !in) rej = max(rej, kyq[q]);
                 }
-                if (__ballot(mo4 != 0u)) {
-                    uint32_t p = rw_wave_reserve_n(&sh.sel_st[2], (uint32_t)__popc(mo4));
+                if (!__ballot((mo4 | ms4) != 0u)) continue;
+                uint32_t po, ps;
+                rw_wave_reserve2(&sh.n_os, (uint32_t)__popc(mo4), (uint32_t)__popc(ms4), po, ps);
 #pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        if (!((mo4 >> q) & 1u)) continue;
-                        if (p < RW_GOBS) sh.u.b.o[p] = ((unsigned long long)(~kxq[q]) << 32) | (idx0 + q);
-                        p++;
+                for (int q = 0; q < 4; q++) {
+                    if ((mo4 >> q) & 1u) {
+                        if (po < RW_GOBS) sh.u.b.o[po] = ((unsigned long long)(~kxq[q]) << 32) | (idx0 + q);
+                        po++;
                     }
-                }
-                if (__ballot(ms4 != 0u)) {
-                    uint32_t p = rw_wave_reserve_n(&sh.sel_st[3], (uint32_t)__popc(ms4));
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        if (!((ms4 >> q) & 1u)) continue;
-                        if (p < scap) {
-                            if (smode == 3) wk[p] = kyq[q];
-                            else sh.u.b.s[p] = ((unsigned long long)(~zs_total_key(y[q])) << 32) | (idx0 + q);
+                    if ((ms4 >> q) & 1u) {
+                        if (ps < scap) {
+                            if (smode == 3) wk[ps] = kyq[q];
+                            else sh.u.b.s[ps] = ((unsigned long long)(~zs_total_key(y[q])) << 32) | (idx0 + q);
                         }
-                        p++;
+                        ps++;
                     }
                 }
             }
         }
         __syncthreads();
-        n_o = rw_uni(sh.sel_st[2]);
-        n_s = rw_uni(sh.sel_st[3]);
+        n_o = rw_uni((uint32_t)sh.n_os);
+        n_s = rw_uni((uint32_t)(sh.n_os >> 32));
         __syncthreads();   // (the counts are read before they change below)
         const bool many = n_gl > RW_GTIES + Ks || (smode == 1 && Ks <= ZS_KS && n_s > scap);
         if (cut || !(many || n_o > RW_GOBS)) break;
@@ -1299,34 +1342,16 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
         // k-th value, Ks places at it (the others count as turned away).
         if (ol) {
             to = max(rw_kth_key(2 * R.words, ng, Ko), kinf + 1u);
-#pragma unroll
-            for (int e = 0; e < RW_GPT; e++) {
-                const uint32_t c = (uint32_t)__popcll(__ballot(kx[e] == to));
-                if (zs_lane() == 0) sh.sel_hist[0][(uint32_t)e * RW_NW + wid] = c;
-            }
-            rw_bar();
-            uint32_t run = 0;
-            keep = 0;
-#pragma unroll
-            for (int e = 0; e < RW_GPT; e++) {
-                const unsigned long long m = __ballot(kx[e] == to);
-                uint32_t before = run;
-                for (uint32_t w = 0; w < RW_NW; w++) {
-                    const uint32_t c = sh.sel_hist[0][(uint32_t)e * RW_NW + w];
-                    before += w < wid ? c : 0u;
-                    run += c;
-                }
-                before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, before));
-                if (kx[e] != to || before < Ko) keep |= 1u << e;
-            }
+            keep = rw_first_ties(2 * R.words, ng, to, Ko);
         }
         if (many && sl && (smode & 1u)) {
             ts = max(rw_kth_key(2 * R.words + ng, ng, Ks), kinf + 1u);
             if (ts > kinf + 1u) pad = ts++;
         }
         __syncthreads();
-        if (t == 0) { sh.n_gl = 0; sh.sel_st[2] = 0; sh.sel_st[3] = 0; }
+        if (t == 0) { sh.n_gl = 0; sh.n_os = 0; }
         rw_bar();
+        load_groups();   // (again: no registers are held for them meanwhile)
     }
     if (n_gl > RW_GL || n_o > RW_GOBS) return false;
     if ((smode & 1u) && n_s + (pad ? Ks : 0u) > scap) {
@@ -1353,10 +1378,10 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
             float x[4], y[4];
             rw_load4(R, idx0, v, w, x, y, sh);
             const float xi = (t & 3u) == 0 ? x[0] : (t & 3u) == 1 ? x[1] : (t & 3u) == 2 ? x[2] : x[3];
-            if (t < R.V && xi == -INFINITY) sh.u.b.o[atomicAdd(&sh.sel_st[2], 1u)] = ((unsigned long long)(~kinf) << 32) | t;
+            if (t < R.V && xi == -INFINITY) sh.u.b.o[atomicAdd(reinterpret_cast<uint32_t*>(&sh.n_os), 1u)] = ((unsigned long long)(~kinf) << 32) | t;
         }
         __syncthreads();
-        n_o = rw_uni(sh.sel_st[2]);
+        n_o = rw_uni((uint32_t)sh.n_os);
     }
     if (greedy) {
         // the last id whose y equals the maximum: in the last group at it. A
