@@ -53,3 +53,38 @@ def test_btopk_of_no_ids():
     assert call(65) == 0
     torch.cuda.synchronize()
     assert (idxs == -1).all() and (vals < -2.9e38).all()
+
+
+@pytest.mark.parametrize("V", [3000, 20000, 128256, 163841])
+@pytest.mark.parametrize("K", [1, 40, 64])
+def test_btopk_many_groups_or_ids(V, K):
+    """Rows where more groups or ids than the lists hold reach the first key
+    taken: cut to the first K groups, quads and ids by (key desc, id asc)."""
+    from tests.gpu_util import ctx
+    from zllm_amd.engine import lane_topk
+    rng = np.random.default_rng(V + K)
+    n = 10
+    x = rng.normal(0, 2, (n, V)).astype(np.float32)
+    x[0].sort()
+    x[1] = np.sort(x[1])[::-1]
+    x[2] = np.round(x[2] * 2) / 2                              # ties within and across groups
+    x[3, rng.choice(V, 700, replace=False)] = 11.0             # 700 equal maxima, spread
+    x[4, rng.choice(V, 63, replace=False)] = rng.uniform(12, 13, 63).astype(np.float32)
+    x[4, V // 5:V // 5 + 1500] = 11.0                          # 63 above a run of equal values
+    x[5] = np.sort(x[5])
+    x[5, -1500::2] = np.nan                                    # candidates and others in turn
+    x[6] = rng.integers(0, 2, V).astype(np.float32)
+    x[7] = -np.inf
+    x[7, V // 3:V // 3 + 40] = 5.0                             # fewer candidates than K, all equal
+    x[8, :600] = np.linspace(20, 30, 600, dtype=np.float32)    # the first groups, ascending
+    x[9, -1200:] = 3.0e38                                      # beyond the candidates' range
+    x[9, -1200:-100:3] = 2.9e38
+    print(f"[case] btopk many V={V} K={K}", flush=True)
+    xs = torch.zeros((n, (V + 3) // 4 * 4), device="cuda")
+    xs[:, :V] = torch.from_numpy(x)
+    vals, idxs = lane_topk(ctx(64, max(151936, V)), xs[:, :V], K)
+    vals, idxs = vals.cpu().numpy(), idxs.cpu().numpy().view(np.uint32)
+    for s in range(n):
+        ov, oi = O.btopk(x[s], K)
+        assert idxs[s].tolist() == oi.tolist(), s
+        assert vals[s].tobytes() == ov.tobytes(), s

@@ -270,22 +270,26 @@ __global__ void zs_k_bsample_fin(unsigned long long* keys, uint32_t B, uint32_t*
 __device__ __forceinline__ bool tk_cand(float v) { return v >= -3.0e38f && v < 3.0e38f; }
 __device__ __forceinline__ uint32_t tk_key(float v) { return zs_total_key(v == 0.0f ? 0.0f : v); }
 
-// By an NT-thread workgroup over its row, six passes (buf: KMAX >= K entries).
-template <int NT, int KMAX>
-__device__ __forceinline__ void tk_row_radix(const float* row, uint32_t V, uint32_t K, float* vals, uint32_t* idxs,
-                                             unsigned long long* buf, uint32_t* hist, uint32_t* u, uint32_t* scan_sh) {
+__global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
+                                                     float* vals, uint32_t* idxs) {
+    __shared__ uint32_t hist[256];
+    __shared__ uint32_t u[4];
+    __shared__ unsigned long long buf[TK_MAX];
+    __shared__ uint32_t scan_sh[LN_NT / 64];
+    const uint32_t r = blockIdx.x;
     const int t = threadIdx.x;
+    const float* row = logits + (size_t)r * ld;
     // radix select of the K-th largest candidate key
     uint32_t ncand = 0;
-    for (uint32_t i = t; i < V; i += NT) ncand += tk_cand(row[i]) ? 1u : 0u;
-    ncand = block_sum_u<NT>(ncand, scan_sh);
+    for (uint32_t i = t; i < V; i += LN_NT) ncand += tk_cand(row[i]) ? 1u : 0u;
+    ncand = block_sum_u<LN_NT>(ncand, scan_sh);
     const uint32_t KK = ncand < K ? ncand : K;
     uint32_t prefix = 0, mask = 0, need = KK;
     if (KK > 0) {
         for (int shift = 24; shift >= 0; shift -= 8) {
-            for (int i = t; i < 256; i += NT) hist[i] = 0;
+            if (t < 256) hist[t] = 0;
             __syncthreads();
-            for (uint32_t i = t; i < V; i += NT) {
+            for (uint32_t i = t; i < V; i += LN_NT) {
                 float v = row[i];
                 if (!tk_cand(v)) continue;
                 uint32_t k = tk_key(v);
@@ -313,17 +317,17 @@ __device__ __forceinline__ void tk_row_radix(const float* row, uint32_t V, uint3
     if (t == 0) u[2] = 0;
     __syncthreads();
     uint32_t carry = 0;
-    for (uint32_t base = 0; base < V && KK > 0; base += NT) {
+    for (uint32_t base = 0; base < V && KK > 0; base += LN_NT) {
         uint32_t i = base + t;
         float v = i < V ? row[i] : NAN;
         bool c = i < V && tk_cand(v);
         uint32_t k = c ? tk_key(v) : 0;
         bool gt = c && k > prefix, eq = c && k == prefix;
         uint32_t tot;
-        uint32_t ex = block_excl_scan_u<NT>(eq ? 1u : 0u, scan_sh, &tot);
+        uint32_t ex = block_excl_scan_u<LN_NT>(eq ? 1u : 0u, scan_sh, &tot);
         if (gt || (eq && carry + ex < need)) {
             uint32_t pos = atomicAdd(&u[2], 1u);
-            if (pos < KMAX) buf[pos] = ((unsigned long long)(~k) << 32) | i;
+            if (pos < TK_MAX) buf[pos] = ((unsigned long long)(~k) << 32) | i;
         }
         carry += tot;
     }
@@ -331,29 +335,19 @@ __device__ __forceinline__ void tk_row_radix(const float* row, uint32_t V, uint3
     uint32_t n = KK;
     uint32_t np2 = 1;
     while (np2 < n) np2 <<= 1;
-    for (uint32_t i = n + t; i < np2; i += NT) buf[i] = ~0ull;
+    for (uint32_t i = n + t; i < np2; i += LN_NT) buf[i] = ~0ull;
     __syncthreads();
-    if (np2 > 1) block_sort_u64<NT>(buf, np2);
-    for (uint32_t j = t; j < K; j += NT) {
+    if (np2 > 1) block_sort_u64<LN_NT>(buf, np2);
+    for (uint32_t j = t; j < K; j += LN_NT) {
         if (j < n) {
             uint32_t id = (uint32_t)(buf[j] & 0xffffffffull);
-            vals[j] = row[id];
-            idxs[j] = id;
+            vals[(size_t)r * K + j] = row[id];
+            idxs[(size_t)r * K + j] = id;
         } else {
-            vals[j] = -3.0e38f;
-            idxs[j] = 0xffffffffu;
+            vals[(size_t)r * K + j] = -3.0e38f;
+            idxs[(size_t)r * K + j] = 0xffffffffu;
         }
     }
-}
-
-__global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
-                                                     float* vals, uint32_t* idxs) {
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t u[4];
-    __shared__ unsigned long long buf[TK_MAX];
-    __shared__ uint32_t scan_sh[LN_NT / 64];
-    const size_t r = blockIdx.x;
-    tk_row_radix<LN_NT, TK_MAX>(logits + r * ld, V, K, vals + r * K, idxs + r * K, buf, hist, u, scan_sh);
 }
 
 // BTOPK for K <= 64 from group maxima. zs_k_lane_scan reads the logits once
@@ -364,12 +358,15 @@ __global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_
 // read again, listed and sorted. With the draw of zs_lane_step's top-K path
 // in the same kernel. 256 rows of 151936 ids: the scan 24 us (6.5 TB/s), the
 // pick 20 us; chunks of 16384 ids with a top-K each and a merge took 54 + 20.
+// Rows with many groups or ids at the key (sorted rows, equal values) are cut
+// level by level instead (8 rows of 128256: equal values 18 us a call, sorted
+// 29, of whole numbers 26, rows in no order 13; 256 rows 37, 47, 44 and 34).
 #define LS_NT 256
 #define LS_IDS (16 * LS_NT)   // ids per workgroup of the scan
 #define LP_NT 256
 #define LP_GPT 20             // groups per thread of the pick at most
-#define LP_GL 1024            // listed groups at most
-#define LP_LIST 1024          // listed keys at most
+#define LP_GL 192             // listed groups at most (rows in no order list about K + 20)
+#define LP_LIST LP_NT         // listed keys at most: one per thread
 #define TC_K 64
 template <int GS>
 __global__ __launch_bounds__(LS_NT) void zs_k_lane_scan(const float* logits, uint32_t V, uint64_t ld, uint32_t* gmax,
@@ -414,27 +411,136 @@ struct tm_draw {   // the nucleus draw after the pick (zs_lane_step's top-K path
 };
 __device__ __forceinline__ uint32_t lane_draw64(float v, uint32_t id, uint32_t K, float T, uint32_t top_k, float tp,
                                                 uint32_t seed);
+// Of the workgroup's E * LP_NT places (t, t + LP_NT, ...: bit e), the first K
+// by (key desc, place asc); places of key 0 are none. Radix selection of the
+// K-th key over the digits in which the keys differ, then the places at it in
+// order. Called by every thread; hist: 256 words, u: 4 words.
+template <int E>
+__device__ __forceinline__ uint32_t tk_first(const uint32_t (&k)[E], uint32_t K, uint32_t* hist, uint32_t* u) {
+    constexpr uint32_t NW = LP_NT / 64;
+    static_assert(3 * NW <= 256 && E * NW <= 256 && LP_NT == 256, "one histogram holds the counts");
+    const uint32_t t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
+    uint32_t lo = ~0u, hi = 0, n = 0, all = 0;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if (!k[e]) continue;
+        lo = min(lo, k[e]);
+        hi = max(hi, k[e]);
+        n++;
+        all |= 1u << e;
+    }
+    lo = zs_wave_reduce(lo, [](uint32_t x, uint32_t y) { return min(x, y); });
+    hi = zs_wave_reduce(hi, [](uint32_t x, uint32_t y) { return max(x, y); });
+    n = wave_sum_u(n);
+    if (lane == 0) { hist[wid] = lo; hist[NW + wid] = hi; hist[2 * NW + wid] = n; }
+    __syncthreads();
+    n = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < NW; w++) {
+        lo = min(lo, hist[w]);
+        hi = max(hi, hist[NW + w]);
+        n += hist[2 * NW + w];
+    }
+    __syncthreads();
+    if (n <= K) return all;
+    // key: the K-th once its digits are known; those above the first in which
+    // the keys differ are hi's
+    int shift = lo != hi ? (31 - __clz((int)(lo ^ hi))) & ~7 : -8;
+    uint32_t mask = shift < 0 ? ~0u : shift == 24 ? 0u : ~0u << (shift + 8);
+    uint32_t key = hi & mask, need = K;
+    for (; shift >= 0; shift -= 8) {
+        hist[t] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; e++)
+            if (k[e] && (k[e] & mask) == key) atomicAdd(&hist[(k[e] >> shift) & 255u], 1u);
+        __syncthreads();
+        if (t < 64) {
+            uint32_t c[4], loc = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) { c[q] = hist[255u - 4u * t - (uint32_t)q]; loc += c[q]; }
+            const uint32_t inc = wave_incl_scan_u(loc);
+            uint32_t before = inc - loc;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (before < need && need <= before + c[q]) { u[0] = 255u - 4u * t - (uint32_t)q; u[1] = need - before; }
+                before += c[q];
+            }
+        }
+        __syncthreads();
+        key |= u[0] << shift;
+        mask |= 0xffu << shift;
+        need = u[1];
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const uint32_t c = (uint32_t)__popcll(__ballot(k[e] == key));
+        if (lane == 0) hist[(uint32_t)e * NW + wid] = c;
+    }
+    __syncthreads();
+    uint32_t run = 0, first = 0;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const unsigned long long m = __ballot(k[e] == key);
+        uint32_t before = run;
+#pragma unroll
+        for (uint32_t w = 0; w < NW; w++) {
+            const uint32_t c = hist[(uint32_t)e * NW + w];
+            before += w < wid ? c : 0u;
+            run += c;
+        }
+        before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, before));
+        if (k[e] > key || (k[e] == key && before < need)) first |= 1u << e;
+    }
+    __syncthreads();
+    return first;
+}
+// The chosen places in ascending order to gl (K <= 64 of them; the return is
+// their number). Called by every thread; u: 4 words, u[2] is 0 before and after.
+__device__ __forceinline__ uint32_t tk_places(uint32_t first, uint16_t* gl, uint32_t* u) {
+    const uint32_t t = threadIdx.x;
+    while (first) {
+        const uint32_t e = (uint32_t)__builtin_ctz(first);
+        first &= first - 1u;
+        gl[atomicAdd(&u[2], 1u)] = (uint16_t)(t + e * LP_NT);
+    }
+    __syncthreads();
+    const uint32_t n = u[2];
+    __syncthreads();
+    if (t < 64) {
+        const uint32_t g = wave_sort_u32(t < n ? (uint32_t)gl[t] : ~0u);
+        if (t < n) gl[t] = (uint16_t)g;
+        if (t == 0) u[2] = 0;
+    }
+    __syncthreads();
+    return n;
+}
+
 template <bool DRAW>
 __global__ __launch_bounds__(LP_NT) void zs_k_btopk_pick(const float* logits, uint32_t V, uint64_t ld, uint32_t K,
                                                          const uint32_t* gmax, uint32_t gstride, uint32_t gs, float* vals,
                                                          uint32_t* idxs, tm_draw d) {
     constexpr uint32_t NW = LP_NT / 64;
+    typedef float ls_f4 __attribute__((ext_vector_type(4)));
     __shared__ unsigned long long list[LP_LIST];
     __shared__ uint16_t gl[LP_GL];
-    __shared__ uint32_t hist[256], u[4], scan_sh[NW], wthr[NW];
+    __shared__ uint32_t hist[256], u[4], wthr[NW];
     const uint32_t r = blockIdx.x, t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
     const float* row = logits + (size_t)r * ld;
     const uint32_t ng = (V + (1u << gs) - 1u) >> gs, last4 = (V - 1u) & ~3u;
     const uint32_t* gm = gmax + (size_t)r * gstride;
     uint32_t k[LP_GPT], tm = 0;
+    auto load_groups = [&]() {
 #pragma unroll
-    for (int e = 0; e < LP_GPT; e++) k[e] = zs_gload(gm + min(t + (uint32_t)e * LP_NT, ng - 1u));
+        for (int e = 0; e < LP_GPT; e++) k[e] = zs_gload(gm + min(t + (uint32_t)e * LP_NT, ng - 1u));
 #pragma unroll
-    for (int e = 0; e < LP_GPT; e++) {
-        if (t + (uint32_t)e * LP_NT >= ng) k[e] = 0u;
-        tm = max(tm, k[e]);
-    }
-    if (t < 2) u[t] = 0;
+        for (int e = 0; e < LP_GPT; e++)
+            if (t + (uint32_t)e * LP_NT >= ng) k[e] = 0u;
+    };
+    load_groups();
+#pragma unroll
+    for (int e = 0; e < LP_GPT; e++) tm = max(tm, k[e]);
+    if (t < 4) u[t] = 0;
     // theta: in every wave the ceil(K / waves)-th largest thread maximum; the
     // smallest of them is reached by K groups (0: too few hold a candidate;
     // every candidate is listed then)
@@ -446,71 +552,136 @@ __global__ __launch_bounds__(LP_NT) void zs_k_btopk_pick(const float* logits, ui
 #pragma unroll
     for (uint32_t w = 1; w < NW; w++) theta = min(theta, wthr[w]);
     theta = max(theta, 1u);
+    uint32_t ngt = 0;
+#pragma unroll
+    for (int e = 0; e < LP_GPT; e++) ngt += k[e] >= theta ? 1u : 0u;
+    // (a thread's places at once: an atomic per group is served lane by lane)
+    uint32_t p = ngt ? atomicAdd(&u[0], ngt) : 0u;
 #pragma unroll
     for (int e = 0; e < LP_GPT; e++) {
         if (k[e] < theta) continue;
-        const uint32_t p = atomicAdd(&u[0], 1u);
         if (p < LP_GL) gl[p] = (uint16_t)(t + (uint32_t)e * LP_NT);
+        p++;
     }
     __syncthreads();
-    const uint32_t n_gl = u[0], qs = gs - 2u, nit = n_gl << qs;
+    const uint32_t n_gl = u[0], qs = gs - 2u, qm = (1u << qs) - 1u;
+    // keys of the ids x.x .. x.w from id on, 0 for no candidate
+    auto keys4 = [&](const ls_f4& x, uint32_t id, uint32_t (&kq)[4]) {
+        const float xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) kq[q] = id + (uint32_t)q < V && tk_cand(xs[q]) ? tk_key(xs[q]) : 0u;
+    };
     if (n_gl <= LP_GL) {
+        const uint32_t nit = n_gl << qs;
         constexpr int NU = 4;
         for (uint32_t i0 = 0; i0 < nit; i0 += NU * LP_NT) {
-            typedef float ls_f4 __attribute__((ext_vector_type(4)));
             ls_f4 v[NU];
             uint32_t id[NU];
 #pragma unroll
             for (int w = 0; w < NU; w++) {
                 const uint32_t i = i0 + t + (uint32_t)w * LP_NT, ic = min(i, nit - 1u);
-                id[w] = ((uint32_t)gl[ic >> qs] << gs) + 4u * (ic & ((1u << qs) - 1u));
+                id[w] = ((uint32_t)gl[ic >> qs] << gs) + 4u * (ic & qm);
                 v[w] = zs_gload(reinterpret_cast<const ls_f4*>(row + min(id[w], last4)));
                 if (i >= nit) id[w] = V;
             }
 #pragma unroll
             for (int w = 0; w < NU; w++) {
-                const float x[4] = {v[w].x, v[w].y, v[w].z, v[w].w};
+                // (one atomic per wave: one per lane is served lane by lane)
+                uint32_t kq[4], p = 0, n = 0;
+                keys4(v[w], id[w], kq);
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    if (id[w] + (uint32_t)q >= V || !tk_cand(x[q])) continue;
-                    const uint32_t kq = tk_key(x[q]);
-                    if (kq < theta) continue;
-                    const uint32_t p = atomicAdd(&u[1], 1u);
-                    if (p < LP_LIST) list[p] = ((unsigned long long)(~kq) << 32) | (id[w] + (uint32_t)q);
+                    const unsigned long long m = __ballot(kq[q] >= theta);
+                    p = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, p));
+                    n += (uint32_t)__popcll(m);
+                }
+                if (!n) continue;
+                uint32_t p0 = 0;
+                if (lane == 0) p0 = atomicAdd(&u[1], n);
+                p += (uint32_t)__builtin_amdgcn_readfirstlane((int)p0);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (kq[q] < theta) continue;
+                    if (p < LP_LIST) list[p] = ((unsigned long long)(~kq[q]) << 32) | (id[w] + (uint32_t)q);
+                    p++;
                 }
             }
         }
     }
     __syncthreads();
-    const uint32_t n = u[1];
+    uint32_t n = u[1];
+    if (n_gl > LP_GL || n > LP_LIST) {
+        // Many groups or ids reach theta. The first K ids lie in the first K
+        // groups by (maximum desc, group asc) -- K groups in front of another
+        // hold K ids in front of any of its -- and in the first K quads of
+        // those by the same order, 4 K ids.
+        constexpr int NQ = TC_K * 16 / LP_NT;   // quads per thread at most (K groups of 64 ids)
+        uint32_t ngl = n_gl;
+        if (n_gl <= LP_GL && (n_gl << qs) <= NQ * LP_NT) {
+            // the listed groups' quads fit as they are: in ascending order
+            static_assert(LP_GL <= LP_NT, "one listed group per thread");
+            const uint32_t g = t < n_gl ? gl[t] : ~0u;
+            uint32_t before = 0;
+            for (uint32_t j = 0; j < n_gl; j++) before += gl[j] < g ? 1u : 0u;
+            __syncthreads();
+            if (t < n_gl) gl[before] = (uint16_t)g;
+            __syncthreads();
+        } else {
+            __syncthreads();
+            load_groups();
+#pragma unroll
+            for (int e = 0; e < LP_GPT; e++)
+                if (k[e] < theta) k[e] = 0u;
+            ngl = tk_places(tk_first<LP_GPT>(k, K, hist, u), gl, u);
+        }
+        const uint32_t nit = ngl << qs;
+        uint32_t qk[NQ], qid[NQ];
+        ls_f4 v[NQ];
+#pragma unroll
+        for (int w = 0; w < NQ; w++) {
+            const uint32_t i = t + (uint32_t)w * LP_NT, ic = min(i, nit - 1u);
+            qid[w] = ((uint32_t)gl[ic >> qs] << gs) + 4u * (ic & qm);
+            v[w] = zs_gload(reinterpret_cast<const ls_f4*>(row + min(qid[w], last4)));
+            if (i >= nit) qid[w] = V;
+        }
+#pragma unroll
+        for (int w = 0; w < NQ; w++) {
+            uint32_t kq[4];
+            keys4(v[w], qid[w], kq);
+            qk[w] = max(max(kq[0], kq[1]), max(kq[2], kq[3]));
+        }
+        uint32_t first = tk_first<NQ>(qk, K, hist, u);
+        if (t == 0) u[1] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NQ; w++) {
+            if (!(first >> w & 1u)) continue;
+            uint32_t kq[4];
+            keys4(v[w], qid[w], kq);
+            uint32_t p = atomicAdd(&u[1], 4u);   // at most 4 K <= LP_LIST
+#pragma unroll
+            for (int q = 0; q < 4; q++) list[p + (uint32_t)q] = kq[q] ? ((unsigned long long)(~kq[q]) << 32) | (qid[w] + (uint32_t)q) : ~0ull;
+        }
+        __syncthreads();
+        n = u[1];
+    }
+    static_assert(4 * TC_K <= LP_LIST, "the quads' ids fit the list");
+    uint32_t np2 = 64;
+    while (np2 < n) np2 <<= 1;
+    if (t >= n && t < np2) list[t] = ~0ull;
+    __syncthreads();
+    block_sort_reg_u64<LP_NT, 1>(list, np2);
+    if (t >= 64) return;
     float v = -3.0e38f;
     uint32_t id = 0xffffffffu;
-    if (n_gl <= LP_GL && n <= LP_LIST) {
-        uint32_t np2 = 64;
-        while (np2 < n) np2 <<= 1;
-        for (uint32_t i = n + t; i < np2; i += LP_NT) list[i] = ~0ull;
-        __syncthreads();
-        block_sort_u64<LP_NT>(list, np2);
-        if (t >= 64) return;
-        const unsigned long long e = lane < min(K, n) ? list[lane] : ~0ull;
-        if (e != ~0ull) {
-            id = (uint32_t)e;
-            v = row[id];
-        }
-        if (lane < K) {
-            vals[(size_t)r * K + lane] = v;
-            idxs[(size_t)r * K + lane] = id;
-        }
-    } else {
-        // more equal maxima or more keys than the lists hold
-        tk_row_radix<LP_NT, LP_LIST>(row, V, K, vals + (size_t)r * K, idxs + (size_t)r * K, list, hist, u, scan_sh);
-        __threadfence_block();
-        __syncthreads();
-        if (t >= 64) return;
-        if (lane < K) {
-            v = vals[(size_t)r * K + lane];
-            id = idxs[(size_t)r * K + lane];
-        }
+    const unsigned long long e = lane < min(K, n) ? list[lane] : ~0ull;
+    if (e != ~0ull) {
+        id = (uint32_t)e;
+        v = row[id];
+    }
+    if (lane < K) {
+        vals[(size_t)r * K + lane] = v;
+        idxs[(size_t)r * K + lane] = id;
     }
     if (DRAW) {
         // the pool as zs_k_sample_topk64 reads it back
