@@ -54,8 +54,8 @@ def test_rows_of_every_launch_beside_a_sampler(B):
     c.close()
 
 
-# one chunk a row: 2048 workgroups decide in front of the residual pass, 2049 before it
-@pytest.mark.parametrize("B,V", [(2048, 37), (2049, 37), (1025, 8193)])
+# one chunk a row: 1024 workgroups decide in front of the residual pass, 1025 before it
+@pytest.mark.parametrize("B,V", [(1024, 37), (1025, 37), (512, 8193), (513, 8193), (2049, 37)])
 @pytest.mark.parametrize("sampled", [True, False])
 def test_decision_in_front_and_alone(B, V, sampled):
     print(f"[case] spec decision B={B} V={V} sampled={sampled}", flush=True)

@@ -71,8 +71,10 @@ __device__ __forceinline__ bool sp_live(float xc, float m, float c) {
 // .. +3. Non-temporal: a verification reads each of its rows once (the residual
 // pass one pair a row again), and its gigabytes would push the sampler's rows,
 // which the kernels beside it read several times, out of the caches (256 rows
-// of 9 positions of 151936 ids beside the sampler: 697 -> 682 us; alone, 64
-// rows of 128256, 88 us either way).
+// of 9 positions of 151936 ids beside the sampler: 697 -> 682 us). Alone, plain
+// / non-temporal loads in both passes: 5 positions greedily 128 x 151936 71 /
+// 64 us, 9 positions 256 x 151936 300 / 295, 64 x 128256 85.0 / 84.5; calls
+// below 25 us lose 1.
 typedef float sp_f4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void sp_load(const float* row, uint32_t base, uint32_t V, float (&x)[SP_EPT]) {
 #pragma unroll
@@ -490,11 +492,14 @@ __global__ __launch_bounds__(SP_NT) void zs_k_spec_decide(zs_spec_args a) {
 }
 
 // pass 3: chunk sums of the residual weights (rows that rejected a draft);
-// DECIDE: the decision in front, stored by chunk 0's workgroup. Rejection
-// sampling alone, in a launch of its own / in front (us a call, 9 positions):
-// 32 x 151936 (608 workgroups) 68 / 67, 64 x 128256 (1024) 91 / 90, 128 x
-// 151936 (2432) 172 / 179, 256 x 151936 (4864) 302 / 323.
-#define SP_DECIDE_WGS 2048u
+// DECIDE: the decision in front, stored by chunk 0's workgroup, as long as all
+// workgroups are resident at once (4 a CU): past that a second round repeats
+// it. Rejection sampling alone, in a launch of its own / in front (us a call; 3,
+// 9 and 17 positions): 32 x 151936 (608 workgroups, 9 positions) 68 / 67,
+// 64 x 128256 (1024) 91 / 90; 60 x 151936 (1140) 54 / 57, 94 / 100, 144 / 149;
+// 80 x 128256 (1280) 53 / 56, 96 / 102, 157 / 166; 128 x 128256 (2048) 68 / 71,
+// 138 / 145, 237 / 253; 256 x 151936 (4864, 9 positions) 302 / 323.
+#define SP_DECIDE_WGS 1024u
 template <bool DECIDE>
 __global__ __launch_bounds__(SP_NT) void zs_k_spec_rsum(zs_spec_args a) {
     const uint32_t c = blockIdx.x, r = blockIdx.y;
