@@ -27,15 +27,17 @@
 //       threshold (greedy argmax: the last maximal element, a NaN restarts
 //       the fold, sampler.rs:35-43);
 //   decisions: greedy / non-finite rows get their token; rows whose survivors
-//       fit ZS_SMALL_CAP are sampled exactly by one wave (small_path_wave);
-//       other rows are "big" and continue in zs_sample.hip;
+//       fit ZS_SMALL_CAP are sampled exactly, up to 64 by one wave
+//       (small_path_wave), more by the workgroup (rw_small_wg); other rows are
+//       "big" and continue in zs_sample.hip;
 //   state: which exact sums the row needs (zs_sums.hip: the observers' S and
 //       entropy, a big row's sampler S), over the whole row or over the
 //       allowed ids a masked row gathered to row scratch.
 #include <hip/hip_runtime.h>
 #ifdef ZS_WALK_DEBUG
-// Debug builds: wall-clock time of zs_k_row's phases (0-5, row count in 7)
-// and of the small path's (8-15), summed over rows (zs_dbg_row_stats).
+// Debug builds: wall-clock time of zs_k_row's phases (0-5, row count in 7; of
+// rw_groups the corrected maxima in 6, the thresholds in 15, both within 2)
+// and of the small path's (8-14), summed over rows (zs_dbg_row_stats).
 __device__ unsigned long long rw_dbg[16];
 #define ZS_SP_T(i)                                               \
     do {                                                         \
@@ -82,7 +84,7 @@ struct rw_shared {
     uint32_t sel_n;                 // list selection: places taken by the gather
     uint32_t inf_lim;               // observers: largest id whose -inf can enter the list
     uint32_t g_n, g_done;           // masked rows: allowed ids gathered to row scratch, gather done
-    uint32_t sel_st[4];             // list selection: chosen digit, count before it, its count, places
+    uint32_t sel_st[2];             // rw_kth_key: chosen digit, rank inside it
 };
 // The workgroup's LDS (one object, so that functions outside the kernel
 // address it directly).
@@ -396,8 +398,7 @@ struct rw_row {
     uint32_t V, np, words;
     uint32_t ldm4, wmax;            // last float4 of the row, last readable word
     uint32_t amask;                 // 15 for an unmasked row, else 0
-    uint32_t glast;                 // the last tile of the streamed range
-    uint32_t vend, gend;            // the streamed range's end: id (its ids >= vend read -inf) and tile
+    uint32_t tiles;                 // tiles of the row
 };
 struct rw_raw {
     float4 v;
@@ -456,33 +457,33 @@ __device__ __forceinline__ void rw_elems(const rw_row& R, uint32_t g, const rw_r
     x[1] = (aw & 2u) ? raw.v.y : -INFINITY;
     x[2] = (aw & 4u) ? raw.v.z : -INFINITY;
     x[3] = (aw & 8u) ? raw.v.w : -INFINITY;
-    const bool last = g >= R.glast;   // uniform
+    const bool last = g >= R.tiles - 1u;   // uniform
     if (last) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) x[q] = idx0 + q < R.vend ? x[q] : -INFINITY;
+        for (int q = 0; q < 4; q++) x[q] = idx0 + q < R.V ? x[q] : -INFINITY;
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) y[q] = x[q];
     if (R.np) {
         const uint32_t wd = raw.pw;
         uint32_t pb = (wd >> (idx0 & 31)) & 15u;
-        if (last) pb = idx0 < R.vend ? pb : 0u;
+        if (last) pb = idx0 < R.V ? pb : 0u;
         if (pb) rw_patch4<GP>(R, idx0, pb, wd, x, y, sh);
     }
 }
 
-// Calls f(g, u, x, y) for the tiles from g_begin up to R.gend in order, in
+// Calls f(g, u, x, y) for the tiles from g_begin on in order, in
 // groups of four (u = 0..3, a constant in each unrolled copy: per-tile state
 // of a group can live in registers indexed by u), with four tiles of loads in
 // flight: unrolled by four so that each load stays in its own registers until
 // used (copying a register whose load is outstanding waits for every load). f
 // returns true (uniformly) to stop; rw_stream then returns that tile's index,
-// else R.gend. The last group is padded with tiles past the range (ids >=
-// R.vend, read as -inf), which f must treat as neutral. f must not call functions: a call inside the
+// else R.tiles. The last group is padded with tiles past the row (ids >= R.V,
+// read as -inf), which f must treat as neutral. f must not call functions: a call inside the
 // loop saves the registers of the loads in flight, which waits for them.
 template <bool GP, class F>
 __device__ __forceinline__ uint32_t rw_stream(const rw_row& R, const rw_shared& sh, uint32_t g_begin, const F& f) {
-    const uint32_t ng = R.gend;
+    const uint32_t ng = R.tiles;
     rw_raw raw[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -524,7 +525,6 @@ struct rw_list {
     unsigned long long* buf;
     uint32_t* cnt;      // [3] per-tile reservation counters (rotating)
     long long* thr;     // admission threshold: keys > thr enter
-    uint32_t* flag;     // bit 0: the last compaction cut entries equal to its K-th key
 };
 
 // Selection on a list (list 0: observers, 1: sampler): of its first n
@@ -535,8 +535,8 @@ struct rw_list {
 // An MSB radix selection on the 64-bit entries, 8-bit digits: the digits
 // above the first bit where the members' keys differ are skipped; each pass
 // histograms one digit of the members that share the bits above it with the
-// K1-th smallest, and one wave picks the digit where the count reaches K1. It stops once the members up to and including the chosen digit
-// number at most the cap (always by the last digit: entries are distinct;
+// K1-th smallest, and one wave picks the digit where the count reaches K1. It
+// stops once the members up to and including the chosen digit number at most the cap (always by the last digit: entries are distinct;
 // K1 <= RW_SEL_MAX); those are gathered to the front and sorted, by one wave
 // up to RW_SEL_CAP, else by the workgroup.
 #define RW_SEL_CAP 256
@@ -658,8 +658,7 @@ __device__ __noinline__ uint32_t rw_select(int which, uint32_t n, uint32_t K1, u
 
 // Cuts a list to its K smallest members (rw_select); the K-th key becomes the
 // threshold (below K members: every id is admitted). Also records the value
-// of the threshold, whether entries equal to the K-th key were cut, and the
-// largest value cut (into *cutmax).
+// of the threshold and the largest value cut (into *cutmax).
 // Returns the new entry count. Called by every thread.
 __device__ uint32_t rw_compact(int which, const rw_list& L, uint32_t n, uint32_t K, uint32_t idlim, float* fthr,
                                float* cutmax) {
@@ -670,12 +669,10 @@ __device__ uint32_t rw_compact(int which, const rw_list& L, uint32_t n, uint32_t
             const uint32_t kk = ~(uint32_t)(L.buf[K - 1] >> 32);
             *L.thr = (long long)kk;
             *fthr = zs_key_to_float(kk);
-            *L.flag = (c > K && ~(uint32_t)(L.buf[K] >> 32) == kk) ? 1u : 0u;
             if (c > K) *cutmax = fmaxf(*cutmax, zs_key_to_float(~(uint32_t)(L.buf[K] >> 32)));
         } else {
             *L.thr = -1;
             *fthr = -INFINITY;
-            *L.flag = 0u;
         }
     }
     __syncthreads();
@@ -885,7 +882,7 @@ __device__ __forceinline__ void rw_small(uint64_t seed, uint64_t counter, uint32
     if (nsv > 64) {
         rw_small_wg(seed, counter, V, P.top_p, P.min_p, nsv, zmax);
     } else if (threadIdx.x < 64) {
-        const uint32_t tk = small_path_wave<1>(seed, counter, V, P, nsv, zmax, sh.sval, sh.sidx);
+        const uint32_t tk = small_path_wave(seed, counter, V, P, nsv, zmax, sh.sval, sh.sidx);
         if (threadIdx.x == 0) sh.tok = tk;
     }
 }
@@ -1553,7 +1550,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     const uint32_t t = threadIdx.x;
     const uint32_t V = b.V;
     rw_shared& sh = rw_sh;
-    __shared__ uint32_t cnt_o[3], cnt_s[3], flag_o, flag_s;
+    __shared__ uint32_t cnt_o[3], cnt_s[3];
     __shared__ long long thr_o, thr_s;
     const zs_row_params P = b.d_params[r];
     zs_row_state& st = a.rst[r];
@@ -1583,9 +1580,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     R.allow_or_row = R.allow ? R.allow : reinterpret_cast<const uint32_t*>(R.row);
     R.wmax = R.allow ? R.words - 1 : R.ldm4;
     R.amask = R.allow ? 0u : 15u;
-    R.gend = (V + RW_G - 1) / RW_G;
-    R.vend = V;
-    R.glast = (V - 1) / RW_G;
+    R.tiles = (V + RW_G - 1) / RW_G;
 
     // ---------------- P1: statistics and candidate lists
     // The sampler's z = y / T (sampler.rs:47-51) is not formed per element
@@ -1603,10 +1598,10 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
     uint32_t Ks = (smode & 1u) ? P.top_k : 0u;
     const uint32_t Ko = want_obs ? (ZS_OBS_CAND < V ? ZS_OBS_CAND : V) : 0u;
     rw_list LO, LS;
-    LO.buf = sh.u.b.o; LO.cnt = cnt_o; LO.thr = &thr_o; LO.flag = &flag_o;
-    LS.buf = sh.u.b.s; LS.cnt = cnt_s; LS.thr = &thr_s; LS.flag = &flag_s;
+    LO.buf = sh.u.b.o; LO.cnt = cnt_o; LO.thr = &thr_o;
+    LS.buf = sh.u.b.s; LS.cnt = cnt_s; LS.thr = &thr_s;
     if (t < 3) { cnt_o[t] = 0; cnt_s[t] = 0; }
-    if (t == 0) { thr_o = -1; thr_s = -1; flag_o = 0; flag_s = 0; }
+    if (t == 0) { thr_o = -1; thr_s = -1; }
     float omax = -INFINITY, ymax = -INFINITY;
     uint32_t fl = 0;                // ZS_CF_OBS_NAN, ZS_CF_Z_NAN
     float rejf = -INFINITY;         // largest y turned away from the top-k list
@@ -1675,8 +1670,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
         if ((!fast && Ks > ZS_KS) || G.s_drop) { smode = 0; Ks = 0; }
     }
     uint32_t g = 0;
-    const uint32_t ng = (gath || fast) ? 0u : R.gend;
-    const uint32_t Vend = R.vend;
+    const uint32_t ng = (gath || fast) ? 0u : R.tiles;
     // the admission thresholds in scalar registers: they change only where
     // the lists are set up (first tile) and compacted (outside the stream)
     float r_tfo = -INFINITY, r_tfs = -INFINITY;
@@ -1734,7 +1728,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
                 last_nan = max(last_nan, (int)(idx0 + 31 - __clz(ny)));
             }
             // valid ids of the thread (the last tile only is partial)
-            const uint32_t vm = idx0 + 4 <= Vend ? 15u : (idx0 >= Vend ? 0u : (1u << (Vend - idx0)) - 1u);
+            const uint32_t vm = idx0 + 4 <= V ? 15u : (idx0 >= V ? 0u : (1u << (V - idx0)) - 1u);
             if (tinf) {
                 // y / inf is NaN for a real y = +-inf (ids past the range read
                 // -inf and are no elements)
@@ -1745,7 +1739,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
             if (greedy) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    if (y[q] != y[q] || idx0 + q >= Vend) continue;
+                    if (y[q] != y[q] || idx0 + q >= V) continue;
                     // -0.0 and +0.0 compare equal in the reference (partial_cmp)
                     const uint32_t k = zs_total_key(y[q] == 0.0f ? 0.0f : y[q]);
                     const unsigned long long c = ((unsigned long long)k << 32) | (idx0 + q + 1);
@@ -1755,7 +1749,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
             if (!thr_init) {
                 // initial thresholds (first tile): in every wave the c-th largest
                 // thread maximum has at least c elements of that wave at or above
-                // it, so the smallest of the waves' values, with c = ceil(K / 16),
+                // it, so the smallest of the waves' values, with c = ceil(K / RW_NW),
                 // has at least K elements of this tile at or above it (ids >= V
                 // hold key 0)
                 thr_init = true;
@@ -1924,7 +1918,7 @@ __global__ __launch_bounds__(RW_NT) void zs_k_row(zs_sargs a) {
             uint32_t kx[4], ky[4];
             keys(x, y, kx, ky);
             const uint32_t idx0 = ovf * RW_G + 4 * t;
-            const uint32_t vm = idx0 + 4 <= Vend ? 15u : (idx0 >= Vend ? 0u : (1u << (Vend - idx0)) - 1u);
+            const uint32_t vm = idx0 + 4 <= V ? 15u : (idx0 >= V ? 0u : (1u << (V - idx0)) - 1u);
             uint32_t po = 0, ps = 0;
             for (int round = 0; ; round++) {
                 // the tile's elements above the current thresholds, minus those placed

@@ -64,8 +64,9 @@ __device__ __forceinline__ bool zs_allowed_bit(const zs_batch& b, uint32_t r, ui
 }
 
 // Small survivor sets (n <= ZS_SMALL_CAP, all other logits are -inf after
-// top-k / mask) are sampled exactly by one wave of the row kernel: zero terms
-// of the reference's full-vocabulary loops do not change a running sum.
+// top-k / mask) are sampled exactly in the row kernel, up to 64 by one wave
+// (small_path_wave), more by the workgroup: zero terms of the reference's
+// full-vocabulary loops do not change a running sum.
 #define ZS_SMALL_CAP 512
 
 // Ascending bitonic sort of 64*E u64 keys by one wave, element i = lane*E + e
@@ -105,14 +106,11 @@ __device__ __forceinline__ void wave_sort_u64_e(unsigned long long (&v)[E]) {
 #define ZS_SP_T(i) do { } while (0)
 #endif
 
-// The wave's values (element i = lane * E + e in register e of lane i / E;
-// the first n) written to LDS scratch in element order, for a serial pass.
-template <int E>
-__device__ __forceinline__ void wave_stage_f(float* buf, const float (&v)[E], uint32_t n) {
+// The wave's values (one per lane, the first n) written to LDS scratch, for a
+// serial pass.
+__device__ __forceinline__ void wave_stage_f(float* buf, float v, uint32_t n) {
     const uint32_t lane = (uint32_t)zs_lane();
-#pragma unroll
-    for (int e = 0; e < E; e++)
-        if (lane * E + e < n) buf[lane * E + e] = v[e];
+    if (lane < n) buf[lane] = v;
     __builtin_amdgcn_s_waitcnt(0);   // the wave's own LDS writes before its reads
     __builtin_amdgcn_wave_barrier();
 }
@@ -158,40 +156,28 @@ __device__ __forceinline__ uint32_t serial_scan_f(const float* buf, uint32_t n, 
     return n;
 }
 
-// Exact sampler over a small survivor set (n <= 64 * E, every other element
-// below the top-k threshold, masked or -inf), by one wave: the reference's
+// Exact sampler over a small survivor set (n <= 64, every other element below
+// the top-k threshold, masked or -inf), by one wave: the reference's
 // sequential f32 sums are done literally, one addition at a time in the
 // reference's order, with no workgroup synchronisation (sampler.rs:46-127).
 // The additions run over LDS copies of the values (sval, sidx: the survivors
 // on entry, then scratch; 16-byte aligned). Called by the 64 lanes of one
 // wave; returns the token on every lane.
-template <int E>
-__device__ uint32_t small_path_wave(uint64_t seed, uint64_t counter, uint32_t V, const zs_row_params& P, uint32_t n, float m,
-                                    float* sval, uint32_t* sidx) {
+__device__ __forceinline__ uint32_t small_path_wave(uint64_t seed, uint64_t counter, uint32_t V, const zs_row_params& P,
+                                                    uint32_t n, float m, float* sval, uint32_t* sidx) {
     const uint32_t lane = (uint32_t)zs_lane();
+    const bool live = lane < n;
 #ifdef ZS_WALK_DEBUG
     unsigned long long sp_t0 = wall_clock64();
 #endif
-    // survivors by index: element i (sorted) in register i % E of lane i / E
-    unsigned long long key[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const uint32_t i = lane * E + e;
-        key[e] = i < n ? (((unsigned long long)sidx[i] << 32) | zs_f2u(sval[i])) : ~0ull;
-    }
-    wave_sort_u64_e<E>(key);
+    // survivors by index, one per lane
+    const unsigned long long key = wave_sort_u64(live ? (((unsigned long long)sidx[lane] << 32) | zs_f2u(sval[lane])) : ~0ull);
     ZS_SP_T(0);
-    uint32_t id[E];
-    float p[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const bool live = lane * E + e < n;
-        id[e] = (uint32_t)(key[e] >> 32);
-        p[e] = live ? zs_expf(zs_u2f((uint32_t)key[e]) - m) : 0.0f;
-    }
-    // s0 + v[0] + v[1] + ... in order (sampler.rs:68, 80, 107)
-    auto seq_sum = [&](const float (&v)[E], float s0) {
-        wave_stage_f<E>(sval, v, n);
+    const uint32_t id = (uint32_t)(key >> 32);
+    float p = live ? zs_expf(zs_u2f((uint32_t)key) - m) : 0.0f;
+    // s0 + v of lane 0 + v of lane 1 + ... (sampler.rs:68, 80, 107)
+    auto seq_sum = [&](float v, float s0) {
+        wave_stage_f(sval, v, n);
         float s;
         serial_scan_f(sval, n, s0, NAN, &s);
         __builtin_amdgcn_wave_barrier();
@@ -199,42 +185,24 @@ __device__ uint32_t small_path_wave(uint64_t seed, uint64_t counter, uint32_t V,
     };
     // softmax (sampler.rs:67-69)
     ZS_SP_T(1);
-    const float S = seq_sum(p, -0.0f);
-#pragma unroll
-    for (int e = 0; e < E; e++) p[e] = p[e] / S;
+    p = p / seq_sum(p, -0.0f);
     ZS_SP_T(2);
     // min-p (sampler.rs:72-88)
     if (P.min_p > 0.0f) {
-        float pm = 0.0f;
-#pragma unroll
-        for (int e = 0; e < E; e++) if (lane * E + e < n) pm = fmaxf(pm, p[e]);
-        pm = wave_max_f(pm);
-        const float cut = P.min_p * pm;
-#pragma unroll
-        for (int e = 0; e < E; e++) if (p[e] < cut) p[e] = 0.0f;
+        const float cut = P.min_p * wave_max_f(live ? p : 0.0f);
+        if (p < cut) p = 0.0f;
         const float kept = seq_sum(p, 0.0f);
-        if (kept > 0.0f)
-#pragma unroll
-            for (int e = 0; e < E; e++) p[e] = p[e] / kept;
+        if (kept > 0.0f) p = p / kept;
     }
     // top-p (sampler.rs:91-115): cumsum in (p desc, idx asc) order
     if (P.top_p < 1.0f) {
         uint32_t vstar = 0, istar = 0xffffffffu;
         const bool none = !(P.top_p > 0.0f);  // cumsum 0 >= top_p: nothing kept
         if (!none) {
-            unsigned long long k2[E];
-#pragma unroll
-            for (int e = 0; e < E; e++)
-                k2[e] = lane * E + e < n ? (((unsigned long long)(~zs_f2u(p[e])) << 32) | id[e]) : ~0ull;
-            wave_sort_u64_e<E>(k2);
+            const unsigned long long k2 = wave_sort_u64(live ? (((unsigned long long)(~zs_f2u(p)) << 32) | id) : ~0ull);
             ZS_SP_T(3);
-            float ps[E];
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                ps[e] = zs_u2f(~(uint32_t)(k2[e] >> 32));
-                if (lane * E + e < n) sidx[lane * E + e] = (uint32_t)k2[e];
-            }
-            wave_stage_f<E>(sval, ps, n);
+            if (live) sidx[lane] = (uint32_t)k2;
+            wave_stage_f(sval, zs_u2f(~(uint32_t)(k2 >> 32)), n);
             float cum;
             const uint32_t i = serial_scan_f(sval, n, 0.0f, P.top_p, &cum);
             if (i < n) {
@@ -244,26 +212,18 @@ __device__ uint32_t small_path_wave(uint64_t seed, uint64_t counter, uint32_t V,
             __builtin_amdgcn_wave_barrier();
             ZS_SP_T(4);
         }
-        float f[E];
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            const uint32_t pb = zs_f2u(p[e]);
-            const bool keep = !none && (pb > vstar || (pb == vstar && id[e] <= istar));
-            f[e] = keep ? p[e] : 0.0f;
-        }
+        const uint32_t pb = zs_f2u(p);
+        const bool keep = !none && (pb > vstar || (pb == vstar && id <= istar));
+        const float f = keep ? p : 0.0f;
         const float sum = seq_sum(f, -0.0f);
-        if (sum > 0.0f)
-#pragma unroll
-            for (int e = 0; e < E; e++) p[e] = f[e] / sum;
+        if (sum > 0.0f) p = f / sum;
         ZS_SP_T(5);
     }
     // draw (sampler.rs:118-127); r == 0 stops at index 0 whatever its p
     const float rr = zs_philox_uniform(seed, counter, 0u);
     if (rr <= 0.0f) return 0;
-#pragma unroll
-    for (int e = 0; e < E; e++)
-        if (lane * E + e < n) sidx[lane * E + e] = id[e];
-    wave_stage_f<E>(sval, p, n);
+    if (live) sidx[lane] = id;
+    wave_stage_f(sval, p, n);
     float cum;
     const uint32_t i = serial_scan_f(sval, n, 0.0f, rr, &cum);
     ZS_SP_T(6);
