@@ -106,12 +106,13 @@ def algorithmic_bytes_per_row(V, H, masked):
 
 
 SPEC_K = 4
-# HBM bytes per launch of the C5 batch's dispatches, measured with rocprofv3
-# --pmc FETCH_SIZE / WRITE_SIZE and scaled by the copy-kernel calibration
-# (profiles/c5_kernels_counters.md, the tree of the commit that added it)
-TRAFFIC = {"zs_k_spec_chunk": 1402.4e6, "zs_k_row": 107.8e6, "zs_k_sapx1": 26.6e6, "zs_k_sround1": 30.1e6,
+# HBM bytes of the C5 batch's kernel marks, measured with rocprofv3 --pmc
+# FETCH_SIZE / WRITE_SIZE and scaled by the copy-kernel calibration
+# (profiles/c5_kernels_counters.md, the tree of the commit that added it;
+# zs_k_row is the mark of zs_k_scan and zs_k_row together)
+TRAFFIC = {"zs_k_spec_chunk": 1402.5e6, "zs_k_row": 122.1e6, "zs_k_sapx1": 26.6e6, "zs_k_sround1": 30.1e6,
            "zs_k_sapx2": 87.1e6, "zs_k_sround2": 97.2e6, "zs_k_sround3": 97.5e6, "zs_k_pv": 64.1e6,
-           "zs_k_tp_inc": 36.4e6, "zs_k_big": 0.6e6}
+           "zs_k_tp_inc": 17.2e6, "zs_k_big": 0.6e6}
 
 
 def spec_bytes_per_row(V, k):
