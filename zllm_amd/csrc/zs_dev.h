@@ -25,7 +25,7 @@ __device__ __forceinline__ int zs_wid() { return (int)(threadIdx.x >> 6); }
 // the row swaps of gfx950 across them. A lane shuffle goes through the LDS
 // crossbar instead: its latency (and, for the sorts of a full workgroup, its
 // rate) bounded the sorting networks and reductions that used it (zs_k_row on
-// 64 x 128256: 31.9 -> 30.1 us).
+// 64 x 128256: 31.9 -> 30.4 us).
 template <int J>
 __device__ __forceinline__ uint32_t zs_lane_xor(uint32_t v) {
 #if defined(__HIP_DEVICE_COMPILE__)

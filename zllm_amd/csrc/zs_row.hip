@@ -221,8 +221,8 @@ __device__ __forceinline__ int rw_patches(const zs_sargs& a, uint32_t r, const z
     // its id and its value (bias or count, as bits). The first RW_PE entries
     // of a thread stay in registers with their logit, so that every list
     // element of a row of up to 1024 is loaded once, all loads at once: the
-    // lists re-read per step and the logits gathered word by word took 13 us
-    // on 256 counts, 6 us now.
+    // lists re-read per step and the logits gathered word by word took
+    // 10.5 us on 256 counts, 5.5 now.
     const bool masked = (P.flags & ZS_ROW_MASKED) && b.d_allow_bits;
     auto id_of = [&](uint32_t i) -> uint32_t {
         return i < nb ? b.d_ban_ids[ban0 + i] : i < nb + nbi ? b.d_bias_ids[bi0 + i - nb] : b.d_cnt_ids[c0 + i - nb - nbi];
@@ -949,8 +949,11 @@ __device__ __forceinline__ uint32_t rw_block_row(const zs_batch& b, uint32_t j, 
 // A chain of dependent loads and LDS steps bounds it, not V. The streaming
 // loop with its admissions spent 50 us on half a row of 128256 ids; measured,
 // scan + row kernel against the streaming row kernel (us):
-//   1 x 32000 3 + 24 / 45, 64 x 128256 7 + 32 / 92, 256 x 151936 (half the rows
-//   masked) 23 + 47 / 133, 128 x 151936 masked 11 + 47 / 87.
+//   1 x 32000 3 + 19 / 43, 64 x 128256 8 + 30 / 92, 256 x 151936 (half the rows
+//   masked) 20 + 46 / 139, 128 x 151936 masked 11 + 46 / 87.
+// Longest are the rows of a wide top-k (8 x 100003; k = 40 20 us): k = 500 64,
+// its survivors sampled here, k = 2000 57 (two radix selections, of up to 4096
+// keys).
 // Returns false (uniformly) for rows whose lists would overflow: they take
 // the streaming loop of zs_k_row.
 // ---------------------------------------------------------------------------
@@ -1474,8 +1477,9 @@ __device__ __forceinline__ bool rw_groups(const zs_sargs& a, uint32_t r, const r
 // ---------------------------------------------------------------------------
 // zs_k_scan: the group maxima of every row, over the whole GPU. One read of
 // the logits, 4 16-byte loads in flight per thread; a masked row's loads are
-// skipped where 4 ids in a row are disallowed. HBM-bound: 32.8 MB (64 x 128256)
-// in 7.2 us. (A NaN or few survivors are seen in the maxima: no other statistic
+// skipped where 4 ids in a row are disallowed. 32.8 MB (64 x 128256) take 8 us, 4.1
+// TB/s, 89 MB of 256 x 151936 with half the rows masked 20 us, 4.7 TB/s with the
+// maxima written. (A NaN or few survivors are seen in the maxima: no other statistic
 // is needed.)
 // ---------------------------------------------------------------------------
 #define SC_NT 256
