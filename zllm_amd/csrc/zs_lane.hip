@@ -360,12 +360,12 @@ __global__ __launch_bounds__(LN_NT) void zs_k_btopk(const float* logits, uint32_
 // pick 20 us; chunks of 16384 ids with a top-K each and a merge took 54 + 20.
 // Rows with many groups or ids at the key (sorted rows, equal values) are cut
 // level by level instead (8 rows of 128256: equal values 18 us a call, sorted
-// 29, of whole numbers 26, rows in no order 13; 256 rows 37, 47, 44 and 34).
+// 28, of whole numbers 26, rows in no order 13; 256 rows 37, 47, 44 and 34).
 #define LS_NT 256
 #define LS_IDS (16 * LS_NT)   // ids per workgroup of the scan
 #define LP_NT 256
 #define LP_GPT 20             // groups per thread of the pick at most
-#define LP_GL 192             // listed groups at most (rows in no order list about K + 20)
+#define LP_GL 192             // listed groups at most (rows in no order list K + 20 to K + 80)
 #define LP_LIST LP_NT         // listed keys at most: one per thread
 #define TC_K 64
 template <int GS>
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(LP_NT) void zs_k_btopk_pick(const float* logits, ui
     constexpr uint32_t NW = LP_NT / 64;
     typedef float ls_f4 __attribute__((ext_vector_type(4)));
     __shared__ unsigned long long list[LP_LIST];
-    __shared__ uint16_t gl[LP_GL];
+    __shared__ alignas(16) uint16_t gl[LP_GL];
     __shared__ uint32_t hist[256], u[4], wthr[NW];
     const uint32_t r = blockIdx.x, t = threadIdx.x, lane = (uint32_t)zs_lane(), wid = (uint32_t)zs_wid();
     const float* row = logits + (size_t)r * ld;
@@ -620,9 +620,18 @@ __global__ __launch_bounds__(LP_NT) void zs_k_btopk_pick(const float* logits, ui
         if (n_gl <= LP_GL && (n_gl << qs) <= NQ * LP_NT) {
             // the listed groups' quads fit as they are: in ascending order
             static_assert(LP_GL <= LP_NT, "one listed group per thread");
-            const uint32_t g = t < n_gl ? gl[t] : ~0u;
+            static_assert(LP_GL % 8 == 0, "eight to a read");
+            if (t >= n_gl && t < LP_GL) gl[t] = 0xffffu;
+            __syncthreads();
+            const uint32_t g = t < n_gl ? gl[t] : 0xffffu;
             uint32_t before = 0;
-            for (uint32_t j = 0; j < n_gl; j++) before += gl[j] < g ? 1u : 0u;
+#pragma unroll 4
+            for (uint32_t j = 0; j < LP_GL / 8; j++) {
+                const uint4 o = reinterpret_cast<const uint4*>(gl)[j];
+                const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+                for (int q = 0; q < 4; q++) before += ((ow[q] & 0xffffu) < g ? 1u : 0u) + ((ow[q] >> 16) < g ? 1u : 0u);
+            }
             __syncthreads();
             if (t < n_gl) gl[before] = (uint16_t)g;
             __syncthreads();
